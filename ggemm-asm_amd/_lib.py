@@ -40,6 +40,7 @@ EXPORTS = (
     "ggemm_vark_wgrad_fp8",
     "ggemm_vark_wgrad_fp8_k32",
     "ggemm_vark_wgrad_fp8_out",
+    "ggemm_vark_wgrad_fp8_swapped",
     "ggemm_vark_wgrad_fp8_wide",
     "ggemm_vark_wgrad_mxfp8",
     "ggemm_vark_wgrad_mxfp8_tile",
@@ -73,7 +74,7 @@ QUANT_EXPORTS = (
 # GGEMM_VARK_ABI_VERSION of include/ggemm_vark.h that these bindings are written for. Some exports
 # changed signature between versions (ggemm_vark_wgrad_fp8_out and ggemm_vark_wgrad_mxfp8 took
 # M_total from version 3 on), so a library of another version is refused at load.
-ABI_VERSION = 9
+ABI_VERSION = 10
 
 ERRORS = {
     0: "GGEMM_OK", -1: "GGEMM_E_NULL", -2: "GGEMM_E_SHAPE", -3: "GGEMM_E_STRIDE",
@@ -117,6 +118,8 @@ def load():
         f.restype = ctypes.c_int
     lib.ggemm_vark_wgrad_fp8_out.argtypes = tw[:-1] + [i32, i64, vp]
     lib.ggemm_vark_wgrad_fp8_out.restype = ctypes.c_int
+    lib.ggemm_vark_wgrad_fp8_swapped.argtypes = tw[:-1] + [i64, vp]
+    lib.ggemm_vark_wgrad_fp8_swapped.restype = ctypes.c_int
     lib.ggemm_vark_wgrad_fp8_wide.argtypes = tw[:-1] + [i64, i32, i32, vp]
     lib.ggemm_vark_wgrad_fp8_wide.restype = ctypes.c_int
     lib.ggemm_vark_wgrad_mxfp8.argtypes = [vp, vp, vp, vp, vp, vp] + [i32] * 10 + [i64, vp]

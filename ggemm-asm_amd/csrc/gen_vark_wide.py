@@ -80,12 +80,15 @@ def swizzle(pitch):
 
 
 class Config:
-    def __init__(self, tm, tn, out="bf16", mx=False):
+    def __init__(self, tm, tn, out="bf16", mx=False, swapped=False):
         self.tm, self.tn = tm, tn
         self.out = out                                  # "bf16", "f32" (fp32 C) or "f32acc" (C += result)
         self.mx = mx                                    # MXFP8: e8m0 block scales, scaled MFMA
+        self.swapped = swapped                          # LHS e5m2, RHS e4m3 (dW = dy^T x) instead
         assert not mx or (out == "bf16" and tm == tn == 320)
-        self.name = f"{tm}x{tn}" + ("" if out == "bf16" else "_" + out) + ("_mx" if mx else "")
+        assert not swapped or (out == "bf16" and not mx)
+        self.name = (f"{tm}x{tn}" + ("" if out == "bf16" else "_" + out) + ("_mx" if mx else "")
+                     + ("_swapped" if swapped else ""))
         self.bm, self.bn = tm // 64, tn // 64           # 32-wide blocks per wave (2 x 2 waves)
         self.rhs_off = KS * tm
         self.slot = KS * (tm + tn)
@@ -214,6 +217,8 @@ class Config:
 
 CONFIGS = (Config(256, 384), Config(320, 320), Config(320, 320, "f32"), Config(320, 320, "f32acc"),
            Config(320, 320, mx=True))
+# e5m2 LHS x e4m3 RHS, bf16 C: the same statements but for the MFMA's format bits
+SWAPPED_CONFIGS = (Config(256, 384, swapped=True), Config(320, 320, swapped=True))
 
 
 class Gen:
@@ -423,7 +428,9 @@ class Gen:
             self.emit(f"v_mfma_scale_f32_32x32x64_f8f6f4 {d}, v[{a}:{a + 7}], v[{b}:{b + 7}], {src}, v{ra}, v{rb} "
                       f"op_sel_hi:[{ha},{hb},0] cbsz:1")
             return
-        self.emit(f"v_mfma_f32_32x32x64_f8f6f4 {d}, v[{a}:{a + 7}], v[{b}:{b + 7}], {src} cbsz:1")
+        # A = RHS, B = LHS: e5m2 (format 1) is cbsz for A, blgp for B
+        self.emit(f"v_mfma_f32_32x32x64_f8f6f4 {d}, v[{a}:{a + 7}], v[{b}:{b + 7}], {src} "
+                  + ("blgp:1" if c.swapped else "cbsz:1"))
 
     # ---------------------------------------------------------------- one stage
 
@@ -1242,7 +1249,7 @@ def render():
            "// wgrad kernels (vark_wide.h) and of the wide persistent fwd / dgrad kernel (persistent_wide.h):",
            "// gfx950 assembly, one inline asm statement per tile shape."]
     total = 0
-    for c in CONFIGS + KCONFIGS:
+    for c in CONFIGS + SWAPPED_CONFIGS + KCONFIGS:
         g = GenK(c) if isinstance(c, KConfig) else Gen(c)
         g.tile()
         total += len(g.lines)

@@ -11,15 +11,18 @@
 #include "vark_kernel.h"
 #include "vark_wide.h"
 
-GGEMM_DEFINE_TENSORWISE_LIB_KERNEL(_grouped_variable_k_gemm_kernel, false, uint16_t, ggemm::kOutBF16)
-GGEMM_DEFINE_TENSORWISE_LIB_KERNEL(_grouped_variable_k_gemm_kernel_k32, true, uint16_t, ggemm::kOutBF16)
+GGEMM_DEFINE_TENSORWISE_LIB_KERNEL(_grouped_variable_k_gemm_kernel, false, uint16_t, ggemm::kOutBF16, false)
+GGEMM_DEFINE_TENSORWISE_LIB_KERNEL(_grouped_variable_k_gemm_kernel_k32, true, uint16_t, ggemm::kOutBF16, false)
 GGEMM_DEFINE_MX_KERNEL(_grouped_variable_k_mxfp8_gemm_kernel)
-GGEMM_DEFINE_TENSORWISE_LIB_KERNEL(_grouped_variable_k_gemm_kernel_f32, false, float, ggemm::kOutF32)
-GGEMM_DEFINE_TENSORWISE_LIB_KERNEL(_grouped_variable_k_gemm_kernel_f32_acc, false, float, ggemm::kOutF32Acc)
-GGEMM_DEFINE_WIDE_KERNEL(_grouped_variable_k_gemm_kernel_wide, 256, 384, uint16_t, ggemm::kOutBF16)
-GGEMM_DEFINE_WIDE_KERNEL(_grouped_variable_k_gemm_kernel_wide320, 320, 320, uint16_t, ggemm::kOutBF16)
-GGEMM_DEFINE_WIDE_KERNEL(_grouped_variable_k_gemm_kernel_wide320_f32, 320, 320, float, ggemm::kOutF32)
-GGEMM_DEFINE_WIDE_KERNEL(_grouped_variable_k_gemm_kernel_wide320_f32_acc, 320, 320, float, ggemm::kOutF32Acc)
+GGEMM_DEFINE_TENSORWISE_LIB_KERNEL(_grouped_variable_k_gemm_kernel_f32, false, float, ggemm::kOutF32, false)
+GGEMM_DEFINE_TENSORWISE_LIB_KERNEL(_grouped_variable_k_gemm_kernel_f32_acc, false, float, ggemm::kOutF32Acc, false)
+GGEMM_DEFINE_WIDE_KERNEL(_grouped_variable_k_gemm_kernel_wide, 256, 384, uint16_t, ggemm::kOutBF16, false)
+GGEMM_DEFINE_WIDE_KERNEL(_grouped_variable_k_gemm_kernel_wide320, 320, 320, uint16_t, ggemm::kOutBF16, false)
+GGEMM_DEFINE_WIDE_KERNEL(_grouped_variable_k_gemm_kernel_wide320_f32, 320, 320, float, ggemm::kOutF32, false)
+GGEMM_DEFINE_WIDE_KERNEL(_grouped_variable_k_gemm_kernel_wide320_f32_acc, 320, 320, float, ggemm::kOutF32Acc, false)
+GGEMM_DEFINE_TENSORWISE_LIB_KERNEL(_grouped_variable_k_gemm_kernel_swapped, false, uint16_t, ggemm::kOutBF16, true)
+GGEMM_DEFINE_WIDE_KERNEL(_grouped_variable_k_gemm_kernel_wide_swapped, 256, 384, uint16_t, ggemm::kOutBF16, true)
+GGEMM_DEFINE_WIDE_KERNEL(_grouped_variable_k_gemm_kernel_wide320_swapped, 320, 320, uint16_t, ggemm::kOutBF16, true)
 GGEMM_DEFINE_WIDE_MX_KERNEL(_grouped_variable_k_mxfp8_gemm_kernel_wide320)
 
 namespace {
@@ -70,9 +73,10 @@ int wide_selected(int OUT_M, int OUT_N, int64_t scm, int64_t scg, const void* ou
   return OUT_M >= 1024 && wide_rows_aligned(out, scm, scg) ? wide_tile_for(OUT_M, OUT_N, (int)scm) : 0;
 }
 
-int launch_wide(int tile, int out_mode, const void* lhs, const void* rhs, void* out, const float* lhs_scale,
-                const float* rhs_scale, const int64_t* group_offs, int32_t G, int32_t OUT_M, int32_t OUT_N,
-                int32_t slm, int32_t srm, int32_t scg, int32_t scm, int32_t scn, int64_t M_total, void* stream) {
+// swapped: e5m2 LHS, e4m3 RHS (bf16 C only)
+int launch_wide(bool swapped, int tile, int out_mode, const void* lhs, const void* rhs, void* out,
+                const float* lhs_scale, const float* rhs_scale, const int64_t* group_offs, int32_t G, int32_t OUT_M,
+                int32_t OUT_N, int32_t slm, int32_t srm, int32_t scg, int32_t scm, int32_t scn, int64_t M_total, void* stream) {
   int cus = 0;
   int rc = device_cus(&cus);
   if (rc) return rc;
@@ -80,7 +84,9 @@ int launch_wide(int tile, int out_mode, const void* lhs, const void* rhs, void* 
   const int64_t m_total = M_total < INT32_MAX ? M_total : INT32_MAX;
   const dim3 grid(cus), block(ggemm::wide::kNT);
   if (out_mode == GGEMM_OUT_BF16) {
-    auto kern = tile == 320 ? _grouped_variable_k_gemm_kernel_wide320 : _grouped_variable_k_gemm_kernel_wide;
+    auto kern = swapped ? (tile == 320 ? _grouped_variable_k_gemm_kernel_wide320_swapped
+                                       : _grouped_variable_k_gemm_kernel_wide_swapped)
+                        : (tile == 320 ? _grouped_variable_k_gemm_kernel_wide320 : _grouped_variable_k_gemm_kernel_wide);
     hipLaunchKernelGGL(kern, grid, block, 0, (hipStream_t)stream, (const uint8_t*)lhs, (const uint8_t*)rhs,
                        (uint16_t*)out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N, slm, srm, scg, scm, scn,
                        (void*)nullptr, (void*)nullptr, m_total);
@@ -98,9 +104,11 @@ int launch_wide(int tile, int out_mode, const void* lhs, const void* rhs, void* 
 
 extern "C" {
 
+enum class Mfma { kK128, kK32, kK128Swapped };   // swapped: e5m2 LHS, e4m3 RHS
+
 // m_total: the token count group offsets are clamped to on the device (INT64_MAX for the entry
 // points with the reference's argument list, which carries none).
-static int launch_tensorwise(bool legacy, const void* lhs, const void* rhs, void* out, const float* lhs_scale,
+static int launch_tensorwise(Mfma mfma, const void* lhs, const void* rhs, void* out, const float* lhs_scale,
                              const float* rhs_scale, const int64_t* group_offs, int32_t G, int32_t OUT_M,
                              int32_t OUT_N, int32_t slm, int32_t srm, int32_t scg, int32_t scm, int32_t scn,
                              int64_t m_total, void* stream) {
@@ -108,13 +116,15 @@ static int launch_tensorwise(bool legacy, const void* lhs, const void* rhs, void
                            scn);
   if (rc) return rc;
   if (m_total < 0) return GGEMM_E_SHAPE;
-  if (const int tile = legacy ? 0 : wide_selected(OUT_M, OUT_N, scm, scg, out))
-    return launch_wide(tile, GGEMM_OUT_BF16, lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N, slm,
-                       srm, scg, scm, scn, m_total, stream);
+  if (const int tile = mfma == Mfma::kK32 ? 0 : wide_selected(OUT_M, OUT_N, scm, scg, out))
+    return launch_wide(mfma == Mfma::kK128Swapped, tile, GGEMM_OUT_BF16, lhs, rhs, out, lhs_scale, rhs_scale,
+                       group_offs, G, OUT_M, OUT_N, slm, srm, scg, scm, scn, m_total, stream);
   int cus = 0;
   rc = device_cus(&cus);
   if (rc) return rc;
-  auto kern = legacy ? _grouped_variable_k_gemm_kernel_k32 : _grouped_variable_k_gemm_kernel;
+  auto kern = mfma == Mfma::kK32          ? _grouped_variable_k_gemm_kernel_k32
+              : mfma == Mfma::kK128Swapped ? _grouped_variable_k_gemm_kernel_swapped
+                                           : _grouped_variable_k_gemm_kernel;
   hipLaunchKernelGGL(kern, dim3(cus), dim3(ggemm::kThreads), ggemm::kDynLdsBytes, (hipStream_t)stream,
                      (const uint8_t*)lhs, (const uint8_t*)rhs, (uint16_t*)out, lhs_scale, rhs_scale, group_offs, G,
                      OUT_M, OUT_N, slm, srm, scg, scm, scn, (void*)nullptr, (void*)nullptr, m_total);
@@ -140,7 +150,7 @@ int ggemm_vark_wgrad_fp8_wide(const void* lhs, const void* rhs, void* out, const
   if ((tile != 256 && tile != 320) || fit == 0) return GGEMM_E_SHAPE;
   const int64_t w = out_mode == GGEMM_OUT_BF16 ? 1 : 2;   // strides in bf16 elements
   if (!wide_rows_aligned(out, w * stride_cm, w * stride_cg)) return GGEMM_E_ALIGN;   // 16-byte row chunks
-  return launch_wide(tile, out_mode, lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N, stride_lhs_m,
+  return launch_wide(false, tile, out_mode, lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N, stride_lhs_m,
                      stride_rhs_m, stride_cg, stride_cm, stride_cn, M_total, stream);
 }
 
@@ -148,7 +158,7 @@ int ggemm_vark_wgrad_fp8(const void* lhs, const void* rhs, void* out, const floa
                          const int64_t* group_offs, int32_t G, int32_t OUT_M, int32_t OUT_N, int32_t stride_lhs_m,
                          int32_t stride_rhs_m, int32_t stride_cg, int32_t stride_cm, int32_t stride_cn,
                          void* stream) {
-  return launch_tensorwise(false, lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N, stride_lhs_m,
+  return launch_tensorwise(Mfma::kK128, lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N, stride_lhs_m,
                            stride_rhs_m, stride_cg, stride_cm, stride_cn, INT64_MAX, stream);
 }
 
@@ -156,7 +166,7 @@ int ggemm_vark_wgrad_fp8_k32(const void* lhs, const void* rhs, void* out, const 
                              const float* rhs_scale, const int64_t* group_offs, int32_t G, int32_t OUT_M,
                              int32_t OUT_N, int32_t stride_lhs_m, int32_t stride_rhs_m, int32_t stride_cg,
                              int32_t stride_cm, int32_t stride_cn, void* stream) {
-  return launch_tensorwise(true, lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N, stride_lhs_m,
+  return launch_tensorwise(Mfma::kK32, lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N, stride_lhs_m,
                            stride_rhs_m, stride_cg, stride_cm, stride_cn, INT64_MAX, stream);
 }
 
@@ -166,7 +176,7 @@ int ggemm_vark_wgrad_fp8_out(const void* lhs, const void* rhs, void* out, const 
                              int32_t stride_cm, int32_t stride_cn, int32_t out_mode, int64_t M_total,
                              void* stream) {
   if (out_mode == GGEMM_OUT_BF16)
-    return launch_tensorwise(false, lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N, stride_lhs_m,
+    return launch_tensorwise(Mfma::kK128, lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N, stride_lhs_m,
                              stride_rhs_m, stride_cg, stride_cm, stride_cn, M_total, stream);
   if (out_mode != GGEMM_OUT_F32 && out_mode != GGEMM_OUT_F32_ACCUM) return GGEMM_E_FORMAT;
   int rc = validate_common(lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N, stride_lhs_m,
@@ -176,7 +186,7 @@ int ggemm_vark_wgrad_fp8_out(const void* lhs, const void* rhs, void* out, const 
   if (!aligned(out, 16)) return GGEMM_E_ALIGN;    // 16-byte fp32 row segments
   // fp32 C takes the 320 x 320 wide-tile kernel where the bf16 C of the same shape would
   if (wide_selected(OUT_M, OUT_N, 2 * (int64_t)stride_cm, 2 * (int64_t)stride_cg, out) == 320)
-    return launch_wide(320, out_mode, lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N,
+    return launch_wide(false, 320, out_mode, lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N,
                        stride_lhs_m, stride_rhs_m, stride_cg, stride_cm, stride_cn, M_total, stream);
   int cus = 0;
   rc = device_cus(&cus);
@@ -187,6 +197,14 @@ int ggemm_vark_wgrad_fp8_out(const void* lhs, const void* rhs, void* out, const 
                      OUT_N, stride_lhs_m, stride_rhs_m, stride_cg, stride_cm, stride_cn, (void*)nullptr, (void*)nullptr,
                      M_total);
   return (int)hipGetLastError();
+}
+
+int ggemm_vark_wgrad_fp8_swapped(const void* lhs, const void* rhs, void* out, const float* lhs_scale,
+                                 const float* rhs_scale, const int64_t* group_offs, int32_t G, int32_t OUT_M,
+                                 int32_t OUT_N, int32_t stride_lhs_m, int32_t stride_rhs_m, int32_t stride_cg,
+                                 int32_t stride_cm, int32_t stride_cn, int64_t M_total, void* stream) {
+  return launch_tensorwise(Mfma::kK128Swapped, lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N,
+                           stride_lhs_m, stride_rhs_m, stride_cg, stride_cm, stride_cn, M_total, stream);
 }
 
 // tile_m: 0 = the wide 320 x 320 kernel where the bf16 tensorwise entry would run it, else the

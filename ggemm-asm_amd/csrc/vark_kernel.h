@@ -371,7 +371,8 @@ __device__ __forceinline__ void static_for(F&& f) {
 
 // kSelA / kSelB: the byte of the 32-bit scale operand that holds this MFMA's e8m0 scale (block
 // scales are kept four to a register).
-template <bool kLegacyK32, int kSelA = 0, int kSelB = 0>
+// kSwapped: the RHS is e4m3 and the LHS e5m2.
+template <bool kLegacyK32, int kSelA = 0, int kSelB = 0, bool kSwapped = false>
 __device__ __forceinline__ v4f mfma(const v8i& a_rhs, const v8i& b_lhs, v4f acc, int sc_a, int sc_b) {
   if constexpr (kLegacyK32) {
     // four K=32 steps; the per-lane token pairing of A and B is identical, so the sum matches
@@ -383,8 +384,9 @@ __device__ __forceinline__ v4f mfma(const v8i& a_rhs, const v8i& b_lhs, v4f acc,
     }
     return acc;
   } else {
-    // A (RHS) is e5m2 -> format 1 (bf8); B (LHS) is e4m3 -> format 0 (fp8)
-    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a_rhs, b_lhs, acc, 1, 0, kSelA, sc_a, kSelB, sc_b);
+    // A (RHS) is e5m2 -> format 1 (bf8); B (LHS) is e4m3 -> format 0 (fp8); swapped, the reverse
+    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a_rhs, b_lhs, acc, kSwapped ? 0 : 1, kSwapped ? 1 : 0,
+                                                            kSelA, sc_a, kSelB, sc_b);
   }
 }
 
@@ -700,10 +702,11 @@ __device__ void poison_c(const VarKArgs& a) {
 // the bytes, and the accumulating epilogue also waits for the old values to arrive.
 constexpr int kEpiWF32 = 2, kEpiWF32Acc = 4;
 
-template <bool kMX, bool kLegacyK32, int kTN, int kOut = kOutBF16>
+template <bool kMX, bool kLegacyK32, int kTN, int kOut = kOutBF16, bool kSwapped = false>
 __device__ __forceinline__ void vark_body(const VarKArgs& a, GG_LDS uint8_t* lds) {
   static_assert(kOut == kOutBF16 || !kMX, "fp32 output modes are built for the tensorwise kernel");
   static_assert(!(kMX && kLegacyK32), "block scales need the scaled MFMA");
+  static_assert(!kSwapped || (kOut == kOutBF16 && !kMX && !kLegacyK32), "swapped formats: bf16 C, K=128 MFMA");
   using C = Cfg<kTN>;
   constexpr int NB = C::NB;
   const LdsMap lm = lds_map<kTN>(lds);
@@ -841,8 +844,8 @@ __device__ __forceinline__ void vark_body(const VarKArgs& a, GG_LDS uint8_t* lds
         constexpr int i = decltype(ic)::value;
         static_for<NB>([&](auto jc) {
           constexpr int j = decltype(jc)::value;
-          acc[i][j] = mfma<kLegacyK32, kMX ? j % 4 : 0, kMX ? i % 4 : 0>(bn[j], am[i & 1], acc[i][j], sc_n[j / 4],
-                                                                         sc_m[i / 4]);
+          acc[i][j] = mfma<kLegacyK32, kMX ? j % 4 : 0, kMX ? i % 4 : 0, kSwapped>(bn[j], am[i & 1], acc[i][j],
+                                                                                   sc_n[j / 4], sc_m[i / 4]);
         });
         if constexpr (i == 0 && kIssueFirst < C::DmaPerWave) {
           if (more)
@@ -1282,7 +1285,7 @@ __device__ __forceinline__ void vark_body32(const VarKArgs& a, GG_LDS uint8_t* l
 // Entry body shared by all kernels: checks the launch's LDS, then runs the 384-wide tile
 // configuration when OUT_N is a multiple of 384 (tensorwise kernels) and the 320-wide one
 // otherwise.
-template <bool kMX, bool kLegacyK32, int kOut = kOutBF16>
+template <bool kMX, bool kLegacyK32, int kOut = kOutBF16, bool kSwapped = false>
 __device__ __forceinline__ void vark_entry(const VarKArgs& a, GG_LDS uint8_t* dyn) {
   __shared__ __attribute__((aligned(1024))) uint8_t static_lds[kStaticLdsBytes];
   const hsa_kernel_dispatch_packet_t* pkt = dispatch_packet();
@@ -1299,9 +1302,9 @@ __device__ __forceinline__ void vark_entry(const VarKArgs& a, GG_LDS uint8_t* dy
     if constexpr (kMX)
       vark_body32(a, st);
     else
-      vark_body<false, kLegacyK32, 384, kOut>(a, st);
+      vark_body<false, kLegacyK32, 384, kOut, kSwapped>(a, st);
   } else {
-    vark_body<kMX, kLegacyK32, 320, kOut>(a, st);
+    vark_body<kMX, kLegacyK32, 320, kOut, kSwapped>(a, st);
   }
 }
 
@@ -1327,15 +1330,15 @@ __device__ __forceinline__ void vark_entry(const VarKArgs& a, GG_LDS uint8_t* dy
 
 // Library kernels: the same 16 arguments plus the token count M_total (group offsets clamped to
 // [0, M_total] on the device). CT / OUT: bf16 C (kOutBF16), or an fp32 C for the fp32 output
-// modes (kOutF32 / kOutF32Acc, strides in fp32 elements).
-#define GGEMM_DEFINE_TENSORWISE_LIB_KERNEL(NAME, LEGACY, CT, OUT)                                       \
+// modes (kOutF32 / kOutF32Acc, strides in fp32 elements). SWAPPED: e5m2 LHS, e4m3 RHS.
+#define GGEMM_DEFINE_TENSORWISE_LIB_KERNEL(NAME, LEGACY, CT, OUT, SWAPPED)                              \
   extern "C" __global__ __launch_bounds__(ggemm::kThreads) void NAME(GGEMM_VARK_TW_PARAMS(CT),           \
                                                                      int64_t m_total) {                  \
     extern __shared__ __attribute__((aligned(1024))) uint8_t ggemm_dyn_lds[];                           \
     ggemm::VarKArgs a{lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N,                  \
                       stride_lhs_m, stride_rhs_m, stride_cg, stride_cm, stride_cn, 0, 0, m_total};       \
     (void)global_scratch; (void)profile_scratch;                                                        \
-    ggemm::vark_entry<false, LEGACY, OUT>(a, (GG_LDS uint8_t*)ggemm_dyn_lds);                             \
+    ggemm::vark_entry<false, LEGACY, OUT, SWAPPED>(a, (GG_LDS uint8_t*)ggemm_dyn_lds);                   \
   }
 
 #define GGEMM_DEFINE_MX_KERNEL(NAME)                                                                    \

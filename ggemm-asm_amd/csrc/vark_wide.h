@@ -84,12 +84,14 @@ __device__ __forceinline__ uint32_t hi32(const void* p) {
 
 // OUT: kOutBF16 (bf16 C), kOutF32 (fp32 C) or kOutF32Acc (fp32 C += result); the fp32 modes are
 // built for 320 x 320 tiles. MX: e8m0 block scales (one per 32 tokens and column) applied by the
-// scaled MFMA, bf16 C, 320 x 320 tiles.
-template <int TM, int TN, int OUT = kOutBF16, bool MX = false>
+// scaled MFMA, bf16 C, 320 x 320 tiles. SWAPPED: e5m2 LHS and e4m3 RHS (dW[g] = dy_g^T x_g in the
+// weight's own [N, K] orientation), bf16 C.
+template <int TM, int TN, int OUT = kOutBF16, bool MX = false, bool SWAPPED = false>
 __device__ __forceinline__ void vark_wide_body(const VarKArgs& a, GG_LDS uint8_t* lds) {
   using namespace wide;
   static_assert(OUT == kOutBF16 || (TM == 320 && TN == 320), "fp32 epilogues of the 320 x 320 tile");
   static_assert(!MX || (OUT == kOutBF16 && TM == 320 && TN == 320), "MX: bf16 C, 320 x 320 tiles");
+  static_assert(!SWAPPED || (OUT == kOutBF16 && !MX), "swapped formats: bf16 C");
   using CT = std::conditional_t<OUT == kOutBF16, uint16_t, float>;
   constexpr int kCB = sizeof(CT);                 // bytes per C element
   constexpr int BM = TM / 64, BN = TN / 64;       // 32-wide blocks per wave, 2 x 2 waves
@@ -203,12 +205,17 @@ __device__ __forceinline__ void vark_wide_body(const VarKArgs& a, GG_LDS uint8_t
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
     if constexpr (TM == 256 && TN == 384) {
-      asm volatile(GGEMM_WIDE_ASM_256x384 GGEMM_WIDE_SCALAR_OPERANDS,
-                   "v"(voffl[0]), "v"(voffl[1]), "v"(voffl[2]), "v"(voffl[3]), "v"(voffr[0]), "v"(voffr[1]),
-                   "v"(voffr[2]), "v"(voffr[3]), "v"(voffr[4]), "v"(voffr[5]), "v"(amb[0]), "v"(amb[1]),
-                   "v"(amb[2]), "v"(amb[3]), "v"(bnb[0]), "v"(bnb[1]), "v"(bnb[2]), "v"(bnb[3]), "v"(bnb[4]),
-                   "v"(bnb[5]), "v"(ew_base), "v"(ew_s), "v"(rb_even), "v"(rb_odd), "v"(gb)
-                   : GGEMM_WIDE_CLOBBERS_256x384);
+#define GGEMM_WIDE_OPERANDS_256x384 \
+  GGEMM_WIDE_SCALAR_OPERANDS, \
+    "v"(voffl[0]), "v"(voffl[1]), "v"(voffl[2]), "v"(voffl[3]), "v"(voffr[0]), "v"(voffr[1]), \
+    "v"(voffr[2]), "v"(voffr[3]), "v"(voffr[4]), "v"(voffr[5]), "v"(amb[0]), "v"(amb[1]), \
+    "v"(amb[2]), "v"(amb[3]), "v"(bnb[0]), "v"(bnb[1]), "v"(bnb[2]), "v"(bnb[3]), "v"(bnb[4]), \
+    "v"(bnb[5]), "v"(ew_base), "v"(ew_s), "v"(rb_even), "v"(rb_odd), "v"(gb)
+      if constexpr (SWAPPED)
+        asm volatile(GGEMM_WIDE_ASM_256x384_swapped GGEMM_WIDE_OPERANDS_256x384 : GGEMM_WIDE_CLOBBERS_256x384_swapped);
+      else
+        asm volatile(GGEMM_WIDE_ASM_256x384 GGEMM_WIDE_OPERANDS_256x384 : GGEMM_WIDE_CLOBBERS_256x384);
+#undef GGEMM_WIDE_OPERANDS_256x384
     } else if constexpr (MX) {
       const int amb0 = amb[0], amb1 = amb[1] - 32, bnb0 = bnb[0], bnb1 = bnb[1] - 32;
       asm volatile(GGEMM_WIDE_ASM_320x320_mx GGEMM_WIDE_SCALAR_OPERANDS,
@@ -236,11 +243,16 @@ __device__ __forceinline__ void vark_wide_body(const VarKArgs& a, GG_LDS uint8_t
       // two read bases per side: block b reads at base[b & 1] + 32 b (the one-bit swizzle of
       // 320-byte rows moves a chunk pair by +-32 bytes with the parity of its index)
       const int amb0 = amb[0], amb1 = amb[1] - 32, bnb0 = bnb[0], bnb1 = bnb[1] - 32;
-      asm volatile(GGEMM_WIDE_ASM_320x320 GGEMM_WIDE_SCALAR_OPERANDS,
-                   "v"(voffl[0]), "v"(voffl[1]), "v"(voffl[2]), "v"(voffl[3]), "v"(voffl[4]), "v"(voffr[0]),
-                   "v"(voffr[1]), "v"(voffr[2]), "v"(voffr[3]), "v"(voffr[4]), "v"(amb0), "v"(amb1), "v"(bnb0),
-                   "v"(bnb1), "v"(ew_base), "v"(ew_s), "v"(rb_even), "v"(rb_odd), "v"(gb)
-                   : GGEMM_WIDE_CLOBBERS_320x320);
+#define GGEMM_WIDE_OPERANDS_320x320 \
+  GGEMM_WIDE_SCALAR_OPERANDS, \
+    "v"(voffl[0]), "v"(voffl[1]), "v"(voffl[2]), "v"(voffl[3]), "v"(voffl[4]), "v"(voffr[0]), \
+    "v"(voffr[1]), "v"(voffr[2]), "v"(voffr[3]), "v"(voffr[4]), "v"(amb0), "v"(amb1), "v"(bnb0), \
+    "v"(bnb1), "v"(ew_base), "v"(ew_s), "v"(rb_even), "v"(rb_odd), "v"(gb)
+      if constexpr (SWAPPED)
+        asm volatile(GGEMM_WIDE_ASM_320x320_swapped GGEMM_WIDE_OPERANDS_320x320 : GGEMM_WIDE_CLOBBERS_320x320_swapped);
+      else
+        asm volatile(GGEMM_WIDE_ASM_320x320 GGEMM_WIDE_OPERANDS_320x320 : GGEMM_WIDE_CLOBBERS_320x320);
+#undef GGEMM_WIDE_OPERANDS_320x320
     }
 #pragma clang diagnostic pop
     c0 = (c0 + (uint32_t)T.nsteps) % 3u;
@@ -256,15 +268,16 @@ __device__ __forceinline__ void vark_wide_body(const VarKArgs& a, GG_LDS uint8_t
 }  // namespace ggemm
 
 // Library kernels: the tensorwise kernel's 16 arguments plus M_total, 256 threads, 136 KiB of
-// static LDS and no dynamic LDS. CT / OUT: bf16 C (kOutBF16) or fp32 C (kOutF32, kOutF32Acc).
-#define GGEMM_DEFINE_WIDE_KERNEL(NAME, TM, TN, CT, OUT)                                                  \
+// static LDS and no dynamic LDS. CT / OUT: bf16 C (kOutBF16) or fp32 C (kOutF32, kOutF32Acc);
+// SWAPPED: e5m2 LHS, e4m3 RHS.
+#define GGEMM_DEFINE_WIDE_KERNEL(NAME, TM, TN, CT, OUT, SWAPPED)                                         \
   extern "C" __global__ __launch_bounds__(ggemm::wide::kNT) __attribute__((amdgpu_waves_per_eu(1, 1)))   \
   void NAME(GGEMM_VARK_TW_PARAMS(CT), int64_t m_total) {                                                \
     __shared__ __attribute__((aligned(1024))) uint8_t ggemm_wide_lds[ggemm::wide::kLdsBytes];            \
     ggemm::VarKArgs a{lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N,                  \
                       stride_lhs_m, stride_rhs_m, stride_cg, stride_cm, stride_cn, 0, 0, m_total};       \
     (void)global_scratch; (void)profile_scratch;                                                        \
-    if (G > 0) ggemm::vark_wide_body<TM, TN, OUT>(a, (GG_LDS uint8_t*)ggemm_wide_lds);                   \
+    if (G > 0) ggemm::vark_wide_body<TM, TN, OUT, false, SWAPPED>(a, (GG_LDS uint8_t*)ggemm_wide_lds);   \
   }
 
 // MXFP8 library kernel, 320 x 320 tiles: the MX kernel's arguments without the scratch pointers,

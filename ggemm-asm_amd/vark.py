@@ -147,6 +147,25 @@ def grouped_gemm_fp8_tensorwise_variable_k(lhs: torch.Tensor, rhs: torch.Tensor,
     return out
 
 
+def weight_grad_fp8(dy: torch.Tensor, x: torch.Tensor, dy_scale: torch.Tensor, x_scale: torch.Tensor,
+                    group_offs: torch.Tensor) -> torch.Tensor:
+    """``dw[g] = dy_scale * x_scale * dy[offs[g]:offs[g+1]]^T @ x[offs[g]:offs[g+1]]``, bf16 [G, N, K]:
+    the weight gradient in the weight's own orientation. dy: float8_e5m2 [M_total, N]; x:
+    float8_e4m3fn [M_total, K]; scales: fp32 scalar tensors on the device."""
+    _check_inputs(dy, x, group_offs, (torch.float8_e5m2,), (torch.float8_e4m3fn,))
+    G = group_offs.numel() - 1
+    M_total, N = dy.shape
+    out = torch.empty((G, N, x.shape[1]), dtype=torch.bfloat16, device=dy.device)
+    dy, x = _nonempty(dy), _nonempty(x)
+    with torch.cuda.device(dy.device):
+        rc = _lib.load().ggemm_vark_wgrad_fp8_swapped(
+            dy.data_ptr(), x.data_ptr(), out.data_ptr(), dy_scale.data_ptr(), x_scale.data_ptr(),
+            group_offs.data_ptr(), G, N, x.shape[1], dy.stride(0), x.stride(0), out.stride(0), out.stride(1), 1,
+            M_total, _stream(dy.device))
+    _lib.check(rc, "ggemm_vark_wgrad_fp8_swapped")
+    return out
+
+
 def grouped_gemm_mxfp8_variable_k(lhs: torch.Tensor, rhs: torch.Tensor, lhs_scale: torch.Tensor,
                                   rhs_scale: torch.Tensor, group_offs: torch.Tensor,
                                   out: torch.Tensor | None = None, *, validate: bool = False,

@@ -17,7 +17,7 @@
 extern "C" {
 #endif
 
-#define GGEMM_VARK_ABI_VERSION 9
+#define GGEMM_VARK_ABI_VERSION 10
 
 enum {
   GGEMM_OK = 0,
@@ -97,6 +97,15 @@ int ggemm_vark_wgrad_fp8_wide(const void* lhs, const void* rhs, void* out, const
                               int32_t OUT_N, int32_t stride_lhs_m, int32_t stride_rhs_m, int32_t stride_cg,
                               int32_t stride_cm, int32_t stride_cn, int64_t M_total, int32_t tile_m,
                               int32_t out_mode, void* stream);
+
+/* ggemm_vark_wgrad_fp8_out with bf16 C for an e5m2 LHS and an e4m3 RHS: C[g] = dy_g^T x_g, a linear
+ * layer's weight gradient in the weight's own [N, K] orientation (the e4m3 x e5m2 entry points give
+ * x_g^T dy_g, its transpose). No reference counterpart. Same kernels but for the operand formats,
+ * same arguments, checks and choice of kernel. */
+int ggemm_vark_wgrad_fp8_swapped(const void* lhs, const void* rhs, void* out, const float* lhs_scale,
+                                 const float* rhs_scale, const int64_t* group_offs, int32_t G, int32_t OUT_M,
+                                 int32_t OUT_N, int32_t stride_lhs_m, int32_t stride_rhs_m, int32_t stride_cg,
+                                 int32_t stride_cm, int32_t stride_cn, int64_t M_total, void* stream);
 
 /* MXFP8 block-scaled grouped wgrad (no reference counterpart: the reference imports only the
  * tensorwise kernels, reference bench.py:241-246). lhs_scale: e8m0 bytes [ceil(M_total/32), OUT_M]
