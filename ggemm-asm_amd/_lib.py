@@ -56,6 +56,7 @@ PERSISTENT_EXPORTS = (
     "ggemm_persistent_fp8",
     "ggemm_persistent_fp8_kernel",
     "ggemm_persistent_selected_kernel",
+    "ggemm_persistent_tile_rows",
     "ggemm_persistent_clear_tail",
     "ggemm_persistent_transpose_u8",
 )
@@ -144,6 +145,8 @@ def load():
     lib.ggemm_persistent_fp8_kernel.restype = ctypes.c_int
     lib.ggemm_persistent_selected_kernel.argtypes = [i32] * 5
     lib.ggemm_persistent_selected_kernel.restype = ctypes.c_int32
+    lib.ggemm_persistent_tile_rows.argtypes = [i32] * 6 + [i64, i32]
+    lib.ggemm_persistent_tile_rows.restype = ctypes.c_int32
     lib.ggemm_persistent_clear_tail.argtypes = [vp, i32, i32, vp, i32, i64, vp]
     lib.ggemm_persistent_clear_tail.restype = ctypes.c_int
     lib.ggemm_persistent_transpose_u8.argtypes = [vp, i32, i32, i32, i64, i64, vp, i64, i64, vp]

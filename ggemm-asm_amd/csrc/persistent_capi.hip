@@ -1,14 +1,18 @@
 // extern "C" launcher of the persistent grouped FP8 GEMM (forward / data-gradient sites), part of
 // libggemm_vark.so. Validates arguments on the host, then launches either the kernel of the
 // reference's geometry (grid (num_cus, 1, 1), block (512, 1, 1), 64 KiB dynamic LDS, reference
-// bench.py:339-355) or, for the shapes it takes, the wide-tile kernel (persistent_wide.h: grid
-// (num_cus, 1, 1), block (256, 1, 1), 160 KiB static LDS).
+// bench.py:339-355) for the shapes it takes, the wide-tile kernel (persistent_wide.h: grid
+// (num_cus, 1, 1), block (256, 1, 1), 160 KiB static LDS), or, for launches of too few such tiles, the
+// mid-tile kernel (mid_gemm.h: one tile per 256-thread workgroup).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
 #include <cstdint>
 
 #include "../../include/ggemm_persistent.h"
 #include "capi_common.h"
+#include "mid_gemm.h"
 #include "persistent_kernel.h"
 #include "persistent_wide.h"
 #include "transpose_tile.h"
@@ -17,6 +21,10 @@ GGEMM_DEFINE_PERSISTENT_LIB_KERNEL(_grouped_fp8_persistent_gemm_kernel, false)
 GGEMM_DEFINE_PERSISTENT_LIB_KERNEL(_grouped_fp8_persistent_gemm_kernel_e5m2, true)
 GGEMM_DEFINE_PERSISTENT_WIDE_KERNEL(_grouped_fp8_persistent_gemm_kernel_wide, false)
 GGEMM_DEFINE_PERSISTENT_WIDE_KERNEL(_grouped_fp8_persistent_gemm_kernel_wide_e5m2, true)
+GGEMM_DEFINE_MID_GEMM_KERNEL(_grouped_fp8_gemm_kernel_mid64, false, 64)
+GGEMM_DEFINE_MID_GEMM_KERNEL(_grouped_fp8_gemm_kernel_mid64_e5m2, true, 64)
+GGEMM_DEFINE_MID_GEMM_KERNEL(_grouped_fp8_gemm_kernel_mid128, false, 128)
+GGEMM_DEFINE_MID_GEMM_KERNEL(_grouped_fp8_gemm_kernel_mid128_e5m2, true, 128)
 
 static_assert(GGEMM_PERSISTENT_MAX_GROUPS == ggemm::nt::kMaxGroups, "header and kernel agree");
 
@@ -127,6 +135,41 @@ bool wide_fits(int N, int K, int sam, int sbn, int scm) {
 // four sites, same box), on line-aligned rows more.
 bool wide_preferred(int N, int K, int sam, int sbn, int scm) { return wide_fits(N, K, sam, sbn, scm); }
 
+int64_t mid_tiles(int rows, int G, int N, int64_t M_total) {
+  return (M_total / rows + (G < M_total ? G : M_total)) * ((N + 127) / 128);
+}
+
+// The mid-tile kernel's row-tile height (64 or 128) where it is the faster one, else 0: the estimated
+// microseconds of each kernel compared. The lengths of the groups are on the device; M_total rows over
+// G groups are taken to make max(g, M_total / height + g / 2) row tiles, g the groups that can have a
+// row. Per 128-byte K stage and tile: 2.1 us for the persistent kernels with every CU busy (1.7 with
+// few), their tiles one to a CU in whole rounds, 12 us around them; 0.84 / 1.26 us for the mid tiles
+// of 64 / 128 rows with two workgroups on every CU (0.41 / 0.64 with few), 4 us around them, and they
+// feel the memory's time too. Measured (us, the better of 512-thread and wide kernel -> the choice):
+// N = 5760, K = 2880, G = 32: 256 rows 136 -> 95 (64), 2048 rows 129 -> 109 (128), 6144 rows 161, mid
+// 186 (stays); N = K = 2880, G = 4: 512 rows 52 -> 14, 8192 rows 89 -> 70, 16384 rows 137, mid 151
+// (stays); N = 2048, K = 1424, G = 7: 5003 rows 40 -> 32, 20000 rows 86, mid 93 (stays).
+int mid_preferred(int G, int N, int K, int scm, int64_t M_total, bool wide, int cus) {
+  if (G > ggemm::mid::kMaxGroups || M_total <= 0 || mid_tiles(64, G, N, M_total) > (1 << 22)) return 0;
+  if ((int64_t)scm * 2 * 64 >= (int64_t)ggemm::nt::kOob) return 0;   // a wave's rows of C: 32-bit offsets
+  const double M = (double)M_total, g = G < M ? G : M;
+  const double stages = (K + 127) / 128 + 2;                          // two more for the tile's ends
+  const double mem = (M * K + g * N * K + 2 * M * N) / 5.1e6;
+  auto tiles = [&](double h, double w) { return std::max(g, M / h + g / 2) * std::ceil(N / w); };
+  double big;
+  if (wide) {
+    big = 12 + std::ceil(tiles(256, 320) / cus) * stages * 1.85;
+  } else {
+    const int tn = ggemm::wide_tiles(N, false) ? 384 : 320;
+    big = 12 + std::ceil(tiles(192, tn) / cus) * stages * (tn == 384 ? 1.75 : 1.58) + 0.2 * mem;
+  }
+  const double f64 = tiles(64, 128) / (2 * cus), f128 = tiles(128, 128) / (2 * cus);
+  const double c64 = 4 + std::max(1.0, f64) * stages * (0.41 + 0.28 * std::min(1.0, f64)) + 0.3 * mem;
+  const double c128 = 4 + std::max(1.0, f128) * stages * (0.64 + 0.42 * std::min(1.0, f128)) + 0.3 * mem;
+  if (std::min(c64, c128) >= 0.92 * big) return 0;   // near the line the estimate is a few per cent off
+  return c64 <= c128 ? 64 : 128;
+}
+
 int launch(const void* a, const void* b, void* out, const float* a_scale, const float* b_scale,
            const int64_t* group_offs, int G, int N, int K, int sam, int sbg, int sbn, int scm, int scn, int fmt,
            int64_t M_total, int kernel, void* stream) {
@@ -134,7 +177,8 @@ int launch(const void* a, const void* b, void* out, const float* a_scale, const 
   if (rc) return rc;
   const bool fits = wide_fits(N, K, sam, sbn, scm);
   if (kernel == GGEMM_PERSISTENT_KERNEL_WIDE && !fits) return GGEMM_E_SHAPE;
-  if (kernel == GGEMM_PERSISTENT_KERNEL_AUTO)
+  const bool automatic = kernel == GGEMM_PERSISTENT_KERNEL_AUTO;
+  if (automatic)
     kernel = wide_preferred(N, K, sam, sbn, scm) ? GGEMM_PERSISTENT_KERNEL_WIDE : GGEMM_PERSISTENT_KERNEL_512;
   if (kernel < GGEMM_PERSISTENT_KERNEL_AUTO || kernel > GGEMM_PERSISTENT_KERNEL_WIDE) return GGEMM_E_SHAPE;
   int cus = 0;
@@ -142,6 +186,17 @@ int launch(const void* a, const void* b, void* out, const float* a_scale, const 
   if (rc) return rc;
   if (M_total == 0) return GGEMM_OK;   // no rows: nothing to write
   const bool e5m2 = fmt == GGEMM_FP8_E5M2;
+  const int mid = automatic ? mid_preferred(G, N, K, scm, M_total, kernel == GGEMM_PERSISTENT_KERNEL_WIDE, cus) : 0;
+  if (mid) {
+    auto kern = mid == 64 ? (e5m2 ? _grouped_fp8_gemm_kernel_mid64_e5m2 : _grouped_fp8_gemm_kernel_mid64)
+                          : (e5m2 ? _grouped_fp8_gemm_kernel_mid128_e5m2 : _grouped_fp8_gemm_kernel_mid128);
+    // at most one partial row tile per group, none for a group without rows; whole runs of 8 XCDs
+    const int64_t tiles = mid_tiles(mid, G, N, M_total), run = ggemm::kXcds * ggemm::mid::kXcdRun;
+    hipLaunchKernelGGL(kern, dim3((uint32_t)((tiles + run - 1) / run * run)), dim3(ggemm::mid::kNT), 0,
+                       (hipStream_t)stream, (const uint8_t*)a, (const uint8_t*)b, (uint16_t*)out, a_scale, b_scale,
+                       group_offs, G, N, K, sam, sbg, sbn, scm, scn, (void*)nullptr, (void*)nullptr, M_total);
+    return (int)hipGetLastError();
+  }
   if (kernel == GGEMM_PERSISTENT_KERNEL_WIDE) {
     auto kern = e5m2 ? _grouped_fp8_persistent_gemm_kernel_wide_e5m2 : _grouped_fp8_persistent_gemm_kernel_wide;
     hipLaunchKernelGGL(kern, dim3(cus), dim3(ggemm::pw::kNT), 0, (hipStream_t)stream, (const uint8_t*)a,
@@ -180,6 +235,13 @@ int32_t ggemm_persistent_selected_kernel(int32_t N, int32_t K, int32_t stride_am
                                          int32_t stride_cm) {
   return wide_preferred(N, K, stride_am, stride_bn, stride_cm) ? GGEMM_PERSISTENT_KERNEL_WIDE
                                                                : GGEMM_PERSISTENT_KERNEL_512;
+}
+
+int32_t ggemm_persistent_tile_rows(int32_t G, int32_t N, int32_t K, int32_t stride_am, int32_t stride_bn,
+                                   int32_t stride_cm, int64_t M_total, int32_t num_cus) {
+  const bool wide = wide_preferred(N, K, stride_am, stride_bn, stride_cm);
+  const int mid = mid_preferred(G, N, K, stride_cm, M_total, wide, num_cus);
+  return mid ? mid : wide ? ggemm::pw::kTM : ggemm::kTileM;
 }
 
 int ggemm_persistent_clear_tail(void* out, int32_t N, int32_t stride_cm, const int64_t* group_offs, int32_t G,

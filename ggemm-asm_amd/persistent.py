@@ -27,9 +27,17 @@ KERNELS = {"auto": 0, "512": 1, "wide": 2}
 
 
 def selected_kernel(N: int, K: int, stride_am: int, stride_bn: int, stride_cm: int) -> str:
-    """The kernel the library runs for this shape and these strides ("512" or "wide")."""
+    """The kernel the library runs for this shape and these strides ("512" or "wide") when there are
+    rows enough to fill its tiles (see ``tile_rows``)."""
     k = _lib.load().ggemm_persistent_selected_kernel(N, K, stride_am, stride_bn, stride_cm)
     return {v: n for n, v in KERNELS.items()}[k]
+
+
+def tile_rows(G: int, N: int, K: int, stride_am: int, stride_bn: int, stride_cm: int, M_total: int,
+              num_cus: int = 256) -> int:
+    """Rows of the output tiles of the kernel that the automatic choice runs: 256 (wide), 192
+    (512-thread), 128 or 64 (the mid-tile kernel, for launches of few rows)."""
+    return _lib.load().ggemm_persistent_tile_rows(G, N, K, stride_am, stride_bn, stride_cm, M_total, num_cus)
 
 
 def _a_format(a: torch.Tensor, a_format: str | None) -> int:
@@ -81,7 +89,8 @@ def grouped_gemm_fp8_tensorwise(a: torch.Tensor, b: torch.Tensor, a_scale: torch
     are left unwritten, or set to zero with ``zero_tail=True`` (the library's device-side clear, no
     sync: dropped tokens get exact zeros). ``validate=True`` checks group_offs on the host first (a
     sync). Offsets past M_total are clamped to it on the device. ``kernel``: "auto" (the library's
-    choice: the wide-tile kernel where N % 320 == 0 and K % 64 == 0, else the 512-thread kernel),
+    choice: the wide-tile kernel where N % 320 == 0 and K % 64 == 0, else the 512-thread kernel; the
+    mid-tile kernel for launches of few rows, ``tile_rows``),
     "512" or "wide" (GGemmError GGEMM_E_SHAPE where the wide kernel does not apply).
     """
     if a.dim() != 2 or b.dim() != 3:

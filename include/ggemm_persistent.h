@@ -57,7 +57,8 @@ int ggemm_persistent_fp8(const void* a, const void* b, void* out, const float* a
  * also the drop-in code objects) and a wide-tile kernel (256 threads, one wave per SIMD, 256 x 320
  * tiles, 160 KiB of LDS) for N % 320 == 0, K % 64 == 0, 256*stride_am, 320*stride_bn and
  * 512*stride_cm below 2^31 - 2^16. ggemm_persistent_fp8 runs the wide kernel wherever it applies
- * (faster at every measured shape, most on line-aligned rows of 128-byte multiples). */
+ * (faster at every measured shape, most on line-aligned rows of 128-byte multiples), unless the
+ * launch has too few rows for either (ggemm_persistent_tile_rows). */
 #define GGEMM_PERSISTENT_KERNEL_AUTO 0
 #define GGEMM_PERSISTENT_KERNEL_512 1
 #define GGEMM_PERSISTENT_KERNEL_WIDE 2
@@ -70,10 +71,18 @@ int ggemm_persistent_fp8_kernel(const void* a, const void* b, void* out, const f
                                 int32_t stride_bg, int32_t stride_bn, int32_t stride_cm, int32_t stride_cn,
                                 int32_t a_format, int64_t M_total, int32_t kernel, void* stream);
 
-/* The kernel ggemm_persistent_fp8 runs for this shape and these strides (_512 or _WIDE). No
- * reference counterpart. */
+/* The kernel ggemm_persistent_fp8 runs for this shape and these strides (_512 or _WIDE) when there
+ * are rows enough to fill its tiles. No reference counterpart. */
 int32_t ggemm_persistent_selected_kernel(int32_t N, int32_t K, int32_t stride_am, int32_t stride_bn,
                                          int32_t stride_cm);
+
+/* Rows of the output tiles of the kernel that ggemm_persistent_fp8 runs for a launch on a device of
+ * num_cus compute units: 256 (wide), 192 (512-thread), or 128 / 64, the mid-tile kernel: one
+ * 128- or 64-row x 128-column tile per 256-thread workgroup, several workgroups per CU, for at most
+ * 256 groups whose rows would leave most of the larger tiles' rows or of the CUs unused. Its results
+ * are the 512-thread kernel's bit for bit. No reference counterpart. Touches no device. */
+int32_t ggemm_persistent_tile_rows(int32_t G, int32_t N, int32_t K, int32_t stride_am, int32_t stride_bn,
+                                   int32_t stride_cm, int64_t M_total, int32_t num_cus);
 
 /* Zeroes rows [min(offs[G], M_total), M_total) of out (bf16 [M_total, N], row stride stride_cm):
  * the rows ggemm_persistent_fp8 leaves unwritten when routing drops tokens (offs[G] < M_total).
