@@ -49,6 +49,7 @@ EXPORTS = (
     "ggemm_vark_strerror",
     "ggemm_vark_abi_version",
     "ggemm_vark_bf16_kernel",
+    "ggemm_vark_tile_rows",
     "ggemm_vark_launch_geometry",
 )
 
@@ -137,6 +138,8 @@ def load():
     lib.ggemm_vark_abi_version.restype = ctypes.c_int32
     lib.ggemm_vark_bf16_kernel.argtypes = [i32, i32, i32, vp]
     lib.ggemm_vark_bf16_kernel.restype = ctypes.c_int32
+    lib.ggemm_vark_tile_rows.argtypes = [i32] * 5 + [i64, i32]
+    lib.ggemm_vark_tile_rows.restype = ctypes.c_int32
     lib.ggemm_vark_launch_geometry.argtypes = [i32] + [ctypes.POINTER(ctypes.c_int32)] * 5
     lib.ggemm_vark_launch_geometry.restype = None
     lib.ggemm_persistent_fp8.argtypes = [vp, vp, vp, vp, vp, vp] + [i32] * 9 + [i64, vp]
@@ -189,7 +192,7 @@ def check(code: int, what: str) -> None:
 def bf16_kernel(out_m: int, out_n: int, stride_cm: int | None = None) -> str:
     """Which kernel the bf16 wgrad entry points run for this shape (a 256-byte aligned C assumed):
     "wide320" / "wide256" (320 x 320 / 256 x 384 tiles, one wave per SIMD) or "192-row" (the
-    reference launch geometry)."""
+    reference launch geometry), when there are tokens enough to fill its tiles."""
     sel = load().ggemm_vark_bf16_kernel(int(out_m), int(out_n), int(stride_cm or out_n), 256)
     return {320: "wide320", 256: "wide256"}.get(sel, "192-row")
 

@@ -1,13 +1,17 @@
 // extern "C" launcher library for the variable-K FP8 grouped wgrad kernels (libggemm_vark.so).
 // Validates arguments on the host, then launches the persistent kernel with the reference's
 // geometry: grid (num_cus, 1, 1), block (512, 1, 1), 64 KiB dynamic LDS
-// (reference launcher.cpp:142-171, bench.py:388-398).
+// (reference launcher.cpp:142-171, bench.py:388-398), or the wide-tile (vark_wide.h) or the mid-tile
+// kernel (mid_wgrad.h) where it serves the launch better.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
 #include <cstdint>
 
 #include "../../include/ggemm_vark.h"
 #include "capi_common.h"
+#include "mid_wgrad.h"
 #include "vark_kernel.h"
 #include "vark_wide.h"
 
@@ -23,6 +27,10 @@ GGEMM_DEFINE_WIDE_KERNEL(_grouped_variable_k_gemm_kernel_wide320_f32_acc, 320, 3
 GGEMM_DEFINE_TENSORWISE_LIB_KERNEL(_grouped_variable_k_gemm_kernel_swapped, false, uint16_t, ggemm::kOutBF16, true)
 GGEMM_DEFINE_WIDE_KERNEL(_grouped_variable_k_gemm_kernel_wide_swapped, 256, 384, uint16_t, ggemm::kOutBF16, true)
 GGEMM_DEFINE_WIDE_KERNEL(_grouped_variable_k_gemm_kernel_wide320_swapped, 320, 320, uint16_t, ggemm::kOutBF16, true)
+GGEMM_DEFINE_MID_WGRAD_KERNEL(_grouped_variable_k_gemm_kernel_mid, uint16_t, ggemm::kOutBF16, false)
+GGEMM_DEFINE_MID_WGRAD_KERNEL(_grouped_variable_k_gemm_kernel_mid_swapped, uint16_t, ggemm::kOutBF16, true)
+GGEMM_DEFINE_MID_WGRAD_KERNEL(_grouped_variable_k_gemm_kernel_mid_f32, float, ggemm::kOutF32, false)
+GGEMM_DEFINE_MID_WGRAD_KERNEL(_grouped_variable_k_gemm_kernel_mid_f32_acc, float, ggemm::kOutF32Acc, false)
 GGEMM_DEFINE_WIDE_MX_KERNEL(_grouped_variable_k_mxfp8_gemm_kernel_wide320)
 
 namespace {
@@ -73,6 +81,42 @@ int wide_selected(int OUT_M, int OUT_N, int64_t scm, int64_t scg, const void* ou
   return OUT_M >= 1024 && wide_rows_aligned(out, scm, scg) ? wide_tile_for(OUT_M, OUT_N, (int)scm) : 0;
 }
 
+int64_t mid_tiles(int G, int OUT_M, int OUT_N) {
+  return (int64_t)G * ((OUT_M + ggemm::mid::kWT - 1) / ggemm::mid::kWT) *
+         ((OUT_N + ggemm::mid::kWT - 1) / ggemm::mid::kWT);
+}
+
+// Whether the mid-tile kernel is the faster one: the estimated microseconds of both sides compared,
+// M_total / G tokens in every group. Per 128-token stage and tile: 2.06 us for a wide tile and 1.2
+// (few CUs busy) to 2.1 us for a 192-row one, tiles one to a CU in whole rounds, 12 us around them;
+// 0.55 (few) to 1.27 us (two workgroups on every CU) for a mid tile, 4 us around them; a tile's ends
+// cost 3 stages more (an fp32 C: 4; wide 7 us, 13). wide_tile: the wide kernel the entry would run, 0 the
+// 192-row kernel. Measured (us, large -> mid): 64 x 128, 512 tokens, G = 4: 21 -> 5.3; 2880 x 2880, G = 4:
+// 1024 tokens 37 -> 31, 4096 tokens 56, mid 60 (stays), accumulated fp32 92 -> 77; 512 x 1024, G = 8:
+// 1000 tokens 25 -> 6.5, 100000 tokens 148 -> 69; 1600 x 1600, G = 12, 1000 tokens: 33 -> 24, accumulated
+// 73 -> 42, 100000 tokens 292, mid 352 (stays). The fp32 modes take one line for both, so that
+// accumulating adds exactly what the fp32 mode writes. No token count (INT64_MAX): the large kernels.
+bool mid_preferred(int G, int OUT_M, int OUT_N, int64_t scm, int64_t scg, const void* out, bool f32, int64_t M_total,
+                   int wide_tile, int cus) {
+  const int64_t w = f32 ? 2 : 1;                             // strides in bf16 elements
+  if (G > ggemm::mid::kMaxGroups || M_total > INT32_MAX || !wide_rows_aligned(out, w * scm, w * scg)) return false;
+  if (scm * 2 * w * 64 >= (int64_t)ggemm::mid::kOob) return false;   // a wave's rows of C: 32-bit offsets
+  if (mid_tiles(G, OUT_M, OUT_N) > (1 << 22)) return false;
+  const double stages = (double)M_total / G / ggemm::kKStep + 0.5;
+  auto tiles = [&](int h, int n) { return (double)G * ((OUT_M + h - 1) / h) * ((OUT_N + n - 1) / n); };
+  const double f = tiles(ggemm::mid::kWT, ggemm::mid::kWT) / (2 * cus);
+  const double mid = 4 + std::max(1.0, f) * (stages + (f32 ? 4 : 3)) * (0.55 + 0.72 * std::min(1.0, f));
+  double big;
+  if (wide_tile) {
+    const double t = wide_tile == 320 ? tiles(320, 320) : tiles(256, 384);
+    big = 12 + std::ceil(t / cus) * (stages * 2.06 + (f32 ? 13 : 7));
+  } else {
+    const double t = tiles(ggemm::kTileM, ggemm::wide_tiles(OUT_N, false) ? 384 : 320) / cus;
+    big = 12 + std::ceil(t) * (stages + 3) * (1.2 + 0.9 * std::min(1.0, t));
+  }
+  return mid < 0.92 * big;                                   // near the line the estimate is a few per cent off
+}
+
 // swapped: e5m2 LHS, e4m3 RHS (bf16 C only)
 int launch_wide(bool swapped, int tile, int out_mode, const void* lhs, const void* rhs, void* out,
                 const float* lhs_scale, const float* rhs_scale, const int64_t* group_offs, int32_t G, int32_t OUT_M,
@@ -100,6 +144,27 @@ int launch_wide(bool swapped, int tile, int out_mode, const void* lhs, const voi
   return (int)hipGetLastError();
 }
 
+// The mid-tile kernel's launch, arguments as for the entry points; out_mode GGEMM_OUT_*.
+int launch_mid(bool swapped, int out_mode, const void* lhs, const void* rhs, void* out, const float* lhs_scale,
+               const float* rhs_scale, const int64_t* group_offs, int32_t G, int32_t OUT_M, int32_t OUT_N, int32_t slm,
+               int32_t srm, int32_t scg, int32_t scm, int32_t scn, int64_t M_total, void* stream) {
+  const int64_t tiles = mid_tiles(G, OUT_M, OUT_N), run = ggemm::kXcds * ggemm::mid::kXcdRun;
+  const dim3 grid((uint32_t)((tiles + run - 1) / run * run)), block(ggemm::mid::kNT);
+  if (out_mode == GGEMM_OUT_BF16) {
+    auto kern = swapped ? _grouped_variable_k_gemm_kernel_mid_swapped : _grouped_variable_k_gemm_kernel_mid;
+    hipLaunchKernelGGL(kern, grid, block, 0, (hipStream_t)stream, (const uint8_t*)lhs, (const uint8_t*)rhs,
+                       (uint16_t*)out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N, slm, srm, scg, scm, scn,
+                       (void*)nullptr, (void*)nullptr, M_total);
+  } else {
+    auto kern = out_mode == GGEMM_OUT_F32 ? _grouped_variable_k_gemm_kernel_mid_f32
+                                          : _grouped_variable_k_gemm_kernel_mid_f32_acc;
+    hipLaunchKernelGGL(kern, grid, block, 0, (hipStream_t)stream, (const uint8_t*)lhs, (const uint8_t*)rhs,
+                       (float*)out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N, slm, srm, scg, scm, scn,
+                       (void*)nullptr, (void*)nullptr, M_total);
+  }
+  return (int)hipGetLastError();
+}
+
 }  // namespace
 
 extern "C" {
@@ -116,12 +181,16 @@ static int launch_tensorwise(Mfma mfma, const void* lhs, const void* rhs, void* 
                            scn);
   if (rc) return rc;
   if (m_total < 0) return GGEMM_E_SHAPE;
-  if (const int tile = mfma == Mfma::kK32 ? 0 : wide_selected(OUT_M, OUT_N, scm, scg, out))
-    return launch_wide(mfma == Mfma::kK128Swapped, tile, GGEMM_OUT_BF16, lhs, rhs, out, lhs_scale, rhs_scale,
-                       group_offs, G, OUT_M, OUT_N, slm, srm, scg, scm, scn, m_total, stream);
   int cus = 0;
   rc = device_cus(&cus);
   if (rc) return rc;
+  const int tile = mfma == Mfma::kK32 ? 0 : wide_selected(OUT_M, OUT_N, scm, scg, out);
+  if (mfma != Mfma::kK32 && mid_preferred(G, OUT_M, OUT_N, scm, scg, out, false, m_total, tile, cus))
+    return launch_mid(mfma == Mfma::kK128Swapped, GGEMM_OUT_BF16, lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G,
+                      OUT_M, OUT_N, slm, srm, scg, scm, scn, m_total, stream);
+  if (tile)
+    return launch_wide(mfma == Mfma::kK128Swapped, tile, GGEMM_OUT_BF16, lhs, rhs, out, lhs_scale, rhs_scale,
+                       group_offs, G, OUT_M, OUT_N, slm, srm, scg, scm, scn, m_total, stream);
   auto kern = mfma == Mfma::kK32          ? _grouped_variable_k_gemm_kernel_k32
               : mfma == Mfma::kK128Swapped ? _grouped_variable_k_gemm_kernel_swapped
                                            : _grouped_variable_k_gemm_kernel;
@@ -184,13 +253,17 @@ int ggemm_vark_wgrad_fp8_out(const void* lhs, const void* rhs, void* out, const 
   if (rc) return rc;
   if (M_total < 0) return GGEMM_E_SHAPE;
   if (!aligned(out, 16)) return GGEMM_E_ALIGN;    // 16-byte fp32 row segments
-  // fp32 C takes the 320 x 320 wide-tile kernel where the bf16 C of the same shape would
-  if (wide_selected(OUT_M, OUT_N, 2 * (int64_t)stride_cm, 2 * (int64_t)stride_cg, out) == 320)
-    return launch_wide(false, 320, out_mode, lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N,
-                       stride_lhs_m, stride_rhs_m, stride_cg, stride_cm, stride_cn, M_total, stream);
   int cus = 0;
   rc = device_cus(&cus);
   if (rc) return rc;
+  // fp32 C takes the 320 x 320 wide-tile kernel where the bf16 C of the same shape would
+  const bool wide = wide_selected(OUT_M, OUT_N, 2 * (int64_t)stride_cm, 2 * (int64_t)stride_cg, out) == 320;
+  if (mid_preferred(G, OUT_M, OUT_N, stride_cm, stride_cg, out, true, M_total, wide ? 320 : 0, cus))
+    return launch_mid(false, out_mode, lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N, stride_lhs_m,
+                      stride_rhs_m, stride_cg, stride_cm, stride_cn, M_total, stream);
+  if (wide)
+    return launch_wide(false, 320, out_mode, lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N,
+                       stride_lhs_m, stride_rhs_m, stride_cg, stride_cm, stride_cn, M_total, stream);
   auto kern = out_mode == GGEMM_OUT_F32 ? _grouped_variable_k_gemm_kernel_f32 : _grouped_variable_k_gemm_kernel_f32_acc;
   hipLaunchKernelGGL(kern, dim3(cus), dim3(ggemm::kThreads), ggemm::kDynLdsBytes, (hipStream_t)stream,
                      (const uint8_t*)lhs, (const uint8_t*)rhs, (float*)out, lhs_scale, rhs_scale, group_offs, G, OUT_M,
@@ -307,6 +380,16 @@ int32_t ggemm_vark_abi_version(void) { return GGEMM_VARK_ABI_VERSION; }
 
 int32_t ggemm_vark_bf16_kernel(int32_t OUT_M, int32_t OUT_N, int32_t stride_cm, const void* out) {
   return wide_selected(OUT_M, OUT_N, stride_cm, (int64_t)OUT_M * stride_cm, out);
+}
+
+int32_t ggemm_vark_tile_rows(int32_t G, int32_t OUT_M, int32_t OUT_N, int32_t stride_cm, int32_t out_mode,
+                             int64_t M_total, int32_t num_cus) {
+  const bool f32 = out_mode != GGEMM_OUT_BF16;
+  const int64_t scm = stride_cm, scg = scm * OUT_M, w = f32 ? 2 : 1;
+  int tile = wide_selected(OUT_M, OUT_N, w * scm, w * scg, nullptr);
+  if (f32 && tile != 320) tile = 0;
+  if (mid_preferred(G, OUT_M, OUT_N, scm, scg, nullptr, f32, M_total, tile, num_cus)) return ggemm::mid::kWT;
+  return tile ? tile : ggemm::kTileM;
 }
 
 void ggemm_vark_launch_geometry(int32_t out_n, int32_t* block_threads, int32_t* dynamic_lds, int32_t* tile_m,

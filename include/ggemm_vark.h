@@ -156,8 +156,18 @@ int32_t ggemm_vark_abi_version(void);
  * points also require to be a multiple of 8 for a wide kernel), 0 = the 192-row-tile kernel of the
  * reference launch geometry. The fp32 modes of ggemm_vark_wgrad_fp8_out run the 320 x 320 kernel
  * where this returns 320 for stride_cm twice the fp32 row stride, ggemm_vark_wgrad_mxfp8 its MX
- * variant where this returns 320. No reference counterpart. Touches no device. */
+ * variant where this returns 320. Launches that carry a token count too small for these tiles run
+ * the mid-tile kernel instead (ggemm_vark_tile_rows). No reference counterpart. Touches no device. */
 int32_t ggemm_vark_bf16_kernel(int32_t OUT_M, int32_t OUT_N, int32_t stride_cm, const void* out);
+
+/* Rows of the output tiles of the kernel that ggemm_vark_wgrad_fp8_out (and _swapped, with
+ * GGEMM_OUT_BF16) runs for a launch with a 16-byte aligned C of contiguous groups on a device of
+ * num_cus compute units: 320 or 256 (wide), 192 (reference geometry), or 128, the mid-tile kernel:
+ * one 128 x 128 tile per 256-thread workgroup, several workgroups per CU, for at most 256 groups
+ * whose tokens and output are too few to keep the larger tiles' CUs busy. Its results are the
+ * 192-row kernel's bit for bit. No reference counterpart. Touches no device. */
+int32_t ggemm_vark_tile_rows(int32_t G, int32_t OUT_M, int32_t OUT_N, int32_t stride_cm, int32_t out_mode,
+                             int64_t M_total, int32_t num_cus);
 
 /* Launch geometry the library uses (and the drop-in code object expects) for a problem of width
  * OUT_N = out_n: block threads, dynamic LDS bytes, output tile (OUT_M x OUT_N; the N tile is 384

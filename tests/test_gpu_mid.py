@@ -43,3 +43,54 @@ def test_gemm_equals_512_thread_kernel(pkg, cuda, lens, N, K, rows):
             assert bool((buf[M:] == 7).all()) and bool((buf[:, N:] == 7).all())   # nothing outside is written
             outs.append(buf[:M, :N].contiguous().view(torch.int16))
         assert torch.equal(*outs)
+
+
+# rows of each group, OUT_M, OUT_N: ragged stages, tiles' edges, the ranked and the unranked deal
+WGRAD = [
+    ([5], 16, 16), ([0, 1, 127, 128, 129, 0, 300, 200], 208, 272), ([300, 0, 7], 640, 1152),
+    ([3, 1] * 32, 128, 144), ([2, 0, 1] * 85 + [140], 144, 128),
+]
+
+
+@pytest.mark.parametrize("lens,m,n", WGRAD, ids=[f"{len(r[0])}groups{r[1]}x{r[2]}" for r in WGRAD])
+def test_wgrad_equals_192_row_kernel(pkg, cuda, lens, m, n):
+    """The bf16 result equals the drop-in code object's (the 192-row kernel), the transposed formats'
+    result is the transpose's, and the fp32 modes agree with both, through padded and offset rows."""
+    from ggemm_asm_amd import harness
+    from ggemm_asm_amd.vark import weight_grad_fp8
+    gen = torch.Generator().manual_seed(m + n)
+    G, M = len(lens), sum(lens)
+    offs = torch.tensor([0] + lens, device=cuda).cumsum(0)
+    s = torch.tensor(0.01, device=cuda)
+    run = pkg.grouped_gemm_fp8_tensorwise_variable_k
+    module, func, _ = harness.load_kernel(pkg.CODE_OBJECT_PATH)
+    try:
+        for pad in (0, 48):
+            assert pkg.load_library().ggemm_vark_tile_rows(G, m, n, n + pad, 0, M + 3, 256) == 128
+            assert pkg.load_library().ggemm_vark_tile_rows(G, m, n, n + pad, 1, M + 3, 256) == 128
+            lhs, rhs = (_fp8_bytes((M + 3, w), gen, pad, cuda) for w in (m, n))
+            print(f"[gpu-case] mid wgrad {lens[:8]} {m}x{n} pad={pad}", flush=True)
+            buf = torch.full((G, m, n + pad), 7.0, dtype=torch.bfloat16, device=cuda)
+            run(lhs, rhs, s, s, offs, out=buf[..., :n])
+            torch.cuda.synchronize()
+            assert bool((buf[..., n:] == 7).all())
+            got = buf[..., :n].contiguous()
+            cl, cr = lhs.contiguous(), rhs.contiguous()
+            ref = torch.full_like(got, 7.0)
+            torch.cuda.synchronize()
+            harness.launch_variable_k_kernel(func, cl, cr, ref, s, s, offs, G, m, n, harness.get_num_cus(0))
+            torch.cuda.synchronize()
+            assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+            f32 = run(lhs, rhs, s, s, offs, out_dtype=torch.float32)
+            assert torch.equal(f32.bfloat16().view(torch.int16), got.view(torch.int16))
+            wide = torch.randn((G, m, n + 12), device=cuda)
+            acc = wide.clone()
+            run(lhs, rhs, s, s, offs, out=acc[..., :n], accumulate=True)
+            assert torch.equal(acc[..., :n], wide[..., :n] + f32) and torch.equal(acc[..., n:], wide[..., n:])
+            e4m3, e5m2 = lhs.view(torch.float8_e4m3fn), rhs.view(torch.float8_e5m2)
+            dw = weight_grad_fp8(e5m2, e4m3, s, s, offs)     # [G, n, m]
+            err = (dw.transpose(1, 2).float() - f32).abs()
+            # both round the same fp32 sums (of up to 3 more orders of additions) to bf16
+            assert bool((err <= 2.0 ** -8 * f32.abs() + 1e-5 * float(f32.abs().max())).all())
+    finally:
+        harness.unload_kernel(module)

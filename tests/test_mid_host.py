@@ -15,3 +15,29 @@ def test_gemm_tile_rows(pkg, G, N, K, M, rows):
 def test_gemm_rows_of_c_within_32_bits(pkg):
     assert pkg.persistent.tile_rows(4, 2048, 1424, 1424, 1424, 2 ** 24 - 512 - 8, 100) == 64
     assert pkg.persistent.tile_rows(4, 2048, 1424, 1424, 1424, 2 ** 24, 100) == 192
+
+
+@pytest.mark.parametrize("G,m,n,M,mode,rows", [
+    (32, 2880, 5760, 131072, 0, 320), (4, 2880, 2880, 16384, 2, 320), (12, 1600, 1600, 100000, 0, 320),
+    (1, 16, 16, 0, 0, 128), (4, 64, 128, 512, 0, 128), (4, 2880, 2880, 1024, 0, 128), (8, 512, 1024, 100000, 0, 128),
+    (12, 1600, 1600, 1000, 2, 128), (257, 64, 128, 512, 0, 192),
+    (4, 64, 128, 2 ** 31, 0, 192),                           # no 32-bit token count
+    (256, 65536, 65536, 256, 0, 192),                        # more tiles than one launch
+])
+def test_wgrad_tile_rows(pkg, G, m, n, M, mode, rows):
+    assert pkg.load_library().ggemm_vark_tile_rows(G, m, n, n, mode, M, 256) == rows
+
+
+def test_wgrad_fp32_modes_take_the_same_kernel(pkg):
+    """Accumulating adds what the fp32 mode writes, bit for bit, only if one kernel computes both."""
+    rows = pkg.load_library().ggemm_vark_tile_rows
+    for G in (1, 4, 32):
+        for m, n in ((64, 128), (1600, 1600), (2880, 2880), (2880, 5760), (2048, 528)):
+            for M in (16, 1000, 4096, 16384, 131072):
+                assert rows(G, m, n, n, 1, M, 256) == rows(G, m, n, n, 2, M, 256)
+
+
+def test_wgrad_unaligned_rows_of_c_keep_the_192_row_kernel(pkg):
+    rows = pkg.load_library().ggemm_vark_tile_rows
+    assert rows(4, 64, 128, 136, 0, 512, 256) == 128 and rows(4, 64, 128, 132, 0, 512, 256) == 192
+    assert rows(4, 64, 128, 132, 1, 512, 256) == 128
