@@ -449,18 +449,31 @@ struct Tile {
 //    largest groups' tiles are few and heavy, and the slice holding them ends late; this deal
 //    spreads them over every workgroup.
 // Every workgroup computes each deal's heaviest per-workgroup weight (the same integers in every
-// workgroup) and takes the lighter deal, slices on a tie. Tiles of a group are visited in bands of
+// workgroup) and takes the lighter deal, slices on a tie. In the rounds deal all CUs multiply in the
+// large groups' tiles first and all store C in the small and empty groups' tiles at the end, each
+// phase idling what the other needs. Where those C-bound tiles are a quarter of the work or more
+// (kLight: the stages whose time a tile's C takes at the memory's rate), the odd XCDs walk their
+// tiles from the last one back, so that half of the chip stores while the other half multiplies;
+// each XCD's 32 workgroups stay on neighbouring tiles. Accumulated fp32 C, [32, 2880, 5760]: 846 ->
+// 784 us (16384 tokens, Zipf lengths), 987 -> 862 us (32768), 1022 -> 950 us (32768, exponential
+// lengths); fp32 C 538 -> 483 us (16384, Zipf). With a twentieth instead of a quarter, fp32 C of
+// 131072 tokens was 3 % slower. A bf16 C is stored too fast for it (1 % either way, 276 -> 292 us at
+// 2880 x 2880): not done there (kLight 0).
+// Tiles of a group are visited in bands of
 // kBandN N-tiles, M-tile by M-tile inside a band, down the M-tiles in even bands and back up in
 // odd ones (serpentine), so 32 consecutive tiles (one XCD's round) form a compact block of the
 // group's grid also where a round crosses from one band into the next: the two bands then share
 // M-tiles, whose LHS rows the XCD's L2 fetches once for both (gate_up 320 x 320: 9 % fewer bytes
 // fetched from HBM than the same bands walked one way, 0.3 % less time).
 struct Sched {
-  int t_first, t_end;         // this workgroup's first tile, and the end of its tiles
-  int d0, d1;                 // its next tile is d0 further after an even round, d1 after an odd
+  int t_first, t_end;         // this workgroup's first tile, and the end of all tiles it may take
+  int d0, d1;                 // its next tile is d0 further after an even round, d1 after an odd; both
+                              // negative for a workgroup that walks its tiles from the last one back
   int n_tm, n_tn, tiles_per_group;
   bool sorted;                // groups ranked by size, their offsets held in LDS (s_kb)
   bool valid;                 // false: more tiles than 32-bit indices cover (C would need > 512 GiB)
+  // t is a tile: forward walks end at t_end, backward ones below zero
+  __device__ __forceinline__ bool has(int t) const { return (uint32_t)t < (uint32_t)t_end; }
 };
 
 __device__ __forceinline__ int64_t uniform64(int64_t v) {
@@ -511,8 +524,8 @@ __device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
 // Groups are sorted (and their offsets kept in LDS, so the tile loop reads them there instead of
 // issuing a global load whose wait would drain the prefetched stage) when G <= kMaxSortG and every
 // offset fits 31 bits; otherwise natural order with offsets read from memory.
-// kTM / kNT: tile height (OUT_M) and workgroup threads of the calling kernel.
-template <int kTN, int kK, int kEpiW = 1, int kTM = kTileM, int kNT = kThreads>
+// kTM / kNT: tile height (OUT_M) and workgroup threads of the calling kernel; kLight: above.
+template <int kTN, int kK, int kEpiW = 1, int kTM = kTileM, int kNT = kThreads, int kLight = 0>
 __device__ __forceinline__ Sched make_sched(const VarKArgs& a, GG_LDS int* s_order, GG_LDS int* s_kb,
                                             GG_LDS int* s_flag, GG_LDS int64_t* s_bound) {
   constexpr int kNW = kNT / 64;
@@ -626,9 +639,33 @@ __device__ __forceinline__ Sched make_sched(const VarKArgs& a, GG_LDS int* s_ord
       m1 = s_pred[2 * w + 1] > m1 ? s_pred[2 * w + 1] : m1;
     }
     rounds = m1 < m0;
-    __syncthreads();   // s_w and s_pred alias the first stage's scale region
   }
-  const Deal D = rounds ? rounds_deal(pid) : slice_deal(pid);
+  Deal D = rounds ? rounds_deal(pid) : slice_deal(pid);
+  if (kLight > 0 && rounds && D.t_first < D.t_end) {
+    int64_t work = 0, light = 0;
+    for (int sl = tid & 63; sl < G; sl += 64) {
+      const int w = s_w[sl];
+      work += w;
+      light += max(0, kLight + kEpiW - w);
+    }
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) {
+      work += __shfl_xor(work, m, 64);
+      light += __shfl_xor(light, m, 64);
+    }
+    if (4 * light >= work && (pid & 1)) {
+      // back from this workgroup's last tile: round k holds k num_wg + p, or (k + 1) num_wg - 1 - p if
+      // k is odd
+      const int p = D.t_first, k = ((int)total - 1) / num_wg;
+      const int at_k = (k & 1) ? (k + 1) * num_wg - 1 - p : k * num_wg + p;
+      const int last = at_k < D.t_end ? k : k - 1;
+      D.t_first = (last & 1) ? (last + 1) * num_wg - 1 - p : last * num_wg + p;
+      const int d0 = D.d0, d1 = D.d1;
+      D.d0 = (last & 1) ? -d0 : -d1;
+      D.d1 = (last & 1) ? -d1 : -d0;
+    }
+  }
+  if (choose) __syncthreads();   // s_w and s_pred alias the first stage's scale region
   S.t_first = D.t_first;
   S.t_end = D.t_end;
   S.d0 = D.d0;
@@ -720,7 +757,8 @@ __device__ __forceinline__ void vark_body(const VarKArgs& a, GG_LDS uint8_t* lds
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-  const Sched S = make_sched<kTN, kKStep, kOut == kOutBF16 ? 1 : kOut == kOutF32 ? kEpiWF32 : kEpiWF32Acc>(
+  const Sched S = make_sched<kTN, kKStep, kOut == kOutBF16 ? 1 : kOut == kOutF32 ? kEpiWF32 : kEpiWF32Acc, kTileM,
+                              kThreads, kOut == kOutBF16 ? 0 : kOut == kOutF32 ? 8 : 16>(
       a, s_order, s_kb, s_flag, s_bound);
   if (!S.valid) {
     poison_c<kOut>(a);
@@ -775,10 +813,10 @@ __device__ __forceinline__ void vark_body(const VarKArgs& a, GG_LDS uint8_t* lds
   constexpr int kIssueFirst = (!kMX && kOut == kOutF32Acc) ? kDmaLhs / kWaves : C::DmaPerWave;
   int t = S.t_first, d = S.d0, d_alt = S.d1;   // d: distance to this workgroup's next tile
   Tile T;
-  if (t < S.t_end) T = tile_at_(t);
-  while (t < S.t_end) {
+  if (S.has(t)) T = tile_at_(t);
+  while (S.has(t)) {
     const int t_next = t + d;
-    const bool has_next = t_next < S.t_end;
+    const bool has_next = S.has(t_next);
     Tile N;
     if (has_next) N = tile_at_(t_next);
 
@@ -1164,10 +1202,10 @@ __device__ __forceinline__ void vark_body32(const VarKArgs& a, GG_LDS uint8_t* l
   bool full_prev = false;   // the previous epilogue issued all kEpiStores stores in every wave
   int t = S.t_first, d = S.d0, d_alt = S.d1;   // d: distance to this workgroup's next tile
   Tile T;
-  if (t < S.t_end) T = tile_at<kTN, kKStep>(S, a, s_order, s_kb, t);
-  while (t < S.t_end) {
+  if (S.has(t)) T = tile_at<kTN, kKStep>(S, a, s_order, s_kb, t);
+  while (S.has(t)) {
     const int t_next = t + d;
-    const bool has_next = t_next < S.t_end;
+    const bool has_next = S.has(t_next);
     Tile N;
     if (has_next) N = tile_at<kTN, kKStep>(S, a, s_order, s_kb, t_next);
 

@@ -101,7 +101,7 @@ __device__ __forceinline__ void vark_wide_body(const VarKArgs& a, GG_LDS uint8_t
   GG_LDS uint8_t* misc = lds + (MX ? kMiscOffMX : kMiscOff);
   GG_LDS int* s_order = (GG_LDS int*)misc;
   GG_LDS int* s_kb = (GG_LDS int*)(misc + kKbOffset);
-  const Sched S = make_sched<TN, kKS, kEpiW, TM, kNT>(a, s_order, s_kb, (GG_LDS int*)(misc + kFlagOffset),
+  const Sched S = make_sched<TN, kKS, kEpiW, TM, kNT, OUT == kOutBF16 ? 0 : OUT == kOutF32 ? 16 : 32>(a, s_order, s_kb, (GG_LDS int*)(misc + kFlagOffset),
                                                         (GG_LDS int64_t*)(misc + kBoundOffset));
   if (!S.valid) {
     poison_c<OUT>(a);
@@ -184,11 +184,11 @@ __device__ __forceinline__ void vark_wide_body(const VarKArgs& a, GG_LDS uint8_t
   // pipeline state carried between tiles
   uint32_t c0 = 0, nis = 0, vmt = 0, q0 = 0, q1 = 0, q2 = 0, np = 0;
   int t = S.t_first, d = S.d0, d_alt = S.d1;
-  if (t >= S.t_end) return;
+  if (!S.has(t)) return;
   Tile T = tile_at<TN, kKS, TM>(S, a, s_order, s_kb, t);
   for (;;) {
     const int t_next = t + d;
-    const bool has_next = t_next < S.t_end;
+    const bool has_next = S.has(t_next);
     Tile N{};
     if (has_next) N = tile_at<TN, kKS, TM>(S, a, s_order, s_kb, t_next);
     const uint8_t* blt = lhs + T.kb * (int64_t)stride_l + T.m0;

@@ -94,3 +94,26 @@ def test_wgrad_equals_192_row_kernel(pkg, cuda, lens, m, n):
             assert bool((err <= 2.0 ** -8 * f32.abs() + 1e-5 * float(f32.abs().max())).all())
     finally:
         harness.unload_kernel(module)
+
+
+@pytest.mark.parametrize("m,n", [(1280, 960), (2112, 1904)])
+def test_fp32_backward_walk_of_light_tiles(pkg, cuda, m, n):
+    """Skewed lengths whose many small groups make the odd XCDs walk their tiles backwards, on the
+    wide and the 192-row kernel: the fp32 result rounds to the bf16 one (whose walk is forward) and
+    accumulating adds it exactly; the shape's tiles outnumber the workgroups."""
+    lens = [5000, 3000, 0, 7, 64, 1, 31, 900] * 4
+    gen = torch.Generator().manual_seed(m)
+    offs = torch.tensor([0] + lens, device=cuda).cumsum(0)
+    rows = pkg.load_library().ggemm_vark_tile_rows
+    assert rows(len(lens), m, n, n, 1, sum(lens), 256) == rows(len(lens), m, n, n, 0, sum(lens), 256) != 128
+    lhs, rhs = (_fp8_bytes((sum(lens), w), gen, 0, cuda) for w in (m, n))
+    s = torch.tensor(0.01, device=cuda)
+    run = pkg.grouped_gemm_fp8_tensorwise_variable_k
+    bf16 = run(lhs, rhs, s, s, offs)
+    f32 = run(lhs, rhs, s, s, offs, out=torch.full((len(lens), m, n), float("nan"), device=cuda),
+              out_dtype=torch.float32)
+    assert torch.equal(f32.bfloat16().view(torch.int16), bf16.view(torch.int16))
+    c0 = torch.randn_like(f32)
+    acc = c0.clone()
+    run(lhs, rhs, s, s, offs, out=acc, accumulate=True)
+    assert torch.equal(acc, c0 + f32)
