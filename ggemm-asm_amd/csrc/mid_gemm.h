@@ -154,15 +154,16 @@ __device__ __forceinline__ void gemm_body(const nt::Args& a, GG_LDS uint8_t* lds
 }  // namespace mid
 }  // namespace ggemm
 
-// Library kernel: the 512-thread kernel's 16 arguments plus M_total; 256 threads, static LDS, one
-// tile per workgroup (workgroups past the last tile return at once).
+// Library kernel: the 512-thread kernel's 16 arguments plus M_total and zero_tail; 256 threads, static
+// LDS, one tile per workgroup (workgroups past the last tile have none).
 #define GGEMM_DEFINE_MID_GEMM_KERNEL(NAME, AE5M2, BM)                                                    \
   extern "C" __global__ __launch_bounds__(ggemm::mid::kNT, 2) void NAME(GGEMM_PERSISTENT_PARAMS,          \
-                                                                        int64_t m_total) {               \
+                                                                        int64_t m_total, int zero_tail) { \
     __shared__ __attribute__((aligned(1024))) uint8_t ggemm_mid_lds[ggemm::mid::GemmCfg<BM>::LdsBytes];   \
     ggemm::nt::Args args{a, b, c, a_scale, b_scale, group_offs, G, N, K,                                 \
-                         stride_am, stride_bg, stride_bn, stride_cm, stride_cn, m_total};                \
+                         stride_am, stride_bg, stride_bn, stride_cm, stride_cn, m_total, zero_tail};     \
     (void)global_scratch; (void)profile_scratch;                                                        \
     if (G > 0 && G <= ggemm::mid::kMaxGroups && K > 0 && N > 0)                                          \
       ggemm::mid::gemm_body<AE5M2, BM>(args, (GG_LDS uint8_t*)ggemm_mid_lds);                             \
+    ggemm::nt::clear_tail_rows(args);                                                                   \
   }

@@ -103,22 +103,13 @@ __global__ void __launch_bounds__(kXThreads) transpose_u8_kernel(const uint8_t* 
   }
 }
 
-// Zeroes rows [clamp(offs[G]), m_total) of a bf16 [m_total, N] output (ggemm_persistent_clear_tail):
-// the row range comes from the device copy of the offsets, so no host synchronisation is needed;
-// rows are dealt to workgroups round robin, 16-byte chunks of a row to threads (N is a multiple of
-// 16, rows 16-byte aligned).
+// ggemm_persistent_clear_tail on its own: the rows that a GEMM left as they were.
 constexpr int kTailThreads = 256;
 
 __global__ void __launch_bounds__(kTailThreads) clear_tail_kernel(uint16_t* out, int64_t stride_cm, int N,
                                                                   const int64_t* group_offs, int G,
                                                                   int64_t m_total) {
-  int64_t r0 = group_offs[G];
-  r0 = r0 < 0 ? 0 : (r0 > m_total ? m_total : r0);
-  const int chunks = N / 8;
-  for (int64_t r = r0 + blockIdx.x; r < m_total; r += gridDim.x) {
-    xv4u* row = reinterpret_cast<xv4u*>(out + r * stride_cm);
-    for (int c = threadIdx.x; c < chunks; c += kTailThreads) row[c] = xv4u{0u, 0u, 0u, 0u};
-  }
+  ggemm::nt::clear_tail_rows(out, stride_cm, N, group_offs, G, m_total);
 }
 
 // The wide-tile kernel takes N % 320 == 0 and K % 64 == 0 (persistent_wide.h); its 32-bit buffer
@@ -176,10 +167,12 @@ int launch(const void* a, const void* b, void* out, const float* a_scale, const 
   int rc = validate(a, b, out, a_scale, b_scale, group_offs, G, N, K, sam, sbg, sbn, scm, scn, fmt, M_total);
   if (rc) return rc;
   const bool fits = wide_fits(N, K, sam, sbn, scm);
-  if (kernel == GGEMM_PERSISTENT_KERNEL_WIDE && !fits) return GGEMM_E_SHAPE;
+  const int zero_tail = (kernel & GGEMM_PERSISTENT_ZERO_TAIL) != 0;
+  if (kernel >= 0) kernel &= ~GGEMM_PERSISTENT_ZERO_TAIL;
   const bool automatic = kernel == GGEMM_PERSISTENT_KERNEL_AUTO;
   if (automatic)
     kernel = wide_preferred(N, K, sam, sbn, scm) ? GGEMM_PERSISTENT_KERNEL_WIDE : GGEMM_PERSISTENT_KERNEL_512;
+  if (kernel == GGEMM_PERSISTENT_KERNEL_WIDE && !fits) return GGEMM_E_SHAPE;
   if (kernel < GGEMM_PERSISTENT_KERNEL_AUTO || kernel > GGEMM_PERSISTENT_KERNEL_WIDE) return GGEMM_E_SHAPE;
   int cus = 0;
   rc = device_cus(&cus);
@@ -194,20 +187,20 @@ int launch(const void* a, const void* b, void* out, const float* a_scale, const 
     const int64_t tiles = mid_tiles(mid, G, N, M_total), run = ggemm::kXcds * ggemm::mid::kXcdRun;
     hipLaunchKernelGGL(kern, dim3((uint32_t)((tiles + run - 1) / run * run)), dim3(ggemm::mid::kNT), 0,
                        (hipStream_t)stream, (const uint8_t*)a, (const uint8_t*)b, (uint16_t*)out, a_scale, b_scale,
-                       group_offs, G, N, K, sam, sbg, sbn, scm, scn, (void*)nullptr, (void*)nullptr, M_total);
+                       group_offs, G, N, K, sam, sbg, sbn, scm, scn, (void*)nullptr, (void*)nullptr, M_total, zero_tail);
     return (int)hipGetLastError();
   }
   if (kernel == GGEMM_PERSISTENT_KERNEL_WIDE) {
     auto kern = e5m2 ? _grouped_fp8_persistent_gemm_kernel_wide_e5m2 : _grouped_fp8_persistent_gemm_kernel_wide;
     hipLaunchKernelGGL(kern, dim3(cus), dim3(ggemm::pw::kNT), 0, (hipStream_t)stream, (const uint8_t*)a,
                        (const uint8_t*)b, (uint16_t*)out, a_scale, b_scale, group_offs, G, N, K, sam, sbg, sbn, scm,
-                       scn, (void*)nullptr, (void*)nullptr, M_total);
+                       scn, (void*)nullptr, (void*)nullptr, M_total, zero_tail);
     return (int)hipGetLastError();
   }
   auto kern = e5m2 ? _grouped_fp8_persistent_gemm_kernel_e5m2 : _grouped_fp8_persistent_gemm_kernel;
   hipLaunchKernelGGL(kern, dim3(cus), dim3(ggemm::kThreads), ggemm::kDynLdsBytes, (hipStream_t)stream,
                      (const uint8_t*)a, (const uint8_t*)b, (uint16_t*)out, a_scale, b_scale, group_offs, G, N, K, sam,
-                     sbg, sbn, scm, scn, (void*)nullptr, (void*)nullptr, M_total);
+                     sbg, sbn, scm, scn, (void*)nullptr, (void*)nullptr, M_total, zero_tail);
   return (int)hipGetLastError();
 }
 

@@ -62,7 +62,23 @@ struct Args {
   // the tensors is read or written whatever group_offs holds. kMaxRow from the drop-in code
   // object, whose kernarg carries no row count; the library passes the real one.
   int64_t m_total;
+  int zero_tail;       // rows [offs[G], m_total) of C become zero (clear_tail_rows)
 };
+
+// Zeroes this workgroup's share of rows [clamp(offs[G]), m_total) of C, the rows that no group covers:
+// the range comes from the device copy of the offsets, rows are dealt to the grid's workgroups round
+// robin, 16-byte chunks of a row to threads (N is a multiple of 16, rows 16-byte aligned). Run by the
+// GEMM kernels after their tiles when asked to, which saves the launch that cleared them before.
+__device__ __forceinline__ void clear_tail_rows(uint16_t* out, int64_t stride_cm, int N, const int64_t* group_offs,
+                                                int G, int64_t m_total) {
+  int64_t r0 = group_offs[G];
+  r0 = r0 < 0 ? 0 : (r0 > m_total ? m_total : r0);
+  for (int64_t r = r0 + blockIdx.x; r < m_total; r += gridDim.x)
+    for (int c = threadIdx.x; c < N / 8; c += blockDim.x) *(v4i*)(out + r * stride_cm + 8 * c) = v4i{0, 0, 0, 0};
+}
+__device__ __forceinline__ void clear_tail_rows(const Args& a) {
+  if (a.zero_tail) clear_tail_rows(a.c, a.stride_cm, a.N, a.group_offs, a.G, a.m_total);
+}
 
 struct Tile {
   int g, m0, n0;       // group, first row inside the group, first column
@@ -460,19 +476,20 @@ __device__ __forceinline__ void persistent_entry(const Args& a, GG_LDS uint8_t* 
   extern "C" __global__ __launch_bounds__(ggemm::kThreads) void NAME(GGEMM_PERSISTENT_PARAMS) {          \
     extern __shared__ __attribute__((aligned(1024))) uint8_t ggemm_dyn_lds[];                           \
     ggemm::nt::Args args{a, b, c, a_scale, b_scale, group_offs, G, N, K,                                 \
-                         stride_am, stride_bg, stride_bn, stride_cm, stride_cn, ggemm::nt::kMaxRow};     \
+                         stride_am, stride_bg, stride_bn, stride_cm, stride_cn, ggemm::nt::kMaxRow, 0};  \
     (void)global_scratch; (void)profile_scratch;                                                        \
     ggemm::nt::persistent_entry<AE5M2>(args, (GG_LDS uint8_t*)ggemm_dyn_lds);                             \
   }
 
 // Library kernel: the same 16 arguments plus M_total, the row count of A and C (offsets clamped to
-// [0, M_total] on the device).
+// [0, M_total] on the device), and whether the rows past the last group become zero.
 #define GGEMM_DEFINE_PERSISTENT_LIB_KERNEL(NAME, AE5M2)                                                  \
   extern "C" __global__ __launch_bounds__(ggemm::kThreads) void NAME(GGEMM_PERSISTENT_PARAMS,            \
-                                                                     int64_t m_total) {                  \
+                                                                     int64_t m_total, int zero_tail) {   \
     extern __shared__ __attribute__((aligned(1024))) uint8_t ggemm_dyn_lds[];                           \
     ggemm::nt::Args args{a, b, c, a_scale, b_scale, group_offs, G, N, K,                                 \
-                         stride_am, stride_bg, stride_bn, stride_cm, stride_cn, m_total};                \
+                         stride_am, stride_bg, stride_bn, stride_cm, stride_cn, m_total, zero_tail};     \
     (void)global_scratch; (void)profile_scratch;                                                        \
     ggemm::nt::persistent_entry<AE5M2>(args, (GG_LDS uint8_t*)ggemm_dyn_lds);                             \
+    ggemm::nt::clear_tail_rows(args);                                                                   \
   }

@@ -159,15 +159,16 @@ __device__ __forceinline__ void persistent_wide_body(const nt::Args& a, GG_LDS u
 
 }  // namespace ggemm
 
-// Library kernel: the 512-thread kernel's 16 arguments plus M_total, 256 threads, 160 KiB of static
+// Library kernel: the 512-thread kernel's 16 arguments plus M_total and zero_tail, 256 threads, 160 KiB of static
 // LDS and no dynamic LDS.
 #define GGEMM_DEFINE_PERSISTENT_WIDE_KERNEL(NAME, AE5M2)                                                 \
   extern "C" __global__ __launch_bounds__(ggemm::pw::kNT) __attribute__((amdgpu_waves_per_eu(1, 1)))     \
-  void NAME(GGEMM_PERSISTENT_PARAMS, int64_t m_total) {                                                  \
+  void NAME(GGEMM_PERSISTENT_PARAMS, int64_t m_total, int zero_tail) {                                   \
     __shared__ __attribute__((aligned(1024))) uint8_t ggemm_pw_lds[ggemm::pw::kLdsBytes];                \
     ggemm::nt::Args args{a, b, c, a_scale, b_scale, group_offs, G, N, K,                                 \
-                         stride_am, stride_bg, stride_bn, stride_cm, stride_cn, m_total};                \
+                         stride_am, stride_bg, stride_bn, stride_cm, stride_cn, m_total, zero_tail};     \
     (void)global_scratch; (void)profile_scratch;                                                        \
     if (G > 0 && G <= ggemm::nt::kMaxGroups && ggemm::pw::fits(N, K))                                   \
       ggemm::persistent_wide_body<AE5M2>(args, (GG_LDS uint8_t*)ggemm_pw_lds);                           \
+    ggemm::nt::clear_tail_rows(args);                                                                   \
   }

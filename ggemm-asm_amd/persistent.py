@@ -24,6 +24,7 @@ _FORMAT_NAMES = {"e4m3": GGEMM_FP8_E4M3, "e5m2": GGEMM_FP8_E5M2}
 
 # kernel choices of ggemm_persistent_fp8_kernel (include/ggemm_persistent.h)
 KERNELS = {"auto": 0, "512": 1, "wide": 2}
+ZERO_TAIL = 0x100   # added to a kernel code: rows past the last group become zero in the same launch
 
 
 def selected_kernel(N: int, K: int, stride_am: int, stride_bn: int, stride_cm: int) -> str:
@@ -86,8 +87,8 @@ def grouped_gemm_fp8_tensorwise(a: torch.Tensor, b: torch.Tensor, a_scale: torch
     transpose -- a weight quantized with ``quantize_fp8_tensorwise_transpose`` already has that
     layout); scales: single-element
     fp32 tensors on the device; group_offs: int64 [G+1]. Rows outside ``[0, offs[G])`` of ``out``
-    are left unwritten, or set to zero with ``zero_tail=True`` (the library's device-side clear, no
-    sync: dropped tokens get exact zeros). ``validate=True`` checks group_offs on the host first (a
+    are left unwritten, or set to zero with ``zero_tail=True`` (by the same
+    launch, no sync: dropped tokens get exact zeros). ``validate=True`` checks group_offs on the host first (a
     sync). Offsets past M_total are clamped to it on the device. ``kernel``: "auto" (the library's
     choice: the wide-tile kernel where N % 320 == 0 and K % 64 == 0, else the 512-thread kernel; the
     mid-tile kernel for launches of few rows, ``tile_rows``),
@@ -136,12 +137,8 @@ def grouped_gemm_fp8_tensorwise(a: torch.Tensor, b: torch.Tensor, a_scale: torch
         rc = lib.ggemm_persistent_fp8_kernel(
             a.data_ptr(), b.data_ptr(), out.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(), group_offs.data_ptr(),
             G, N, K, a.stride(0), b.stride(0), b.stride(1), out.stride(0), out.stride(1), fmt, M_total,
-            KERNELS[kernel], _stream(dev))
-        _lib.check(rc, "ggemm_persistent_fp8_kernel")
-        if zero_tail:
-            rc = lib.ggemm_persistent_clear_tail(out.data_ptr(), N, out.stride(0), group_offs.data_ptr(), G, M_total,
-                                                 _stream(dev))
-            _lib.check(rc, "ggemm_persistent_clear_tail")
+            KERNELS[kernel] | (ZERO_TAIL if zero_tail else 0), _stream(dev))
+    _lib.check(rc, "ggemm_persistent_fp8_kernel")
     return out
 
 

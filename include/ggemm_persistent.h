@@ -62,10 +62,13 @@ int ggemm_persistent_fp8(const void* a, const void* b, void* out, const float* a
 #define GGEMM_PERSISTENT_KERNEL_AUTO 0
 #define GGEMM_PERSISTENT_KERNEL_512 1
 #define GGEMM_PERSISTENT_KERNEL_WIDE 2
+/* added to a kernel code: rows [min(offs[G], M_total), M_total) of out become zero in the same launch
+ * (as by ggemm_persistent_clear_tail after it; ABI version 10) */
+#define GGEMM_PERSISTENT_ZERO_TAIL 0x100
 
 /* ggemm_persistent_fp8 with the kernel chosen by the caller: GGEMM_PERSISTENT_KERNEL_AUTO (as
- * ggemm_persistent_fp8), _512 or _WIDE (GGEMM_E_SHAPE where the wide kernel does not apply). No
- * reference counterpart (the reference ships one kernel); for comparisons of the two kernels. */
+ * ggemm_persistent_fp8), _512 or _WIDE (GGEMM_E_SHAPE where the wide kernel does not apply), plus
+ * GGEMM_PERSISTENT_ZERO_TAIL. No reference counterpart (the reference ships one kernel); for comparisons of the two kernels. */
 int ggemm_persistent_fp8_kernel(const void* a, const void* b, void* out, const float* a_scale, const float* b_scale,
                                 const int64_t* group_offs, int32_t G, int32_t N, int32_t K, int32_t stride_am,
                                 int32_t stride_bg, int32_t stride_bn, int32_t stride_cm, int32_t stride_cn,

@@ -117,3 +117,23 @@ def test_fp32_backward_walk_of_light_tiles(pkg, cuda, m, n):
     acc = c0.clone()
     run(lhs, rhs, s, s, offs, out=acc, accumulate=True)
     assert torch.equal(acc, c0 + f32)
+
+
+@pytest.mark.parametrize("lens,N,K,kernel", [([0, 0], 208, 272, "auto"), ([70, 0, 5], 2048, 528, "auto"),
+                                             ([300, 300], 208, 272, "512"), ([300, 1], 640, 128, "wide")])
+def test_zero_tail_in_the_same_launch(pkg, cuda, lens, N, K, kernel):
+    """Rows past the last group become zero, and only those, on every kernel; all rows when no group
+    has one."""
+    gen = torch.Generator().manual_seed(N)
+    M, G, s = sum(lens) + 300, len(lens), torch.tensor(0.01, device=cuda)
+    offs = torch.tensor([0] + lens, device=cuda).cumsum(0)
+    a = _fp8_bytes((M, K), gen, 0, cuda).view(torch.float8_e4m3fn)
+    b = _fp8_bytes((G, N, K), gen, 0, cuda).view(torch.float8_e4m3fn)
+    buf = torch.full((2, M + 64, N + 16), 7.0, dtype=torch.bfloat16, device=cuda)
+    for z in (0, 1):
+        pkg.grouped_gemm_fp8_tensorwise(a, b, s, s, offs, out=buf[z, :M, :N], kernel=kernel, zero_tail=bool(z))
+    torch.cuda.synchronize()
+    rows = sum(lens)
+    assert torch.equal(buf[0, :rows].view(torch.int16), buf[1, :rows].view(torch.int16))
+    assert bool((buf[0, rows:] == 7).all()) and bool((buf[1, rows:M, :N] == 0).all())
+    assert bool((buf[1, M:] == 7).all()) and bool((buf[1, :, N:] == 7).all())
