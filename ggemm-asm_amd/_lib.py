@@ -65,9 +65,11 @@ PERSISTENT_EXPORTS = (
 QUANT_EXPORTS = (
     "ggemm_quant_amax",
     "ggemm_quant_fp8_tensorwise",
+    "ggemm_quant_fp8_tensorwise_ws",
     "ggemm_quant_fp8_tensorwise_delayed",
     "ggemm_quant_fp8_tensorwise_delayed_dev",
     "ggemm_quant_fp8_tensorwise_transpose",
+    "ggemm_quant_fp8_tensorwise_transpose_ws",
     "ggemm_quant_fp8_tensorwise_transpose_delayed",
     "ggemm_quant_fp8_tensorwise_transpose_delayed_dev",
     "ggemm_quant_mxfp8_grouped",
@@ -158,6 +160,8 @@ def load():
     lib.ggemm_quant_amax.restype = ctypes.c_int
     lib.ggemm_quant_fp8_tensorwise.argtypes = [vp, i32, i64, i32, i64, i32, vp, i64, vp, vp, vp]
     lib.ggemm_quant_fp8_tensorwise.restype = ctypes.c_int
+    lib.ggemm_quant_fp8_tensorwise_ws.argtypes = [vp, i32, i64, i32, i64, i32, vp, i64, vp, vp, vp, vp]
+    lib.ggemm_quant_fp8_tensorwise_ws.restype = ctypes.c_int
     lib.ggemm_quant_fp8_tensorwise_delayed.argtypes = [vp, i32, i64, i32, i64, i32, vp, i64, vp, i32, i32, vp, vp]
     lib.ggemm_quant_fp8_tensorwise_delayed.restype = ctypes.c_int
     lib.ggemm_quant_fp8_tensorwise_delayed_dev.argtypes = [vp, i32, i64, i32, i64, i32, vp, i64, vp, i32, vp, vp,
@@ -165,6 +169,9 @@ def load():
     lib.ggemm_quant_fp8_tensorwise_delayed_dev.restype = ctypes.c_int
     lib.ggemm_quant_fp8_tensorwise_transpose.argtypes = [vp, i32, i32, i32, i32, i32, vp, i64, vp, i64, vp, vp, vp]
     lib.ggemm_quant_fp8_tensorwise_transpose.restype = ctypes.c_int
+    lib.ggemm_quant_fp8_tensorwise_transpose_ws.argtypes = [vp, i32, i32, i32, i32, i32, vp, i64, vp, i64, vp, vp, vp,
+                                                            vp]
+    lib.ggemm_quant_fp8_tensorwise_transpose_ws.restype = ctypes.c_int
     lib.ggemm_quant_fp8_tensorwise_transpose_delayed.argtypes = [vp, i32, i32, i32, i32, i32, vp, i64, vp, i64, vp,
                                                                  i32, i32, vp, vp]
     lib.ggemm_quant_fp8_tensorwise_transpose_delayed.restype = ctypes.c_int

@@ -9,7 +9,8 @@
 #include "capi_common.h"
 #include "quant_kernel.h"
 
-static_assert(GGEMM_QUANT_MAX_GROUPS == ggemm::qt::kMaxGroups, "header and kernel agree");
+static_assert(GGEMM_QUANT_MAX_GROUPS == ggemm::qt::kMaxGroups && GGEMM_QUANT_WORKSPACE == ggemm::qt::kMaxPartials,
+              "header and kernel agree");
 
 namespace {
 
@@ -38,16 +39,20 @@ int grid_for(int64_t chunks, int cus, int per_cu) {
   return (int)(want < 1 ? 1 : (want > cap ? cap : want));
 }
 
-void launch_amax(const void* x, int in_dtype, int64_t rows, int cols, int64_t stride, float* amax, int cus,
-                 hipStream_t s) {
-  uint32_t* bits = reinterpret_cast<uint32_t*>(amax);
-  hipLaunchKernelGGL(qt::amax_init, dim3(1), dim3(64), 0, s, bits);
-  if (rows == 0) return;
-  const int grid = grid_for(rows * (cols / 8), cus, kAmaxPerCu);
-  if (in_dtype == GGEMM_IN_F32)
-    hipLaunchKernelGGL(qt::amax_kernel<true>, dim3(grid), dim3(qt::kThreads), 0, s, x, rows, cols, stride, bits);
-  else
-    hipLaunchKernelGGL(qt::amax_kernel<false>, dim3(grid), dim3(qt::kThreads), 0, s, x, rows, cols, stride, bits);
+// The amax of x into *amax, zeroed by a launch of its own; or, with a workspace, the workgroups' partial
+// maxima into it, their number returned (0 for no rows).
+int launch_amax(const void* x, int in_dtype, int64_t rows, int cols, int64_t stride, float* amax,
+                uint32_t* workspace, int cus, hipStream_t s) {
+  uint32_t* bits = workspace ? workspace : reinterpret_cast<uint32_t*>(amax);
+  if (!workspace) hipLaunchKernelGGL(qt::amax_init, dim3(1), dim3(64), 0, s, bits);
+  if (rows == 0) return workspace ? 0 : 1;
+  int grid = grid_for(rows * (cols / 8), cus, kAmaxPerCu);
+  if (grid > qt::kMaxPartials) grid = qt::kMaxPartials;
+  const bool f32 = in_dtype == GGEMM_IN_F32;
+  auto k = f32 ? (workspace ? qt::amax_kernel<true, true> : qt::amax_kernel<true, false>)
+               : (workspace ? qt::amax_kernel<false, true> : qt::amax_kernel<false, false>);
+  hipLaunchKernelGGL(k, dim3(grid), dim3(qt::kThreads), 0, s, x, rows, cols, stride, bits);
+  return workspace ? grid : 1;
 }
 
 // Arguments of the transposing quantizer (all but the amax / history pointers).
@@ -95,32 +100,48 @@ int ggemm_quant_amax(const void* x, int32_t in_dtype, int64_t rows, int32_t cols
   int cus = 0;
   rc = device_cus(&cus);
   if (rc) return rc;
-  launch_amax(x, in_dtype, rows, cols, stride, amax_out, cus, (hipStream_t)stream);
+  launch_amax(x, in_dtype, rows, cols, stride, amax_out, nullptr, cus, (hipStream_t)stream);
+  return (int)hipGetLastError();
+}
+
+static int tensorwise(const void* x, int32_t in_dtype, int64_t rows, int32_t cols, int64_t stride, int32_t out_format,
+                      void* out, int64_t out_stride, float* scale_out, float* amax_out, uint32_t* workspace,
+                      void* stream) {
+  int rc = check_2d(x, in_dtype, rows, cols, stride);
+  if (rc) return rc;
+  if (!out || !scale_out || !amax_out) return GGEMM_E_NULL;
+  if (out_format != GGEMM_FP8_E4M3 && out_format != GGEMM_FP8_E5M2) return GGEMM_E_FORMAT;
+  if (out_stride < cols || out_stride % 8) return GGEMM_E_STRIDE;
+  if (!aligned(out, 8) || !aligned(scale_out, 4) || !aligned(amax_out, 4) || !aligned(workspace, 4))
+    return GGEMM_E_ALIGN;
+  int cus = 0;
+  rc = device_cus(&cus);
+  if (rc) return rc;
+  hipStream_t s = (hipStream_t)stream;
+  const int n = launch_amax(x, in_dtype, rows, cols, stride, amax_out, workspace, cus, s);
+  const int grid = grid_for(rows * (cols / 8), cus, kQuantPerCu);
+  const uint32_t* partials = workspace ? workspace : reinterpret_cast<const uint32_t*>(amax_out);
+  uint8_t* o = static_cast<uint8_t*>(out);
+  const bool f32 = in_dtype == GGEMM_IN_F32, e5 = out_format == GGEMM_FP8_E5M2;
+  auto k = f32 ? (e5 ? qt::quant_tensorwise_kernel<true, true> : qt::quant_tensorwise_kernel<true, false>)
+               : (e5 ? qt::quant_tensorwise_kernel<false, true> : qt::quant_tensorwise_kernel<false, false>);
+  hipLaunchKernelGGL(k, dim3(grid), dim3(qt::kThreads), 0, s, x, rows, cols, stride, o, out_stride, partials, n,
+                     workspace ? amax_out : (float*)nullptr, scale_out);
   return (int)hipGetLastError();
 }
 
 int ggemm_quant_fp8_tensorwise(const void* x, int32_t in_dtype, int64_t rows, int32_t cols, int64_t stride,
                                int32_t out_format, void* out, int64_t out_stride, float* scale_out,
                                float* amax_out, void* stream) {
-  int rc = check_2d(x, in_dtype, rows, cols, stride);
-  if (rc) return rc;
-  if (!out || !scale_out || !amax_out) return GGEMM_E_NULL;
-  if (out_format != GGEMM_FP8_E4M3 && out_format != GGEMM_FP8_E5M2) return GGEMM_E_FORMAT;
-  if (out_stride < cols || out_stride % 8) return GGEMM_E_STRIDE;
-  if (!aligned(out, 8) || !aligned(scale_out, 4) || !aligned(amax_out, 4)) return GGEMM_E_ALIGN;
-  int cus = 0;
-  rc = device_cus(&cus);
-  if (rc) return rc;
-  hipStream_t s = (hipStream_t)stream;
-  launch_amax(x, in_dtype, rows, cols, stride, amax_out, cus, s);
-  const int grid = grid_for(rows * (cols / 8), cus, kQuantPerCu);
-  const uint32_t* bits = reinterpret_cast<const uint32_t*>(amax_out);
-  uint8_t* o = static_cast<uint8_t*>(out);
-  const bool f32 = in_dtype == GGEMM_IN_F32, e5 = out_format == GGEMM_FP8_E5M2;
-  auto k = f32 ? (e5 ? qt::quant_tensorwise_kernel<true, true> : qt::quant_tensorwise_kernel<true, false>)
-               : (e5 ? qt::quant_tensorwise_kernel<false, true> : qt::quant_tensorwise_kernel<false, false>);
-  hipLaunchKernelGGL(k, dim3(grid), dim3(qt::kThreads), 0, s, x, rows, cols, stride, o, out_stride, bits, scale_out);
-  return (int)hipGetLastError();
+  return tensorwise(x, in_dtype, rows, cols, stride, out_format, out, out_stride, scale_out, amax_out, nullptr, stream);
+}
+
+int ggemm_quant_fp8_tensorwise_ws(const void* x, int32_t in_dtype, int64_t rows, int32_t cols, int64_t stride,
+                                  int32_t out_format, void* out, int64_t out_stride, float* scale_out,
+                                  float* amax_out, uint32_t* workspace, void* stream) {
+  if (!workspace) return GGEMM_E_NULL;
+  return tensorwise(x, in_dtype, rows, cols, stride, out_format, out, out_stride, scale_out, amax_out, workspace,
+                    stream);
 }
 
 // The delayed quantizers' history argument: a host slot in [0, H), or (slot_dev != nullptr) a device
@@ -207,26 +228,43 @@ int ggemm_quant_fp8_tensorwise_delayed_dev(const void* x, int32_t in_dtype, int6
                             0, slot, scale_out, stream);
 }
 
-int ggemm_quant_fp8_tensorwise_transpose(const void* x, int32_t in_dtype, int32_t batch, int32_t rows, int32_t cols,
-                                         int32_t out_format, void* out, int64_t out_stride, void* out_t,
-                                         int64_t out_t_stride, float* scale_out, float* amax_out, void* stream) {
+static int tensorwise_transpose(const void* x, int32_t in_dtype, int32_t batch, int32_t rows, int32_t cols,
+                                int32_t out_format, void* out, int64_t out_stride, void* out_t, int64_t out_t_stride,
+                                float* scale_out, float* amax_out, uint32_t* workspace, void* stream) {
   if (!amax_out) return GGEMM_E_NULL;
   int rc = check_transpose(x, in_dtype, batch, rows, cols, out_format, out, out_stride, out_t, out_t_stride, scale_out);
   if (rc) return rc;
-  if (!aligned(amax_out, 4)) return GGEMM_E_ALIGN;
+  if (!aligned(amax_out, 4) || !aligned(workspace, 4)) return GGEMM_E_ALIGN;
   int cus = 0;
   rc = device_cus(&cus);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  launch_amax(x, in_dtype, (int64_t)batch * rows, cols, cols, amax_out, cus, s);
+  const int n = launch_amax(x, in_dtype, (int64_t)batch * rows, cols, cols, amax_out, workspace, cus, s);
+  const uint32_t* partials = workspace ? workspace : reinterpret_cast<const uint32_t*>(amax_out);
   const bool f32 = in_dtype == GGEMM_IN_F32, e5 = out_format == GGEMM_FP8_E5M2;
   auto k = f32 ? (e5 ? qt::quant_transpose_kernel<true, true> : qt::quant_transpose_kernel<true, false>)
                : (e5 ? qt::quant_transpose_kernel<false, true> : qt::quant_transpose_kernel<false, false>);
   const int grid = transpose_grid(reinterpret_cast<const void*>(k), batch, rows, cols, cus);
   hipLaunchKernelGGL(k, dim3(grid), dim3(qt::kThreads), 0, s, x, batch, rows, cols, static_cast<uint8_t*>(out),
-                     out_stride, static_cast<uint8_t*>(out_t), out_t_stride,
-                     reinterpret_cast<const uint32_t*>(amax_out), scale_out);
+                     out_stride, static_cast<uint8_t*>(out_t), out_t_stride, partials, n,
+                     workspace ? amax_out : (float*)nullptr, scale_out);
   return (int)hipGetLastError();
+}
+
+int ggemm_quant_fp8_tensorwise_transpose(const void* x, int32_t in_dtype, int32_t batch, int32_t rows, int32_t cols,
+                                         int32_t out_format, void* out, int64_t out_stride, void* out_t,
+                                         int64_t out_t_stride, float* scale_out, float* amax_out, void* stream) {
+  return tensorwise_transpose(x, in_dtype, batch, rows, cols, out_format, out, out_stride, out_t, out_t_stride,
+                              scale_out, amax_out, nullptr, stream);
+}
+
+int ggemm_quant_fp8_tensorwise_transpose_ws(const void* x, int32_t in_dtype, int32_t batch, int32_t rows,
+                                            int32_t cols, int32_t out_format, void* out, int64_t out_stride,
+                                            void* out_t, int64_t out_t_stride, float* scale_out, float* amax_out,
+                                            uint32_t* workspace, void* stream) {
+  if (!workspace) return GGEMM_E_NULL;
+  return tensorwise_transpose(x, in_dtype, batch, rows, cols, out_format, out, out_stride, out_t, out_t_stride,
+                              scale_out, amax_out, workspace, stream);
 }
 
 int ggemm_quant_fp8_tensorwise_transpose_delayed(const void* x, int32_t in_dtype, int32_t batch, int32_t rows,

@@ -34,6 +34,7 @@ namespace qt {
 constexpr int kThreads = 256;
 constexpr int kUnroll = 4;           // 16-byte chunks each thread has in flight in the streaming kernels
 constexpr int kMaxGroups = 2047;     // MX: group offsets and padded offsets held in LDS
+constexpr int kMaxPartials = 2048;   // workgroups of an amax pass that writes partial maxima
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef unsigned int v2u __attribute__((ext_vector_type(2)));
@@ -161,23 +162,40 @@ __global__ void __launch_bounds__(64) history_advance(float* hist, int H, int32_
   }
 }
 
-// The workgroup's max of its threads' m (|x| as fp32 bits) into *amax_bits, one atomic.
-__device__ __forceinline__ void block_amax(uint32_t m, uint32_t* amax_bits) {
+// The workgroup's max of its threads' m, in every thread.
+__device__ __forceinline__ uint32_t block_max(uint32_t m) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, 64));
   __shared__ uint32_t s_m[kThreads / 64];
   if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6] = m;
   __syncthreads();
-  if (threadIdx.x == 0) {
 #pragma unroll
-    for (int w = 1; w < kThreads / 64; ++w) m = max(m, s_m[w]);
-    if (m) atomicMax(amax_bits, m);
+  for (int w = 0; w < kThreads / 64; ++w) m = max(m, s_m[w]);
+  return __builtin_amdgcn_readfirstlane(m);
+}
+
+// The workgroup's max of its threads' m (|x| as fp32 bits) into *amax_bits, one atomic.
+__device__ __forceinline__ void block_amax(uint32_t m, uint32_t* amax_bits) {
+  m = block_max(m);
+  if (threadIdx.x == 0 && m) atomicMax(amax_bits, m);
+}
+
+// The tensor's amax bits from the n partial maxima of an amax pass (n = 1: the finished amax).
+__device__ __forceinline__ uint32_t partials_amax(const uint32_t* partials, int n) {
+  uint32_t m = 0;
+#pragma unroll
+  for (int k = 0; k < kMaxPartials / kThreads; ++k) {
+    const int i = k * kThreads + (int)threadIdx.x;
+    if (i < n) m = max(m, partials[i]);
   }
+  return block_max(m);
 }
 
 // max of |x| as fp32 bits (ordered like unsigned integers for non-negative values; any NaN is
-// larger than +inf, so NaN propagates), one atomic per workgroup
-template <bool kF32>
+// larger than +inf, so NaN propagates): one atomic per workgroup into *amax_bits, or (kPartials) the
+// workgroup's own maximum in amax_bits[blockIdx.x], which needs no zeroing launch before (4-5 us of a
+// small tensor's 14) and is combined by the pass that uses it (partials_amax)
+template <bool kF32, bool kPartials>
 __global__ void __launch_bounds__(kThreads) amax_kernel(const void* x, int64_t rows, int cols, int64_t stride,
                                                         uint32_t* amax_bits) {
   const int cpr = cols / 8;
@@ -199,7 +217,12 @@ __global__ void __launch_bounds__(kThreads) amax_kernel(const void* x, int64_t r
 #pragma unroll
       for (int k = 0; k < 8; ++k) m = max(m, __float_as_uint(v[u][k]) & 0x7fffffffu);
   }
-  block_amax(m, amax_bits);
+  if constexpr (kPartials) {
+    m = block_max(m);
+    if (threadIdx.x == 0) amax_bits[blockIdx.x] = m;
+  } else {
+    block_amax(m, amax_bits);
+  }
 }
 
 // ---------------------------------------------------------------------------------- tensorwise
@@ -316,10 +339,15 @@ __device__ __forceinline__ uint32_t tensorwise_body(const void* x, int64_t rows,
 template <bool kF32, bool kE5M2>
 __global__ void __launch_bounds__(kThreads) quant_tensorwise_kernel(const void* x, int64_t rows, int cols,
                                                                     int64_t stride, uint8_t* out,
-                                                                    int64_t out_stride, const uint32_t* amax_bits,
+                                                                    int64_t out_stride, const uint32_t* partials,
+                                                                    int n_partials, float* amax_out,
                                                                     float* scale_out) {
-  const ScaleDiv d = scale_div<kE5M2>(*amax_bits);
-  if (blockIdx.x == 0 && threadIdx.x == 0) *scale_out = d.scale;
+  const uint32_t bits = partials_amax(partials, n_partials);
+  const ScaleDiv d = scale_div<kE5M2>(bits);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    *scale_out = d.scale;
+    if (amax_out) *amax_out = __uint_as_float(bits);
+  }
   if (d.fast)
     tensorwise_body<kF32, kE5M2, true>(x, rows, cols, stride, out, out_stride, d);
   else
@@ -429,11 +457,15 @@ __device__ __forceinline__ uint32_t transpose_body(const void* x, int batch, int
 template <bool kF32, bool kE5M2>
 __global__ void __launch_bounds__(kThreads) quant_transpose_kernel(const void* x, int batch, int rows, int cols,
                                                                    uint8_t* out, int64_t out_stride, uint8_t* out_t,
-                                                                   int64_t out_t_stride, const uint32_t* amax_bits,
-                                                                   float* scale_out) {
+                                                                   int64_t out_t_stride, const uint32_t* partials,
+                                                                   int n_partials, float* amax_out, float* scale_out) {
   __shared__ __attribute__((aligned(16))) uint8_t s_t[kTT * kTT];
-  const ScaleDiv d = scale_div<kE5M2>(*amax_bits);
-  if (blockIdx.x == 0 && threadIdx.x == 0) *scale_out = d.scale;
+  const uint32_t bits = partials_amax(partials, n_partials);
+  const ScaleDiv d = scale_div<kE5M2>(bits);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    *scale_out = d.scale;
+    if (amax_out) *amax_out = __uint_as_float(bits);
+  }
   if (d.fast)
     transpose_body<kF32, kE5M2, true>(x, batch, rows, cols, out, out_stride, out_t, out_t_stride, d, s_t);
   else

@@ -19,6 +19,7 @@ GGEMM_IN_F32 = 1
 _IN = {torch.bfloat16: GGEMM_IN_BF16, torch.float32: GGEMM_IN_F32}
 _OUT = {"e4m3": (0, torch.float8_e4m3fn), "e5m2": (1, torch.float8_e5m2)}
 MAX_GROUPS = 2047
+WORKSPACE = 2048   # GGEMM_QUANT_WORKSPACE: 32-bit words an amax pass leaves its partial maxima in
 
 
 def _as_2d(x: torch.Tensor) -> torch.Tensor:
@@ -103,10 +104,11 @@ def quantize_fp8_tensorwise(x: torch.Tensor, fmt: str = "e4m3", row_align: int |
     am = torch.empty((), dtype=torch.float32, device=x.device)
     qp = q2 if q2.shape[0] > 0 else torch.empty((1, x.shape[-1]), dtype=dt, device=x.device)
     with torch.cuda.device(x.device):
-        rc = _lib.load().ggemm_quant_fp8_tensorwise(
+        ws = torch.empty(WORKSPACE, dtype=torch.int32, device=x.device)
+        rc = _lib.load().ggemm_quant_fp8_tensorwise_ws(
             _ptr(x2), _IN[x.dtype], x2.shape[0], x2.shape[1], _row_stride(x2), code, qp.data_ptr(),
-            _row_stride(qp), scale.data_ptr(), am.data_ptr(), _stream(x.device))
-    _lib.check(rc, "ggemm_quant_fp8_tensorwise")
+            _row_stride(qp), scale.data_ptr(), am.data_ptr(), ws.data_ptr(), _stream(x.device))
+    _lib.check(rc, "ggemm_quant_fp8_tensorwise_ws")
     return q, scale, am
 
 
@@ -200,10 +202,11 @@ def _transpose(x, fmt, keep, row_align, amax_history, slot):
     with torch.cuda.device(x.device):
         if amax_history is None:
             am = torch.empty((), dtype=torch.float32, device=x.device)
-            name = "ggemm_quant_fp8_tensorwise_transpose"
-            rc = lib.ggemm_quant_fp8_tensorwise_transpose(
+            ws = torch.empty(WORKSPACE, dtype=torch.int32, device=x.device)
+            name = "ggemm_quant_fp8_tensorwise_transpose_ws"
+            rc = lib.ggemm_quant_fp8_tensorwise_transpose_ws(
                 xp, _IN[x.dtype], B, R, C, code, qp, q_stride, tp, t_stride, scale.data_ptr(), am.data_ptr(),
-                _stream(x.device))
+                ws.data_ptr(), _stream(x.device))
         else:
             am = None
             dev_slot = isinstance(slot, torch.Tensor)

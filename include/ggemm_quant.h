@@ -53,6 +53,15 @@ int ggemm_quant_fp8_tensorwise(const void* x, int32_t in_dtype, int64_t rows, in
 /* Longest amax history of ggemm_quant_fp8_tensorwise_delayed. */
 #define GGEMM_QUANT_MAX_HISTORY 1024
 
+/* ggemm_quant_fp8_tensorwise with a workspace (ABI version 10): GGEMM_QUANT_WORKSPACE 32-bit words of
+ * device memory that the call may overwrite, 4-byte aligned, free again once the call's work on
+ * `stream` is done. Same results; the amax pass leaves its workgroups' maxima there for the
+ * quantizing pass, which spares the launch that zeroes *amax_out. No reference counterpart. */
+#define GGEMM_QUANT_WORKSPACE 2048
+int ggemm_quant_fp8_tensorwise_ws(const void* x, int32_t in_dtype, int64_t rows, int32_t cols, int64_t stride,
+                                  int32_t out_format, void* out, int64_t out_stride, float* scale_out,
+                                  float* amax_out, uint32_t* workspace, void* stream);
+
 /* Per-tensor quantization with delayed scaling: the scale comes from earlier amax values, and this
  * tensor's amax is recorded in the same pass (no separate amax pass over x). amax_history is a
  * device fp32 array of history_len entries; scale_out = m / fmax with m the largest entry other
@@ -93,6 +102,12 @@ int ggemm_quant_fp8_tensorwise_delayed_dev(const void* x, int32_t in_dtype, int6
 int ggemm_quant_fp8_tensorwise_transpose(const void* x, int32_t in_dtype, int32_t batch, int32_t rows, int32_t cols,
                                          int32_t out_format, void* out, int64_t out_stride, void* out_t,
                                          int64_t out_t_stride, float* scale_out, float* amax_out, void* stream);
+
+/* ggemm_quant_fp8_tensorwise_transpose with a workspace, as ggemm_quant_fp8_tensorwise_ws. */
+int ggemm_quant_fp8_tensorwise_transpose_ws(const void* x, int32_t in_dtype, int32_t batch, int32_t rows,
+                                            int32_t cols, int32_t out_format, void* out, int64_t out_stride,
+                                            void* out_t, int64_t out_t_stride, float* scale_out, float* amax_out,
+                                            uint32_t* workspace, void* stream);
 
 /* The transposing pass with delayed scaling: out / out_t as in ggemm_quant_fp8_tensorwise_transpose,
  * the scale and amax_history as in ggemm_quant_fp8_tensorwise_delayed (the max |x| over all
