@@ -12,7 +12,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .vark import _stream, _validate_offsets
+from .vark import _validate_offsets
 
 GGEMM_FP8_E4M3 = 0
 GGEMM_FP8_E5M2 = 1
@@ -68,10 +68,8 @@ def transpose_b(b: torch.Tensor) -> torch.Tensor:
     out = torch.empty((G, N, K), dtype=b.dtype, device=b.device)
     if G == 0 or K == 0 or N == 0:
         return out
-    with torch.cuda.device(b.device):
-        rc = _lib.load().ggemm_persistent_transpose_u8(b.data_ptr(), G, K, N, b.stride(0), b.stride(1), out.data_ptr(),
-                                                       out.stride(0), out.stride(1), _stream(b.device))
-    _lib.check(rc, "ggemm_persistent_transpose_u8")
+    _lib.launch("ggemm_persistent_transpose_u8", b.device, G | K | N, b.data_ptr(), G, K, N, b.stride(0), b.stride(1),
+                out.data_ptr(), out.stride(0), out.stride(1))
     return out
 
 
@@ -132,13 +130,10 @@ def grouped_gemm_fp8_tensorwise(a: torch.Tensor, b: torch.Tensor, a_scale: torch
         raise ValueError(f"kernel must be one of {sorted(KERNELS)}, got {kernel!r}")
     if M_total == 0:
         return out
-    lib = _lib.load()
-    with torch.cuda.device(dev):
-        rc = lib.ggemm_persistent_fp8_kernel(
-            a.data_ptr(), b.data_ptr(), out.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(), group_offs.data_ptr(),
-            G, N, K, a.stride(0), b.stride(0), b.stride(1), out.stride(0), out.stride(1), fmt, M_total,
-            KERNELS[kernel] | (ZERO_TAIL if zero_tail else 0), _stream(dev))
-    _lib.check(rc, "ggemm_persistent_fp8_kernel")
+    sam, (sbg, sbn, _), (scm, scn) = a.stride(0), b.stride(), out.stride()
+    _lib.launch("ggemm_persistent_fp8_kernel", dev, G | N | K | sam | sbg | sbn | scm | scn, a.data_ptr(),
+                b.data_ptr(), out.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(), group_offs.data_ptr(), G, N, K,
+                sam, sbg, sbn, scm, scn, fmt, M_total, KERNELS[kernel] | (ZERO_TAIL if zero_tail else 0))
     return out
 
 

@@ -9,10 +9,11 @@ launch goes through libggemm_vark.so on torch's current stream; there is no CPU 
 """
 from __future__ import annotations
 
+import operator
+
 import torch
 
 from . import _lib
-from .vark import _stream
 
 GGEMM_IN_BF16 = 0
 GGEMM_IN_F32 = 1
@@ -68,10 +69,9 @@ def amax(x: torch.Tensor) -> torch.Tensor:
     _check(x, "e4m3")
     x2 = _as_2d(x)
     out = torch.empty((), dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
-        rc = _lib.load().ggemm_quant_amax(_ptr(x2), _IN[x.dtype], x2.shape[0], x2.shape[1], _row_stride(x2),
-                                          out.data_ptr(), _stream(x.device))
-    _lib.check(rc, "ggemm_quant_amax")
+    rows, cols = x2.shape
+    _lib.launch("ggemm_quant_amax", x.device, cols, _ptr(x2), _IN[x.dtype], rows, cols, _row_stride(x2),
+                out.data_ptr())
     return out
 
 
@@ -97,18 +97,15 @@ def quantize_fp8_tensorwise(x: torch.Tensor, fmt: str = "e4m3", row_align: int |
     _check(x, fmt)
     x2 = _as_2d(x)
     code, dt = _OUT[fmt]
-    q = _padded_empty(x.shape, row_align, dt, x.device)
+    dev, (rows, cols) = x.device, x2.shape
     # q's rows, contiguous or padded, are evenly strided over one buffer
-    q2 = q.as_strided((x2.shape[0], x.shape[-1]), (q.stride(-2), 1))
-    scale = torch.empty((), dtype=torch.float32, device=x.device)
-    am = torch.empty((), dtype=torch.float32, device=x.device)
-    qp = q2 if q2.shape[0] > 0 else torch.empty((1, x.shape[-1]), dtype=dt, device=x.device)
-    with torch.cuda.device(x.device):
-        ws = torch.empty(WORKSPACE, dtype=torch.int32, device=x.device)
-        rc = _lib.load().ggemm_quant_fp8_tensorwise_ws(
-            _ptr(x2), _IN[x.dtype], x2.shape[0], x2.shape[1], _row_stride(x2), code, qp.data_ptr(),
-            _row_stride(qp), scale.data_ptr(), am.data_ptr(), ws.data_ptr(), _stream(x.device))
-    _lib.check(rc, "ggemm_quant_fp8_tensorwise_ws")
+    q = _padded_empty(x.shape, row_align, dt, dev)
+    scale = torch.empty((), dtype=torch.float32, device=dev)
+    am = torch.empty((), dtype=torch.float32, device=dev)
+    ws = torch.empty(WORKSPACE, dtype=torch.int32, device=dev)
+    qp = q if rows > 0 else torch.empty((1, cols), dtype=dt, device=dev)
+    _lib.launch("ggemm_quant_fp8_tensorwise_ws", dev, cols, _ptr(x2), _IN[x.dtype], rows, cols, _row_stride(x2), code,
+                qp.data_ptr(), q.stride(-2) if rows > 1 else cols, scale.data_ptr(), am.data_ptr(), ws.data_ptr())
     return q, scale, am
 
 
@@ -129,17 +126,16 @@ def quantize_fp8_tensorwise_delayed(x: torch.Tensor, amax_history: torch.Tensor,
     dev_slot = isinstance(slot, torch.Tensor)
     x2 = _as_2d(x)
     code, dt = _OUT[fmt]
-    q = _padded_empty(x.shape, row_align, dt, x.device)
-    q2 = q.as_strided((x2.shape[0], x.shape[-1]), (q.stride(-2), 1))
-    scale = torch.empty((), dtype=torch.float32, device=x.device)
-    qp = q2 if q2.shape[0] > 0 else torch.empty((1, x.shape[-1]), dtype=dt, device=x.device)
-    name = "ggemm_quant_fp8_tensorwise_delayed" + ("_dev" if dev_slot else "")
-    with torch.cuda.device(x.device):
-        rc = getattr(_lib.load(), name)(
-            _ptr(x2), _IN[x.dtype], x2.shape[0], x2.shape[1], _row_stride(x2), code, qp.data_ptr(),
-            _row_stride(qp), amax_history.data_ptr(), H, slot.data_ptr() if dev_slot else slot, scale.data_ptr(),
-            _stream(x.device))
-    _lib.check(rc, name)
+    dev, (rows, cols) = x.device, x2.shape
+    q = _padded_empty(x.shape, row_align, dt, dev)
+    scale = torch.empty((), dtype=torch.float32, device=dev)
+    qp = q if rows > 0 else torch.empty((1, cols), dtype=dt, device=dev)
+    if dev_slot:
+        name, at = "ggemm_quant_fp8_tensorwise_delayed_dev", slot.data_ptr()
+    else:
+        name, at = "ggemm_quant_fp8_tensorwise_delayed", operator.index(slot)
+    _lib.launch(name, dev, cols, _ptr(x2), _IN[x.dtype], rows, cols, _row_stride(x2), code, qp.data_ptr(),
+                q.stride(-2) if rows > 1 else cols, amax_history.data_ptr(), H, at, scale.data_ptr())
     return q, scale
 
 
@@ -198,24 +194,19 @@ def _transpose(x, fmt, keep, row_align, amax_history, slot):
         qp = torch.empty((R, q_stride), dtype=dt, device=x.device).data_ptr() if keep else None
     else:
         xp, tp, qp = x.data_ptr(), q_t.data_ptr(), (q.data_ptr() if keep else None)
-    lib = _lib.load()
-    with torch.cuda.device(x.device):
-        if amax_history is None:
-            am = torch.empty((), dtype=torch.float32, device=x.device)
-            ws = torch.empty(WORKSPACE, dtype=torch.int32, device=x.device)
-            name = "ggemm_quant_fp8_tensorwise_transpose_ws"
-            rc = lib.ggemm_quant_fp8_tensorwise_transpose_ws(
-                xp, _IN[x.dtype], B, R, C, code, qp, q_stride, tp, t_stride, scale.data_ptr(), am.data_ptr(),
-                ws.data_ptr(), _stream(x.device))
-        else:
-            am = None
-            dev_slot = isinstance(slot, torch.Tensor)
-            name = "ggemm_quant_fp8_tensorwise_transpose_delayed" + ("_dev" if dev_slot else "")
-            rc = getattr(lib, name)(
-                xp, _IN[x.dtype], B, R, C, code, qp, q_stride, tp, t_stride, amax_history.data_ptr(),
-                amax_history.numel(), slot.data_ptr() if dev_slot else slot, scale.data_ptr(), _stream(x.device))
-    _lib.check(rc, name)
-    return q, q_t, scale, am
+    common = (xp, _IN[x.dtype], B, R, C, code, qp, q_stride, tp, t_stride)
+    if amax_history is None:
+        am = torch.empty((), dtype=torch.float32, device=x.device)
+        ws = torch.empty(WORKSPACE, dtype=torch.int32, device=x.device)
+        _lib.launch("ggemm_quant_fp8_tensorwise_transpose_ws", x.device, B | R | C, *common, scale.data_ptr(),
+                    am.data_ptr(), ws.data_ptr())
+        return q, q_t, scale, am
+    if isinstance(slot, torch.Tensor):
+        name, at = "ggemm_quant_fp8_tensorwise_transpose_delayed_dev", slot.data_ptr()
+    else:
+        name, at = "ggemm_quant_fp8_tensorwise_transpose_delayed", operator.index(slot)
+    _lib.launch(name, x.device, B | R | C, *common, amax_history.data_ptr(), amax_history.numel(), at, scale.data_ptr())
+    return q, q_t, scale, None
 
 
 def padded_rows(rows: int, G: int) -> int:
@@ -246,9 +237,6 @@ def quantize_mxfp8_grouped(x: torch.Tensor, group_offs: torch.Tensor, fmt: str =
     q = torch.empty((rows_out, N), dtype=dt, device=x.device)
     scales = torch.empty((rows_out // 32, N), dtype=torch.uint8, device=x.device)
     padded = torch.empty(G + 1, dtype=torch.int64, device=x.device)
-    with torch.cuda.device(x.device):
-        rc = _lib.load().ggemm_quant_mxfp8_grouped(
-            _ptr(x), _IN[x.dtype], M, N, _row_stride(x), group_offs.data_ptr(), G, code, q.data_ptr(),
-            q.stride(0), rows_out, scales.data_ptr(), scales.stride(0), padded.data_ptr(), _stream(x.device))
-    _lib.check(rc, "ggemm_quant_mxfp8_grouped")
+    _lib.launch("ggemm_quant_mxfp8_grouped", x.device, N | G, _ptr(x), _IN[x.dtype], M, N, _row_stride(x),
+                group_offs.data_ptr(), G, code, q.data_ptr(), N, rows_out, scales.data_ptr(), N, padded.data_ptr())
     return q, scales, padded

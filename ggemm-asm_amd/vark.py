@@ -33,6 +33,8 @@ def _check_inputs(lhs, rhs, group_offs, lhs_dt=_FP8_LHS, rhs_dt=_FP8_RHS):
         raise ValueError("lhs/rhs must be contiguous along the feature dimension")
     for name, t in (("lhs", lhs), ("rhs", rhs)):
         # the kernels may read a token row up to its stride: the last row's padding must exist
+        if t.stride(0) == t.shape[1] and t.is_contiguous():
+            continue
         end = (t.storage_offset() + t.shape[0] * t.stride(0)) * t.element_size()
         if t.shape[0] > 0 and end > t.untyped_storage().nbytes():
             raise ValueError(f"{name}'s last row does not extend to its row stride ({t.stride(0)}) within its "
@@ -74,10 +76,6 @@ def _nonempty(t: torch.Tensor) -> torch.Tensor:
     return torch.zeros((1, t.shape[1]), dtype=t.dtype, device=t.device)
 
 
-def _stream(dev) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
-
-
 def grouped_gemm_fp8_tensorwise_variable_k(lhs: torch.Tensor, rhs: torch.Tensor, lhs_scale: torch.Tensor,
                                            rhs_scale: torch.Tensor, group_offs: torch.Tensor,
                                            out: torch.Tensor | None = None, *, mfma: str = "k128",
@@ -111,26 +109,19 @@ def grouped_gemm_fp8_tensorwise_variable_k(lhs: torch.Tensor, rhs: torch.Tensor,
     if validate:
         _validate_offsets(group_offs, M_total, mx=False)
     lhs, rhs = _nonempty(lhs), _nonempty(rhs)
-    lib = _lib.load()
+    sl, sr, (scg, scm, scn) = lhs.stride(0), rhs.stride(0), out.stride()
+    sizes = G | OUT_M | OUT_N | sl | sr | scg | scm | scn
+    args = (lhs.data_ptr(), rhs.data_ptr(), out.data_ptr(), lhs_scale.data_ptr(), rhs_scale.data_ptr(),
+            group_offs.data_ptr(), G, OUT_M, OUT_N, sl, sr, scg, scm, scn)
+    mode = 2 if accumulate else (1 if out_dtype == torch.float32 else 0)
     if wide:
         if mfma != "k128":
             raise ValueError("the wide-tile kernels use the 32x32x64 MFMA (mfma='k128' family)")
-        mode = 2 if accumulate else (1 if out_dtype == torch.float32 else 0)
-        with torch.cuda.device(lhs.device):
-            rc = lib.ggemm_vark_wgrad_fp8_wide(
-                lhs.data_ptr(), rhs.data_ptr(), out.data_ptr(), lhs_scale.data_ptr(), rhs_scale.data_ptr(),
-                group_offs.data_ptr(), G, OUT_M, OUT_N, lhs.stride(0), rhs.stride(0), out.stride(0), out.stride(1),
-                out.stride(2), M_total, 0 if wide is True else int(wide), mode, _stream(lhs.device))
-        _lib.check(rc, "ggemm_vark_wgrad_fp8_wide")
+        tile = 0 if wide is True else _lib._I32.from_param(int(wide)).value
+        _lib.launch("ggemm_vark_wgrad_fp8_wide", lhs.device, sizes, *args, M_total, tile, mode)
         return out
     if mfma == "k128":
-        mode = 2 if accumulate else (1 if out_dtype == torch.float32 else 0)
-        with torch.cuda.device(lhs.device):
-            rc = lib.ggemm_vark_wgrad_fp8_out(
-                lhs.data_ptr(), rhs.data_ptr(), out.data_ptr(), lhs_scale.data_ptr(), rhs_scale.data_ptr(),
-                group_offs.data_ptr(), G, OUT_M, OUT_N, lhs.stride(0), rhs.stride(0), out.stride(0), out.stride(1),
-                out.stride(2), mode, M_total, _stream(lhs.device))
-        _lib.check(rc, "ggemm_vark_wgrad_fp8_out")
+        _lib.launch("ggemm_vark_wgrad_fp8_out", lhs.device, sizes, *args, mode, M_total)
         return out
     if mfma != "k32":
         raise ValueError("mfma must be 'k128' or 'k32'")
@@ -138,12 +129,7 @@ def grouped_gemm_fp8_tensorwise_variable_k(lhs: torch.Tensor, rhs: torch.Tensor,
         raise ValueError("the fp32 output modes use the K=128 MFMA kernel")
     # the K=32 kernel keeps the reference's argument list (no token count): offsets must end
     # within the tensors, as with the reference kernel
-    with torch.cuda.device(lhs.device):
-        rc = lib.ggemm_vark_wgrad_fp8_k32(
-            lhs.data_ptr(), rhs.data_ptr(), out.data_ptr(), lhs_scale.data_ptr(), rhs_scale.data_ptr(),
-            group_offs.data_ptr(), G, OUT_M, OUT_N, lhs.stride(0), rhs.stride(0), out.stride(0), out.stride(1),
-            out.stride(2), _stream(lhs.device))
-    _lib.check(rc, "ggemm_vark_wgrad_fp8_k32")
+    _lib.launch("ggemm_vark_wgrad_fp8_k32", lhs.device, sizes, *args)
     return out
 
 
@@ -157,12 +143,10 @@ def weight_grad_fp8(dy: torch.Tensor, x: torch.Tensor, dy_scale: torch.Tensor, x
     M_total, N = dy.shape
     out = torch.empty((G, N, x.shape[1]), dtype=torch.bfloat16, device=dy.device)
     dy, x = _nonempty(dy), _nonempty(x)
-    with torch.cuda.device(dy.device):
-        rc = _lib.load().ggemm_vark_wgrad_fp8_swapped(
-            dy.data_ptr(), x.data_ptr(), out.data_ptr(), dy_scale.data_ptr(), x_scale.data_ptr(),
-            group_offs.data_ptr(), G, N, x.shape[1], dy.stride(0), x.stride(0), out.stride(0), out.stride(1), 1,
-            M_total, _stream(dy.device))
-    _lib.check(rc, "ggemm_vark_wgrad_fp8_swapped")
+    K, sl, sr = x.shape[1], dy.stride(0), x.stride(0)
+    _lib.launch("ggemm_vark_wgrad_fp8_swapped", out.device, G | sl | sr | N * K, dy.data_ptr(), x.data_ptr(),
+                out.data_ptr(), dy_scale.data_ptr(), x_scale.data_ptr(), group_offs.data_ptr(), G, N, K, sl, sr,
+                N * K, K, 1, M_total)
     return out
 
 
@@ -192,13 +176,13 @@ def grouped_gemm_mxfp8_variable_k(lhs: torch.Tensor, rhs: torch.Tensor, lhs_scal
         _validate_offsets(group_offs, M_total, mx=True)
     lhs, rhs = _nonempty(lhs), _nonempty(rhs)
     lhs_scale, rhs_scale = _nonempty(lhs_scale), _nonempty(rhs_scale)
-    lib = _lib.load()
-    with torch.cuda.device(lhs.device):
-        rc = lib.ggemm_vark_wgrad_mxfp8_tile(
-            lhs.data_ptr(), rhs.data_ptr(), out.data_ptr(), lhs_scale.data_ptr(), rhs_scale.data_ptr(),
-            group_offs.data_ptr(), G, OUT_M, OUT_N, lhs.stride(0), rhs.stride(0), out.stride(0), out.stride(1),
-            out.stride(2), lhs_scale.stride(0), rhs_scale.stride(0), M_total, int(tile_m), _stream(lhs.device))
-    _lib.check(rc, "ggemm_vark_wgrad_mxfp8_tile")
+    ints = (G, OUT_M, OUT_N, lhs.stride(0), rhs.stride(0), *out.stride(), lhs_scale.stride(0), rhs_scale.stride(0))
+    sizes = 0
+    for v in ints:
+        sizes |= v
+    _lib.launch("ggemm_vark_wgrad_mxfp8_tile", lhs.device, sizes, lhs.data_ptr(), rhs.data_ptr(), out.data_ptr(),
+                lhs_scale.data_ptr(), rhs_scale.data_ptr(), group_offs.data_ptr(), *ints, M_total,
+                _lib._I32.from_param(int(tile_m)).value)
     return out
 
 
