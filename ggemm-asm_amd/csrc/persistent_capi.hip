@@ -133,13 +133,13 @@ int64_t mid_tiles(int rows, int G, int N, int64_t M_total) {
 // The mid-tile kernel's row-tile height (64 or 128) where it is the faster one, else 0: the estimated
 // microseconds of each kernel compared. The lengths of the groups are on the device; M_total rows over
 // G groups are taken to make max(g, M_total / height + g / 2) row tiles, g the groups that can have a
-// row. Per 128-byte K stage and tile: 2.1 us for the persistent kernels with every CU busy (1.7 with
-// few), their tiles one to a CU in whole rounds, 12 us around them; 0.84 / 1.26 us for the mid tiles
-// of 64 / 128 rows with two workgroups on every CU (0.41 / 0.64 with few), 4 us around them, and they
-// feel the memory's time too. Measured (us, the better of 512-thread and wide kernel -> the choice):
-// N = 5760, K = 2880, G = 32: 256 rows 136 -> 95 (64), 2048 rows 129 -> 109 (128), 6144 rows 161, mid
-// 186 (stays); N = K = 2880, G = 4: 512 rows 52 -> 14, 8192 rows 89 -> 70, 16384 rows 137, mid 151
-// (stays); N = 2048, K = 1424, G = 7: 5003 rows 40 -> 32, 20000 rows 86, mid 93 (stays).
+// row. Per 128-byte K stage and tile: 1.85 us (wide) or 1.75 us (512-thread) for the persistent kernels,
+// their tiles one to a CU in whole rounds; 0.69 / 1.06 us for the mid tiles of 64 / 128 rows with two
+// workgroups on every CU (0.41 / 0.64 with few), and they feel the memory's time too; 4 us around
+// either. Measured (us, the better of 512-thread and wide kernel -> the choice): N = 5760, K = 2880, G =
+// 32: 256 rows 149 -> 95 (64), 3072 rows 148 -> 118 (128), 6144 rows 162, mid 182 (stays); N = K = 2880,
+// G = 4: 512 rows 38 -> 14, 8192 rows 83 -> 75, 16384 rows 132, mid 153 (stays); N = 2048, K = 1424, G =
+// 7: 512 rows 25 -> 9, 5003 rows 28, mid 31 (stays); N = 512, K = 1024, G = 8: 100000 rows 92 -> 77.
 int mid_preferred(int G, int N, int K, int scm, int64_t M_total, bool wide, int cus) {
   if (G > ggemm::mid::kMaxGroups || M_total <= 0 || mid_tiles(64, G, N, M_total) > (1 << 22)) return 0;
   if ((int64_t)scm * 2 * 64 >= (int64_t)ggemm::nt::kOob) return 0;   // a wave's rows of C: 32-bit offsets
@@ -149,16 +149,16 @@ int mid_preferred(int G, int N, int K, int scm, int64_t M_total, bool wide, int 
   auto tiles = [&](double h, double w) { return std::max(g, M / h + g / 2) * std::ceil(N / w); };
   double big;
   if (wide) {
-    big = 12 + std::ceil(tiles(256, 320) / cus) * stages * 1.85;
+    big = 4 + std::ceil(tiles(256, 320) / cus) * stages * 1.85;
   } else {
     const int tn = ggemm::wide_tiles(N, false) ? 384 : 320;
-    big = 12 + std::ceil(tiles(192, tn) / cus) * stages * (tn == 384 ? 1.75 : 1.58) + 0.2 * mem;
+    big = 4 + std::ceil(tiles(192, tn) / cus) * stages * (tn == 384 ? 1.75 : 1.58) + 0.2 * mem;
   }
   const double f64 = tiles(64, 128) / (2 * cus), f128 = tiles(128, 128) / (2 * cus);
   const double c64 = 4 + std::max(1.0, f64) * stages * (0.41 + 0.28 * std::min(1.0, f64)) + 0.3 * mem;
   const double c128 = 4 + std::max(1.0, f128) * stages * (0.64 + 0.42 * std::min(1.0, f128)) + 0.3 * mem;
   if (std::min(c64, c128) >= 0.92 * big) return 0;   // near the line the estimate is a few per cent off
-  return c64 <= c128 ? 64 : 128;
+  return c64 < 0.97 * c128 ? 64 : 128;
 }
 
 int launch(const void* a, const void* b, void* out, const float* a_scale, const float* b_scale,

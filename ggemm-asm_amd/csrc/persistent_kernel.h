@@ -63,6 +63,8 @@ struct Args {
   // object, whose kernarg carries no row count; the library passes the real one.
   int64_t m_total;
   int zero_tail;       // rows [offs[G], m_total) of C become zero (clear_tail_rows)
+  int num_wg = 0;      // workgroups of the launch; 0: read from the dispatch packet, 14 us away in
+                       // host memory (VarKArgs)
 };
 
 // Zeroes this workgroup's share of rows [clamp(offs[G]), m_total) of C, the rows that no group covers:
@@ -78,6 +80,12 @@ __device__ __forceinline__ void clear_tail_rows(uint16_t* out, int64_t stride_cm
 }
 __device__ __forceinline__ void clear_tail_rows(const Args& a) {
   if (a.zero_tail) clear_tail_rows(a.c, a.stride_cm, a.N, a.group_offs, a.G, a.m_total);
+}
+
+__device__ __forceinline__ int workgroups(const Args& a) {
+  if (a.num_wg > 0) return a.num_wg;
+  const hsa_kernel_dispatch_packet_t* pkt = dispatch_packet();
+  return (int)((pkt->grid_size_x + pkt->workgroup_size_x - 1) / pkt->workgroup_size_x);
 }
 
 struct Tile {
@@ -244,8 +252,7 @@ __device__ __forceinline__ void persistent_body(const Args& a, GG_LDS uint8_t* l
   // prologue scratch in slot 1: its first stage load is issued after the first stage's barrier
   GG_LDS int64_t* s_scan = (GG_LDS int64_t*)(lds + C2::kSlot);
 
-  const hsa_kernel_dispatch_packet_t* pkt = dispatch_packet();
-  const int num_wg = (int)((pkt->grid_size_x + pkt->workgroup_size_x - 1) / pkt->workgroup_size_x);
+  const int num_wg = workgroups(a);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -445,12 +452,13 @@ __device__ void poison_out(const Args& a) {
 template <bool kAE5M2>
 __device__ __forceinline__ void persistent_entry(const Args& a, GG_LDS uint8_t* dyn) {
   __shared__ __attribute__((aligned(1024))) uint8_t static_lds[kStaticLdsBytes];
-  const hsa_kernel_dispatch_packet_t* pkt = dispatch_packet();
   if (a.G <= 0 || a.G > kMaxGroups || a.K <= 0 || a.N <= 0) return;
   GG_LDS uint8_t* st = (GG_LDS uint8_t*)static_lds;
-  // The launch must provide the contracted dynamic LDS, and the stage slots span both arrays: the
-  // dynamic window must follow the static one directly. Otherwise out becomes NaN (poison_out).
-  if (pkt->group_segment_size < __builtin_amdgcn_groupstaticsize() + (uint32_t)kDynLdsBytes ||
+  // The launch must provide the contracted dynamic LDS (the library's own does), and the stage slots
+  // span both arrays: the dynamic window must follow the static one directly. Otherwise out becomes
+  // NaN (poison_out).
+  if ((a.num_wg == 0 &&
+       dispatch_packet()->group_segment_size < __builtin_amdgcn_groupstaticsize() + (uint32_t)kDynLdsBytes) ||
       lds_u32(dyn) != lds_u32(st) + (uint32_t)kStaticLdsBytes) {
     poison_out(a);
     return;
@@ -488,7 +496,8 @@ __device__ __forceinline__ void persistent_entry(const Args& a, GG_LDS uint8_t* 
                                                                      int64_t m_total, int zero_tail) {   \
     extern __shared__ __attribute__((aligned(1024))) uint8_t ggemm_dyn_lds[];                           \
     ggemm::nt::Args args{a, b, c, a_scale, b_scale, group_offs, G, N, K,                                 \
-                         stride_am, stride_bg, stride_bn, stride_cm, stride_cn, m_total, zero_tail};     \
+                         stride_am, stride_bg, stride_bn, stride_cm, stride_cn, m_total, zero_tail,      \
+                         (int)gridDim.x};                                                               \
     (void)global_scratch; (void)profile_scratch;                                                        \
     ggemm::nt::persistent_entry<AE5M2>(args, (GG_LDS uint8_t*)ggemm_dyn_lds);                             \
     ggemm::nt::clear_tail_rows(args);                                                                   \

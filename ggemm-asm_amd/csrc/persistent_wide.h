@@ -59,8 +59,7 @@ __device__ __forceinline__ void persistent_wide_body(const nt::Args& a, GG_LDS u
   GG_LDS int* s_offs = (GG_LDS int*)(lds + kOffsOff);
   GG_LDS int64_t* s_scan = (GG_LDS int64_t*)(lds + kSlot);   // slot 1: no stage is issued before the scan ends
 
-  const hsa_kernel_dispatch_packet_t* pkt = dispatch_packet();
-  const int num_wg = (int)((pkt->grid_size_x + pkt->workgroup_size_x - 1) / pkt->workgroup_size_x);
+  const int num_wg = nt::workgroups(a);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -166,7 +165,8 @@ __device__ __forceinline__ void persistent_wide_body(const nt::Args& a, GG_LDS u
   void NAME(GGEMM_PERSISTENT_PARAMS, int64_t m_total, int zero_tail) {                                   \
     __shared__ __attribute__((aligned(1024))) uint8_t ggemm_pw_lds[ggemm::pw::kLdsBytes];                \
     ggemm::nt::Args args{a, b, c, a_scale, b_scale, group_offs, G, N, K,                                 \
-                         stride_am, stride_bg, stride_bn, stride_cm, stride_cn, m_total, zero_tail};     \
+                         stride_am, stride_bg, stride_bn, stride_cm, stride_cn, m_total, zero_tail,      \
+                         (int)gridDim.x};                                                               \
     (void)global_scratch; (void)profile_scratch;                                                        \
     if (G > 0 && G <= ggemm::nt::kMaxGroups && ggemm::pw::fits(N, K))                                   \
       ggemm::persistent_wide_body<AE5M2>(args, (GG_LDS uint8_t*)ggemm_pw_lds);                           \

@@ -552,8 +552,8 @@ __global__ void __launch_bounds__(kThreads) quant_mx_grouped_kernel(MxArgs a) {
     }
     // offsets outside [0, rows] or decreasing: nothing is read or written (the host checks the
     // output capacity against rows + 31 G, which holds only for valid offsets). Sums over the waves'
-    // lanes by shuffles and over the waves in LDS, one barrier: a serial check of all threads' flags
-    // and a barrier-per-step scan took 11 us of every workgroup, of 61 us for 32768 x 2880 bf16.
+    // lanes by shuffles and over the waves in LDS, one barrier: with a serial check of all threads'
+    // flags and a barrier-per-step scan two small quantizations took 4 us longer.
     int incl = sum;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {

@@ -88,14 +88,15 @@ int64_t mid_tiles(int G, int OUT_M, int OUT_N) {
 
 // Whether the mid-tile kernel is the faster one: the estimated microseconds of both sides compared,
 // M_total / G tokens in every group. Per 128-token stage and tile: 2.06 us for a wide tile and 1.2
-// (few CUs busy) to 2.1 us for a 192-row one, tiles one to a CU in whole rounds, 12 us around them;
-// 0.55 (few) to 1.27 us (two workgroups on every CU) for a mid tile, 4 us around them; a tile's ends
-// cost 3 stages more (an fp32 C: 4; wide 7 us, 13). wide_tile: the wide kernel the entry would run, 0 the
-// 192-row kernel. Measured (us, large -> mid): 64 x 128, 512 tokens, G = 4: 21 -> 5.3; 2880 x 2880, G = 4:
-// 1024 tokens 37 -> 31, 4096 tokens 56, mid 60 (stays), accumulated fp32 92 -> 77; 512 x 1024, G = 8:
-// 1000 tokens 25 -> 6.5, 100000 tokens 148 -> 69; 1600 x 1600, G = 12, 1000 tokens: 33 -> 24, accumulated
-// 73 -> 42, 100000 tokens 292, mid 352 (stays). The fp32 modes take one line for both, so that
-// accumulating adds exactly what the fp32 mode writes. No token count (INT64_MAX): the large kernels.
+// (few CUs busy) to 2.1 us for a 192-row one, tiles one to a CU in whole rounds; 0.55 (few) to 1.27 us
+// (two workgroups on every CU) for a mid tile; a tile's ends cost 3 stages more (an fp32 C: 4; wide 7
+// us, fp32 16, between the 9 of writing and the 30 of accumulating); 4 to 7 us around all. wide_tile: the
+// wide kernel the entry would run, 0 the 192-row kernel. Measured (us, large -> mid): 64 x 128, 512
+// tokens, G = 4: 14 -> 5.3; 512 x 1024, G = 8: 1000 tokens 15 -> 6.3, 100000 tokens 137 -> 69; 1024 x 2048,
+// G = 2, 8000 tokens 51 -> 25; 2880 x 2880, G = 4: 4096 tokens 54, mid 63 (stays), accumulated fp32 1024
+// tokens 77 -> 52; 1600 x 1600, G = 12: 1000 tokens 24, mid 24 (stays), accumulated 63 -> 42, 100000
+// tokens 294, mid 354 (stays). The fp32 modes take one line for both, so that accumulating adds exactly
+// what the fp32 mode writes. No token count (INT64_MAX): the large kernels.
 bool mid_preferred(int G, int OUT_M, int OUT_N, int64_t scm, int64_t scg, const void* out, bool f32, int64_t M_total,
                    int wide_tile, int cus) {
   const int64_t w = f32 ? 2 : 1;                             // strides in bf16 elements
@@ -109,10 +110,10 @@ bool mid_preferred(int G, int OUT_M, int OUT_N, int64_t scm, int64_t scg, const 
   double big;
   if (wide_tile) {
     const double t = wide_tile == 320 ? tiles(320, 320) : tiles(256, 384);
-    big = 12 + std::ceil(t / cus) * (stages * 2.06 + (f32 ? 13 : 7));
+    big = 5 + std::ceil(t / cus) * (stages * 2.06 + (f32 ? 16 : 7));
   } else {
     const double t = tiles(ggemm::kTileM, ggemm::wide_tiles(OUT_N, false) ? 384 : 320) / cus;
-    big = 12 + std::ceil(t) * (stages + 3) * (1.2 + 0.9 * std::min(1.0, t));
+    big = 7 + std::ceil(t) * (stages + 3) * (1.2 + 0.9 * std::min(1.0, t));
   }
   return mid < 0.92 * big;                                   // near the line the estimate is a few per cent off
 }

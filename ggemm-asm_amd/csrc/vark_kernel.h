@@ -421,6 +421,11 @@ struct VarKArgs {
   // leaves the tensors whatever group_offs holds. INT64_MAX from the drop-in code object, whose
   // kernarg carries no token count (reference launcher.cpp:16-33); the library passes the real one.
   int64_t m_total;
+  // Workgroups of the launch, which the library's kernels take from their kernel arguments; 0: from
+  // the dispatch packet, the only place where the drop-in code object's callers leave it. The packet
+  // lies in host memory: 256 workgroups took 14 us to read it, more than all the rest of a schedule
+  // (make_sched for 32 groups: 27 us with it and a serial pass over the groups, 9 us now).
+  int num_wg = 0;
 };
 
 __device__ __forceinline__ int64_t clamp_off(int64_t o, int64_t m_total) {
@@ -529,11 +534,18 @@ template <int kTN, int kK, int kEpiW = 1, int kTM = kTileM, int kNT = kThreads, 
 __device__ __forceinline__ Sched make_sched(const VarKArgs& a, GG_LDS int* s_order, GG_LDS int* s_kb,
                                             GG_LDS int* s_flag, GG_LDS int64_t* s_bound) {
   constexpr int kNW = kNT / 64;
+  constexpr int kPer = kMaxSortG / kNT;       // groups (or their sorted slots) per thread
+  static_assert(kPer * kNT == kMaxSortG, "groups split evenly over the threads");
   Sched S;
-  const hsa_kernel_dispatch_packet_t* pkt = dispatch_packet();
-  const int num_wg = (int)((pkt->grid_size_x + pkt->workgroup_size_x - 1) / pkt->workgroup_size_x);
-  const int tid = threadIdx.x;
+  int num_wg = a.num_wg;
+  if (num_wg == 0) {
+    const hsa_kernel_dispatch_packet_t* pkt = dispatch_packet();
+    num_wg = (int)((pkt->grid_size_x + pkt->workgroup_size_x - 1) / pkt->workgroup_size_x);
+  }
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int G = a.G;
+  GG_LDS int* s_w = (GG_LDS int*)((GG_LDS uint8_t*)s_order + kScaleOffset);
+  GG_LDS uint64_t* s_pred = (GG_LDS uint64_t*)((GG_LDS uint8_t*)s_order + kPredOffset);
 
   S.sorted = G <= kMaxSortG;
   if (S.sorted) {
@@ -548,16 +560,33 @@ __device__ __forceinline__ Sched make_sched(const VarKArgs& a, GG_LDS int* s_ord
     S.sorted = *s_flag == 0;
   }
   if (S.sorted) {
-    for (int g = tid; g < G; g += kNT) {
-      const int my = group_size(s_kb, g);
-      int rank = 0;
-      for (int h = 0; h < G; ++h) {
-        const int o = group_size(s_kb, h);
-        rank += (o > my) || (o == my && h < g);
+    // ranks by descending size: the sizes in s_w, read four at a time, padded with -1
+    for (int g = tid; g < (G + 3) / 4 * 4; g += kNT) s_w[g] = g < G ? group_size(s_kb, g) : -1;
+    __syncthreads();
+    int rank[kPer], size[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int g = tid + k * kNT;
+      rank[k] = 0;
+      size[k] = 0;
+      if (k * kNT < G) {
+        const int my = size[k] = g < G ? s_w[g] : 0;
+        for (int h = 0; h < G; h += 4) {
+          const v4i o = *(const GG_LDS v4i*)(s_w + h);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) rank[k] += (o[e] > my) || (o[e] == my && h + e < g);
+        }
       }
-      s_order[rank] = g;
     }
     __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int g = tid + k * kNT;
+      if (g < G) {
+        s_order[rank[k]] = g;
+        s_w[rank[k]] = (size[k] + kK - 1) / kK + kEpiW;
+      }
+    }
   }
 
   S.n_tm = (a.OUT_M + kTM - 1) / kTM;
@@ -569,51 +598,70 @@ __device__ __forceinline__ Sched make_sched(const VarKArgs& a, GG_LDS int* s_ord
   if (!S.valid) return S;
 
   const int pid = blockIdx.x;
-  // XCDs per slice and slices: pairs when the grid spreads evenly over the 8 XCDs
+  // slices: XCD pairs when the grid spreads evenly over the 8 XCDs, else one for the whole grid
   const bool spread = num_wg % kXcds == 0;
-  const int xcds = spread ? kXcds : 1;
-  const int n_xcd = spread ? kXcdPairs : 1;   // slices
-  const int per_slice = xcds / n_xcd;
-  const int wgs_per_xcd = num_wg / xcds;
+  const int wgs_per_xcd = spread ? num_wg / kXcds : num_wg;
   const int tpg = S.tiles_per_group;
-  if (tid == 0) {
-    if (S.sorted && n_xcd > 1) {
-      int64_t total_w = 0;
-      for (int sl = 0; sl < G; ++sl)
-        total_w += (int64_t)tpg * (((int64_t)group_size(s_kb, s_order[sl]) + kK - 1) / kK + kEpiW);
-      int64_t acc_w = 0;
-      int x = 1;
-      s_bound[0] = 0;
-      for (int sl = 0; sl < G && x < n_xcd; ++sl) {
-        const int64_t w = ((int64_t)group_size(s_kb, s_order[sl]) + kK - 1) / kK + kEpiW;
-        const int64_t slot_w = w * tpg;
-        while (x < n_xcd && acc_w + slot_w >= (total_w * x) / n_xcd) {
-          const int64_t need = (total_w * x) / n_xcd - acc_w;
-          const int64_t i = (need + w - 1) / w;
-          s_bound[x++] = (int64_t)sl * tpg + (i < tpg ? i : tpg);
-        }
-        acc_w += slot_w;
-      }
-      for (; x <= n_xcd; ++x) s_bound[x] = total;
-    } else {
-      for (int x = 0; x <= n_xcd; ++x) s_bound[x] = total * x / n_xcd;
+  const bool choose = S.sorted && spread;
+  if (choose) {
+    // bounds of the slices: slice x starts at the first tile whose preceding work reaches x / 4 of
+    // all; the slots' work summed over the threads (kPer slots each), waves and workgroup
+    __syncthreads();
+    int64_t w[kPer], sum = 0;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int sl = tid * kPer + k;
+      w[k] = sl < G ? s_w[sl] : 0;
+      sum += w[k];
     }
+    int64_t incl = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int64_t v = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += v;
+    }
+    if (lane == 63) s_pred[wave] = (uint64_t)incl;
+    if (tid == 0) s_bound[0] = 0;
+    __syncthreads();
+    int64_t before = incl - sum, total_w = 0;
+#pragma unroll
+    for (int v = 0; v < kNW; ++v) {
+      const int64_t p = (int64_t)s_pred[v];
+      before += v < wave ? p : 0;
+      total_w += p;
+    }
+    total_w *= tpg;
+    before *= tpg;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int64_t after = before + w[k] * tpg;
+      for (int x = 1; x < kXcdPairs; ++x) {
+        const int64_t target = total_w * x / kXcdPairs;
+        if (before < target && target <= after) {
+          const int64_t need = target - before;               // ceil(need / w) tiles of this slot before it
+          int64_t i = (int64_t)((double)need / (double)w[k]);
+          while (i * w[k] < need) ++i;
+          while (i > 0 && (i - 1) * w[k] >= need) --i;
+          s_bound[x] = (int64_t)(tid * kPer + k) * tpg + (i < tpg ? i : tpg);
+        }
+      }
+      before = after;
+    }
+    if (tid == 0) s_bound[kXcdPairs] = total;
+  } else if (tid == 0) {
+    for (int x = 0; x <= kXcdPairs; ++x) s_bound[x] = spread ? total * x / kXcdPairs : (x ? total : 0);
   }
-  GG_LDS int* s_w = (GG_LDS int*)((GG_LDS uint8_t*)s_order + kScaleOffset);
-  GG_LDS uint64_t* s_pred = (GG_LDS uint64_t*)((GG_LDS uint8_t*)s_order + kPredOffset);
-  const bool choose = S.sorted && n_xcd > 1;
-  if (choose)
-    for (int sl = tid; sl < G; sl += kNT) s_w[sl] = (group_size(s_kb, s_order[sl]) + kK - 1) / kK + kEpiW;
   __syncthreads();
   // workgroup w's tiles under each deal; in the rounds deal, XCD x holds positions [32x, 32x + 32)
   // of a round, and a round's position p is followed by the next round's num_wg - 1 - p
   auto slice_deal = [&](int w) {
-    const int xcd = w % xcds, slice = xcd % n_xcd, part = xcd / n_xcd;
-    const int step = per_slice * wgs_per_xcd;
-    return Deal{(int)s_bound[slice] + part * wgs_per_xcd + w / xcds, (int)s_bound[slice + 1], step, step};
+    const int xcd = spread ? w % kXcds : 0, at = spread ? w / kXcds : w;
+    const int slice = xcd % kXcdPairs, part = xcd / kXcdPairs;
+    const int step = spread ? (kXcds / kXcdPairs) * wgs_per_xcd : num_wg;
+    return Deal{(int)s_bound[slice] + part * wgs_per_xcd + at, (int)s_bound[slice + 1], step, step};
   };
   auto rounds_deal = [&](int w) {
-    const int p = (w % xcds) * wgs_per_xcd + w / xcds;
+    const int p = (w % kXcds) * wgs_per_xcd + w / kXcds;
     return Deal{p, (int)total, 2 * (num_wg - p) - 1, 2 * p + 1};
   };
   bool rounds = false;
@@ -624,10 +672,9 @@ __device__ __forceinline__ Sched make_sched(const VarKArgs& a, GG_LDS int* s_ord
       const uint64_t v = deal_weight(s_w, tpg, d ? rounds_deal(q) : slice_deal(q));
       mx[d] = v > mx[d] ? v : mx[d];
     }
-    const int wave = tid >> 6;
     mx[0] = wave_max_u64(mx[0]);
     mx[1] = wave_max_u64(mx[1]);
-    if ((tid & 63) == 0) {
+    if (lane == 0) {
       s_pred[2 * wave] = mx[0];
       s_pred[2 * wave + 1] = mx[1];
     }
@@ -1326,12 +1373,13 @@ __device__ __forceinline__ void vark_body32(const VarKArgs& a, GG_LDS uint8_t* l
 template <bool kMX, bool kLegacyK32, int kOut = kOutBF16, bool kSwapped = false>
 __device__ __forceinline__ void vark_entry(const VarKArgs& a, GG_LDS uint8_t* dyn) {
   __shared__ __attribute__((aligned(1024))) uint8_t static_lds[kStaticLdsBytes];
-  const hsa_kernel_dispatch_packet_t* pkt = dispatch_packet();
   if (a.G <= 0) return;
   GG_LDS uint8_t* st = (GG_LDS uint8_t*)static_lds;
-  // The launch must provide the contracted dynamic LDS, and the stage slots span both arrays: the
-  // dynamic window must follow the static one directly. Otherwise C becomes NaN (poison_c).
-  if (pkt->group_segment_size < __builtin_amdgcn_groupstaticsize() + (uint32_t)kDynLdsBytes ||
+  // The launch must provide the contracted dynamic LDS (the library's own does, and spares the read of
+  // the packet), and the stage slots span both arrays: the dynamic window must follow the static one
+  // directly. Otherwise C becomes NaN (poison_c).
+  if ((a.num_wg == 0 &&
+       dispatch_packet()->group_segment_size < __builtin_amdgcn_groupstaticsize() + (uint32_t)kDynLdsBytes) ||
       lds_u32(dyn) != lds_u32(st) + (uint32_t)kStaticLdsBytes) {
     poison_c<kOut>(a);
     return;
@@ -1374,7 +1422,8 @@ __device__ __forceinline__ void vark_entry(const VarKArgs& a, GG_LDS uint8_t* dy
                                                                      int64_t m_total) {                  \
     extern __shared__ __attribute__((aligned(1024))) uint8_t ggemm_dyn_lds[];                           \
     ggemm::VarKArgs a{lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N,                  \
-                      stride_lhs_m, stride_rhs_m, stride_cg, stride_cm, stride_cn, 0, 0, m_total};       \
+                      stride_lhs_m, stride_rhs_m, stride_cg, stride_cm, stride_cn, 0, 0, m_total,        \
+                      (int)gridDim.x};                                                                  \
     (void)global_scratch; (void)profile_scratch;                                                        \
     ggemm::vark_entry<false, LEGACY, OUT, SWAPPED>(a, (GG_LDS uint8_t*)ggemm_dyn_lds);                   \
   }
@@ -1389,7 +1438,7 @@ __device__ __forceinline__ void vark_entry(const VarKArgs& a, GG_LDS uint8_t* dy
     extern __shared__ __attribute__((aligned(1024))) uint8_t ggemm_dyn_lds[];                           \
     ggemm::VarKArgs a{lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N,                  \
                       stride_lhs_m, stride_rhs_m, stride_cg, stride_cm, stride_cn,                      \
-                      stride_lhs_scale, stride_rhs_scale, m_total};                                     \
+                      stride_lhs_scale, stride_rhs_scale, m_total, (int)gridDim.x};                     \
     (void)global_scratch; (void)profile_scratch;                                                        \
     ggemm::vark_entry<true, false>(a, (GG_LDS uint8_t*)ggemm_dyn_lds);                                    \
   }

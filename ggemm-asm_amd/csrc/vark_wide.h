@@ -275,7 +275,8 @@ __device__ __forceinline__ void vark_wide_body(const VarKArgs& a, GG_LDS uint8_t
   void NAME(GGEMM_VARK_TW_PARAMS(CT), int64_t m_total) {                                                \
     __shared__ __attribute__((aligned(1024))) uint8_t ggemm_wide_lds[ggemm::wide::kLdsBytes];            \
     ggemm::VarKArgs a{lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N,                  \
-                      stride_lhs_m, stride_rhs_m, stride_cg, stride_cm, stride_cn, 0, 0, m_total};       \
+                      stride_lhs_m, stride_rhs_m, stride_cg, stride_cm, stride_cn, 0, 0, m_total,        \
+                      (int)gridDim.x};                                                                  \
     (void)global_scratch; (void)profile_scratch;                                                        \
     if (G > 0) ggemm::vark_wide_body<TM, TN, OUT, false, SWAPPED>(a, (GG_LDS uint8_t*)ggemm_wide_lds);   \
   }
@@ -291,6 +292,6 @@ __device__ __forceinline__ void vark_wide_body(const VarKArgs& a, GG_LDS uint8_t
     __shared__ __attribute__((aligned(1024))) uint8_t ggemm_wide_lds[ggemm::wide::kLdsBytesMX];          \
     ggemm::VarKArgs a{lhs, rhs, out, lhs_scale, rhs_scale, group_offs, G, OUT_M, OUT_N,                  \
                       stride_lhs_m, stride_rhs_m, stride_cg, stride_cm, stride_cn,                      \
-                      stride_lhs_scale, stride_rhs_scale, m_total};                                     \
+                      stride_lhs_scale, stride_rhs_scale, m_total, (int)gridDim.x};                     \
     if (G > 0) ggemm::vark_wide_body<320, 320, ggemm::kOutBF16, true>(a, (GG_LDS uint8_t*)ggemm_wide_lds); \
   }

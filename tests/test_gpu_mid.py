@@ -19,7 +19,7 @@ GEMM = [  # rows of each group, N, K, tile rows
     ([0, 1, 63, 64, 65, 0, 129, 200], 208, 272, 64),
     ([3] * 256, 144, 128, 64),                       # the most groups it takes
     ([300, 0, 5, 4000], 640, 2880, 64),
-    ([700, 715, 0, 1200, 127, 128, 2133], 2048, 1424, 128),
+    ([400, 415, 0, 900, 127, 128, 1030], 2048, 1424, 128),
 ]
 
 

@@ -4,7 +4,7 @@ import pytest
 
 @pytest.mark.parametrize("G,N,K,M,rows", [
     (32, 5760, 2880, 131072, 256), (4, 2880, 2880, 16384, 256), (7, 2048, 1424, 20000, 192),   # rows enough
-    (32, 5760, 2880, 256, 64), (32, 5760, 2880, 3072, 128), (7, 2048, 1424, 5003, 128), (1, 16, 16, 1, 64),
+    (32, 5760, 2880, 256, 64), (32, 5760, 2880, 3072, 128), (7, 2048, 1424, 5003, 192), (7, 2048, 1424, 3000, 128), (1, 16, 16, 1, 64),
     (257, 2048, 1424, 300, 192),                             # more groups than it holds
     (1, 16, 16, 0, 192), (1, 16, 16, 2 ** 31 - 257, 192),    # no rows; more tiles than one launch
 ])
@@ -19,7 +19,7 @@ def test_gemm_rows_of_c_within_32_bits(pkg):
 
 @pytest.mark.parametrize("G,m,n,M,mode,rows", [
     (32, 2880, 5760, 131072, 0, 320), (4, 2880, 2880, 16384, 2, 320), (12, 1600, 1600, 100000, 0, 320),
-    (1, 16, 16, 0, 0, 128), (4, 64, 128, 512, 0, 128), (4, 2880, 2880, 1024, 0, 128), (8, 512, 1024, 100000, 0, 128),
+    (1, 16, 16, 0, 0, 128), (4, 64, 128, 512, 0, 128), (4, 2880, 2880, 1024, 0, 320), (4, 2880, 2880, 1024, 2, 128), (8, 512, 1024, 100000, 0, 128),
     (12, 1600, 1600, 1000, 2, 128), (257, 64, 128, 512, 0, 192),
     (4, 64, 128, 2 ** 31, 0, 192),                           # no 32-bit token count
     (256, 65536, 65536, 256, 0, 192),                        # more tiles than one launch
