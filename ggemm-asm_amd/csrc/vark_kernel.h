@@ -621,7 +621,8 @@ __device__ __forceinline__ Sched make_sched(const VarKArgs& a, GG_LDS int* s_ord
       if (lane >= d) incl += v;
     }
     if (lane == 63) s_pred[wave] = (uint64_t)incl;
-    if (tid == 0) s_bound[0] = 0;
+    // zero stays where x / 4 of the work is less than one (a tile or two in all): no slot reaches it anew
+    if (tid < kXcdPairs) s_bound[tid] = 0;
     __syncthreads();
     int64_t before = incl - sum, total_w = 0;
 #pragma unroll

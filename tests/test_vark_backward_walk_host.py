@@ -1,5 +1,7 @@
-"""CPU model of the backward walk of the rounds deal (make_sched in vark_kernel.h): the workgroups of
-the odd XCDs may take their tiles from the last one back."""
+"""CPU model of parts of make_sched (vark_kernel.h): the backward walk of the rounds deal, in which the
+workgroups of the odd XCDs may take their tiles from the last one back, and the slices' bounds."""
+import random
+
 import pytest
 
 
@@ -30,3 +32,34 @@ def test_backward_walk_takes_the_same_tiles(num_wg):
     for total in (1, num_wg - 1, num_wg, num_wg + 1, 2 * num_wg, 2 * num_wg + 7, 5 * num_wg + num_wg // 2, 7 * num_wg - 1):
         for p in range(min(num_wg, total)):
             assert _backward(p, num_wg, total) == _forward(p, num_wg, total)[::-1], (total, p)
+
+
+def _bounds(w_slot, tpg):
+    """The kernel's form: every slot looks for the targets that its work reaches."""
+    total_w, before = sum(w_slot) * tpg, 0
+    bounds = [0] * 4 + [len(w_slot) * tpg]
+    for sl, w in enumerate(w_slot):
+        after = before + w * tpg
+        for x in range(1, 4):
+            target = total_w * x // 4
+            if before < target <= after:
+                bounds[x] = sl * tpg + min(-(-(target - before) // w), tpg)
+        before = after
+    return bounds
+
+
+def _first_tiles(w_slot, tpg):
+    """Slice x starts at the first tile that x / 4 of all work precede."""
+    done = [0]
+    for w in w_slot:
+        done += [done[-1] + w * (i + 1) for i in range(tpg)]
+    return [next(t for t, d in enumerate(done) if d >= done[-1] * x // 4) for x in range(4)] + [len(done) - 1]
+
+
+def test_slice_bounds_also_of_one_tile():
+    """The bounds of the smallest launches included, where a quarter of the work rounds to nothing."""
+    rng = random.Random(0)
+    small = [([w] * G, tpg) for w in (1, 2, 3, 5) for G in (1, 2, 3) for tpg in (1, 2, 3)]
+    for w_slot, tpg in small + [([rng.randint(1, 99) for _ in range(rng.randint(1, 40))], rng.randint(1, 50))
+                                for _ in range(200)]:
+        assert _bounds(w_slot, tpg) == _first_tiles(w_slot, tpg), (w_slot, tpg)
