@@ -168,3 +168,23 @@ def test_launches_of_one_to_three_tiles_on_the_192_row_kernel(pkg, cuda, lens):
         bad, _ = vark_oracle.mfma_bound_violations(got.double().cpu().numpy(), bytes_l, bytes_r, o.cpu().numpy(),
                                                    scale, scale, **{k: v.cpu().numpy() for k, v in kw.items()})
         assert not bad.any()
+
+
+@pytest.mark.parametrize("mode", ["bf16", "f32", "accumulate"])
+def test_wgrad_empty_groups_do_not_see_the_scales(pkg, cuda, mode):
+    """A group without tokens gives zeros and leaves an accumulated C as it is, -0 included, also where
+    a scale is NaN or infinite (an activation was)."""
+    lens, m, n = [0, 5, 0, 200], 64, 144
+    gen = torch.Generator().manual_seed(3)
+    offs = torch.tensor([0] + lens, device=cuda).cumsum(0)
+    assert pkg.load_library().ggemm_vark_tile_rows(len(lens), m, n, n, int(mode != "bf16"), sum(lens), 256) == 128
+    lhs, rhs = (_fp8_bytes((sum(lens), w), gen, 0, cuda) for w in (m, n))
+    one = torch.ones((), device=cuda)
+    for bad in (float("nan"), float("inf")):
+        c0 = torch.full((len(lens), m, n), -0.0 if mode == "accumulate" else 7.0,
+                        dtype=torch.bfloat16 if mode == "bf16" else torch.float32, device=cuda)
+        c = pkg.grouped_gemm_fp8_tensorwise_variable_k(lhs, rhs, one * bad, one, offs, out=c0.clone(),
+                                                       out_dtype=c0.dtype, accumulate=mode == "accumulate")
+        for g in (0, 2):
+            assert bool((c[g] == 0).all()) and bool(torch.signbit(c[g]).all()) == (mode == "accumulate")
+        assert not bool(torch.isfinite(c[1]).any()) and not bool(torch.isfinite(c[3]).any())
