@@ -164,6 +164,6 @@ __device__ __forceinline__ void gemm_body(const nt::Args& a, GG_LDS uint8_t* lds
                          stride_am, stride_bg, stride_bn, stride_cm, stride_cn, m_total, zero_tail};     \
     (void)global_scratch; (void)profile_scratch;                                                        \
     if (G > 0 && G <= ggemm::mid::kMaxGroups && K > 0 && N > 0)                                          \
-      ggemm::mid::gemm_body<AE5M2, BM>(args, (GG_LDS uint8_t*)ggemm_mid_lds);                             \
+      ggemm::mid::gemm_body<AE5M2, BM>(ggemm::nt::without_tail(args), (GG_LDS uint8_t*)ggemm_mid_lds);    \
     ggemm::nt::clear_tail_rows(args);                                                                   \
   }

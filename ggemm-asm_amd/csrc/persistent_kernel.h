@@ -82,6 +82,18 @@ __device__ __forceinline__ void clear_tail_rows(const Args& a) {
   if (a.zero_tail) clear_tail_rows(a.c, a.stride_cm, a.N, a.group_offs, a.G, a.m_total);
 }
 
+// The arguments that the GEMM of a launch with zero_tail runs on: groups end at offs[G], so that the rows
+// from there on are written by clear_tail_rows alone, which nothing orders against the tiles (offsets that
+// decrease let an earlier group end past offs[G]: those rows became zero when a later launch cleared them,
+// and do now).
+__device__ __forceinline__ Args without_tail(Args a) {
+  if (a.zero_tail) {
+    const int64_t end = a.group_offs[a.G];
+    a.m_total = end < 0 ? 0 : (end < a.m_total ? end : a.m_total);
+  }
+  return a;
+}
+
 __device__ __forceinline__ int workgroups(const Args& a) {
   if (a.num_wg > 0) return a.num_wg;
   const hsa_kernel_dispatch_packet_t* pkt = dispatch_packet();
@@ -509,6 +521,6 @@ __device__ __forceinline__ void persistent_entry(const Args& a, GG_LDS uint8_t* 
                          stride_am, stride_bg, stride_bn, stride_cm, stride_cn, m_total, zero_tail,      \
                          (int)gridDim.x};                                                               \
     (void)global_scratch; (void)profile_scratch;                                                        \
-    ggemm::nt::persistent_entry<AE5M2>(args, (GG_LDS uint8_t*)ggemm_dyn_lds);                             \
+    ggemm::nt::persistent_entry<AE5M2>(ggemm::nt::without_tail(args), (GG_LDS uint8_t*)ggemm_dyn_lds);    \
     ggemm::nt::clear_tail_rows(args);                                                                   \
   }

@@ -169,6 +169,6 @@ __device__ __forceinline__ void persistent_wide_body(const nt::Args& a, GG_LDS u
                          (int)gridDim.x};                                                               \
     (void)global_scratch; (void)profile_scratch;                                                        \
     if (G > 0 && G <= ggemm::nt::kMaxGroups && ggemm::pw::fits(N, K))                                   \
-      ggemm::persistent_wide_body<AE5M2>(args, (GG_LDS uint8_t*)ggemm_pw_lds);                           \
+      ggemm::persistent_wide_body<AE5M2>(ggemm::nt::without_tail(args), (GG_LDS uint8_t*)ggemm_pw_lds);  \
     ggemm::nt::clear_tail_rows(args);                                                                   \
   }

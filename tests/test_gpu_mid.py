@@ -188,3 +188,24 @@ def test_wgrad_empty_groups_do_not_see_the_scales(pkg, cuda, mode):
         for g in (0, 2):
             assert bool((c[g] == 0).all()) and bool(torch.signbit(c[g]).all()) == (mode == "accumulate")
         assert not bool(torch.isfinite(c[1]).any()) and not bool(torch.isfinite(c[3]).any())
+
+
+@pytest.mark.parametrize("N,K,kernel", [(208, 272, "auto"), (2048, 528, "auto"), (208, 272, "512"), (640, 128, "wide")])
+@pytest.mark.parametrize("offs", [[0, 300, 200], [0, 700, 650, 10], [0, 90, -5], [0, 100, 2000]], ids=str)
+def test_zero_tail_past_offsets_that_decrease(pkg, cuda, offs, N, K, kernel):
+    """Rows from the last offset on become zero also where an earlier group ends past it (its tiles write
+    none of them), the rows before it are the GEMM's; all rows for a negative last offset, none for one
+    past the rows."""
+    gen = torch.Generator().manual_seed(N)
+    M, G, s = 700, len(offs) - 1, torch.tensor(0.01, device=cuda)
+    a = _fp8_bytes((M, K), gen, 0, cuda).view(torch.float8_e4m3fn)
+    b = _fp8_bytes((G, N, K), gen, 0, cuda).view(torch.float8_e4m3fn)
+    at = torch.tensor(offs, device=cuda)
+    buf = torch.full((2, M + 64, N + 16), 7.0, dtype=torch.bfloat16, device=cuda)
+    for z in (0, 1):
+        pkg.grouped_gemm_fp8_tensorwise(a, b, s, s, at, out=buf[z, :M, :N], kernel=kernel, zero_tail=bool(z))
+    torch.cuda.synchronize()
+    rows = min(max(offs[-1], 0), M)
+    assert torch.equal(buf[0, :rows].view(torch.int16), buf[1, :rows].view(torch.int16))
+    assert bool((buf[1, rows:M, :N] == 0).all())
+    assert bool((buf[1, M:] == 7).all()) and bool((buf[1, :, N:] == 7).all())
