@@ -209,3 +209,20 @@ def test_zero_tail_past_offsets_that_decrease(pkg, cuda, offs, N, K, kernel):
     assert torch.equal(buf[0, :rows].view(torch.int16), buf[1, :rows].view(torch.int16))
     assert bool((buf[1, rows:M, :N] == 0).all())
     assert bool((buf[1, M:] == 7).all()) and bool((buf[1, :, N:] == 7).all())
+
+
+def test_gemm_rows_of_several_groups(pkg, cuda):
+    """Offsets that fall and rise again: rows of several groups have more tiles than the launch has
+    workgroups, and the rows that only the last of them holds are computed too. One weight for all
+    groups, so that every row has one result."""
+    N, K, M = 128, 272, 512
+    gen = torch.Generator().manual_seed(1)
+    offs = torch.tensor([0, 400] * 127 + [0, 512], device=cuda)
+    G, s = offs.numel() - 1, torch.tensor(0.01, device=cuda)
+    assert pkg.persistent.tile_rows(G, N, K, K, K, N, M) == 64
+    a = _fp8_bytes((M, K), gen, 0, cuda).view(torch.float8_e4m3fn)
+    b = _fp8_bytes((1, N, K), gen, 0, cuda).view(torch.float8_e4m3fn)
+    out = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=cuda)
+    pkg.grouped_gemm_fp8_tensorwise(a, b.expand(G, N, K).contiguous(), s, s, offs, out=out)
+    one = pkg.grouped_gemm_fp8_tensorwise(a, b, s, s, torch.tensor([0, M], device=cuda), kernel="512")
+    assert torch.equal(out.view(torch.int16), one.view(torch.int16))

@@ -1,4 +1,6 @@
 """CPU checks of the choice between the mid-tile and the large-tile kernels."""
+import random
+
 import pytest
 
 
@@ -41,3 +43,27 @@ def test_wgrad_unaligned_rows_of_c_keep_the_192_row_kernel(pkg):
     rows = pkg.load_library().ggemm_vark_tile_rows
     assert rows(4, 64, 128, 136, 0, 512, 256) == 128 and rows(4, 64, 128, 132, 0, 512, 256) == 192
     assert rows(4, 64, 128, 132, 1, 512, 256) == 128
+
+
+def test_gemm_workgroups_cover_the_tiles_of_any_offsets():
+    """Model of the mid-tile GEMM's grid (capi) and walk (gemm_body): every tile is taken by one workgroup,
+    also where offsets decrease and rise again and the groups' tiles outnumber the workgroups."""
+    rng = random.Random(0)
+    for rows in (64, 128):
+        for _ in range(300):
+            G, M, n_tn = rng.randint(1, 256), rng.randint(1, 3000), rng.randint(1, 9)
+            offs = [rng.randint(0, M) for _ in range(G + 1)]
+            if rng.random() < 0.5:
+                offs.sort()
+            bound = (M // rows + min(G, M)) * n_tn
+            grid = -(-bound // 256) * 256
+            total = sum(-(-max(b - a, 0) // rows) * n_tn for a, b in zip(offs, offs[1:]))
+            assert offs != sorted(offs) or total <= grid
+            taken = []
+            for b in range(grid):
+                r = b % 256
+                t = b - r + (r % 8) * 32 + r // 8
+                while t < total:
+                    taken.append(t)
+                    t += grid
+            assert sorted(taken) == list(range(total))
