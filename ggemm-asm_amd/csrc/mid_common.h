@@ -74,7 +74,9 @@ __device__ __forceinline__ int pick(const int (&v)[4], int lane, int x) {
 
 typedef unsigned v4u32 __attribute__((ext_vector_type(4)));
 
-// The rows of C that a wave stores, as a buffer: rows past it are neither read nor written.
+// The rows of C that a wave stores, as a buffer: rows past it are neither read nor written. A row's offset
+// goes into the lane offset, which the range check compares with num_records; with it in the scalar offset
+// the check subtracts that from num_records, and rows past the block are those where this is negative.
 struct CBlock {
   __amdgpu_buffer_rsrc_t rsrc;
   int pitch;                        // bytes between rows (64 of them within kOob: host-checked)
@@ -82,12 +84,11 @@ struct CBlock {
   __device__ __forceinline__ CBlock(T* c, int64_t stride, int rows)
       : rsrc(__builtin_amdgcn_make_buffer_rsrc(c, 0, max(0, min(rows, 64)) * (int)(stride * sizeof(T)), kRsrcWord3)),
         pitch((int)(stride * sizeof(T))) {}
-  __device__ __forceinline__ v4i load(int voff, int soff) const {
-    return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, soff, 0));
+  __device__ __forceinline__ v4i load(uint32_t off) const {
+    return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, 0));
   }
-  __device__ __forceinline__ void store(v4i v, int voff, int soff) const {   // non-temporal
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u32, v), rsrc,
-                                           voff, soff, 2);
+  __device__ __forceinline__ void store(v4i v, uint32_t off) const {   // non-temporal
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u32, v), rsrc, (int)off, 0, 2);
   }
 };
 
@@ -110,12 +111,12 @@ __device__ __forceinline__ void store_bf16(const v4f (&acc)[4][NB], float alpha,
   // row 64 n / kChunks + lane / kChunks, chunk lane % kChunks: rows past the block fall outside the
   // resource, the other columns' lanes too
   const CBlock b(c, stride, rows);
-  const int v = 8 * (lane % kChunks) < cols ? lane / kChunks * b.pitch + 16 * (lane % kChunks) : (int)kOob;
+  const uint32_t v = 8 * (lane % kChunks) < cols ? lane / kChunks * b.pitch + 16 * (lane % kChunks) : kOob;
 #pragma unroll
   for (int n = 0; n < kChunks; ++n) {
     const int f = 64 * n + lane, r = f / kChunks, k = f % kChunks;
-    b.store(*(const GG_LDS v4i*)(reg + r * kRow + 16 * (k ^ ((r >> 1) & (kChunks - 1)))), v,
-            n * (64 / kChunks) * b.pitch);
+    b.store(*(const GG_LDS v4i*)(reg + r * kRow + 16 * (k ^ ((r >> 1) & (kChunks - 1)))),
+            v + (uint32_t)(n * (64 / kChunks) * b.pitch));
   }
 }
 
@@ -126,13 +127,13 @@ __device__ __forceinline__ void store_f32(const v4f (&acc)[4][4], float alpha, G
                                           int64_t stride, int rows, int cols, int lane) {
   const int q = lane >> 4, s16 = lane & 15;
   const CBlock b(c, stride, rows);
-  const int v = 4 * s16 < cols ? q * b.pitch + 16 * s16 : (int)kOob;
+  const uint32_t v = 4 * s16 < cols ? q * b.pitch + 16 * s16 : kOob;
 #pragma unroll
   for (int p = 0; p < 2; ++p) {
     v4f old[8];
     if constexpr (kAdd) {
 #pragma unroll
-      for (int n = 0; n < 8; ++n) old[n] = __builtin_bit_cast(v4f, b.load(v, (32 * p + 4 * n) * b.pitch));
+      for (int n = 0; n < 8; ++n) old[n] = __builtin_bit_cast(v4f, b.load(v + (uint32_t)((32 * p + 4 * n) * b.pitch)));
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -146,7 +147,7 @@ __device__ __forceinline__ void store_f32(const v4f (&acc)[4][4], float alpha, G
       const int r = 4 * n + q;
       v4f x = *(const GG_LDS v4f*)(reg + r * 256 + 16 * (s16 ^ (r & 15)));
       if constexpr (kAdd) x += old[n];
-      b.store(__builtin_bit_cast(v4i, x), v, (32 * p + 4 * n) * b.pitch);
+      b.store(__builtin_bit_cast(v4i, x), v + (uint32_t)((32 * p + 4 * n) * b.pitch));
     }
   }
 }
