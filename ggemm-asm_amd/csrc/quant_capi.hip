@@ -39,18 +39,40 @@ int grid_for(int64_t chunks, int cus, int per_cu) {
   return (int)(want < 1 ? 1 : (want > cap ? cap : want));
 }
 
+// What reads x after its amax pass.
+enum class Next { kNothing, kStreaming, kTransposing };
+
+// Whether the amax pass loads x the ordinary way (load8), so that the next pass finds part of it in the
+// memory-side cache, or non-temporally, the faster way to read it once. Measured (us, non-temporal ->
+// ordinary, both passes): bf16 streaming 50 MB 28.6 -> 25.7, 800 MB 325.3 -> 322.1, 1 GB 405.6 -> 403.8,
+// 1.3 GB 525.5 -> 527.3, 4 GB 1731 -> 1756; bf16 transposing 200 MB 113.7 -> 106.7, 300 MB 167.2 -> 166.2,
+// 450 MB 247.8 -> 251.3, 1 GB 553.8 -> 565.3; bf16 alone 50 MB 24.7 -> 25.1, 1 GB 152.1 -> 163.8. fp32 takes
+// twice as long over a byte and gains at every size (33 MB 19.3 -> 15.5, 4 GB 1629 -> 1596; transposing
+// 22.6 -> 18.7, 1923 -> 1890); alone 300 MB 58.6 -> 59.3, 600 MB 104.2 -> 103.4, 4 GB 674.8 -> 647.9.
+bool amax_keeps(int64_t bytes, bool f32, Next next) {
+  constexpr int64_t kMB = 1000 * 1000;
+  if (f32) return next != Next::kNothing || bytes > 500 * kMB;
+  return bytes <= (next == Next::kStreaming ? 1100 * kMB : next == Next::kTransposing ? 300 * kMB : 0);
+}
+
+template <bool kPartials, bool kKeep>
+auto amax_kernel_of(bool f32) {
+  return f32 ? qt::amax_kernel<true, kPartials, kKeep> : qt::amax_kernel<false, kPartials, kKeep>;
+}
+
 // The amax of x into *amax, zeroed by a launch of its own; or, with a workspace, the workgroups' partial
 // maxima into it, their number returned (0 for no rows).
 int launch_amax(const void* x, int in_dtype, int64_t rows, int cols, int64_t stride, float* amax,
-                uint32_t* workspace, int cus, hipStream_t s) {
+                uint32_t* workspace, Next next, int cus, hipStream_t s) {
   uint32_t* bits = workspace ? workspace : reinterpret_cast<uint32_t*>(amax);
   if (!workspace) hipLaunchKernelGGL(qt::amax_init, dim3(1), dim3(64), 0, s, bits);
   if (rows == 0) return workspace ? 0 : 1;
   int grid = grid_for(rows * (cols / 8), cus, kAmaxPerCu);
   if (grid > qt::kMaxPartials) grid = qt::kMaxPartials;
   const bool f32 = in_dtype == GGEMM_IN_F32;
-  auto k = f32 ? (workspace ? qt::amax_kernel<true, true> : qt::amax_kernel<true, false>)
-               : (workspace ? qt::amax_kernel<false, true> : qt::amax_kernel<false, false>);
+  const bool keep = amax_keeps(rows * cols * (f32 ? 4 : 2), f32, next);
+  auto k = workspace ? (keep ? amax_kernel_of<true, true>(f32) : amax_kernel_of<true, false>(f32))
+                     : (keep ? amax_kernel_of<false, true>(f32) : amax_kernel_of<false, false>(f32));
   hipLaunchKernelGGL(k, dim3(grid), dim3(qt::kThreads), 0, s, x, rows, cols, stride, bits);
   return workspace ? grid : 1;
 }
@@ -100,7 +122,7 @@ int ggemm_quant_amax(const void* x, int32_t in_dtype, int64_t rows, int32_t cols
   int cus = 0;
   rc = device_cus(&cus);
   if (rc) return rc;
-  launch_amax(x, in_dtype, rows, cols, stride, amax_out, nullptr, cus, (hipStream_t)stream);
+  launch_amax(x, in_dtype, rows, cols, stride, amax_out, nullptr, Next::kNothing, cus, (hipStream_t)stream);
   return (int)hipGetLastError();
 }
 
@@ -118,7 +140,7 @@ static int tensorwise(const void* x, int32_t in_dtype, int64_t rows, int32_t col
   rc = device_cus(&cus);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  const int n = launch_amax(x, in_dtype, rows, cols, stride, amax_out, workspace, cus, s);
+  const int n = launch_amax(x, in_dtype, rows, cols, stride, amax_out, workspace, Next::kStreaming, cus, s);
   const int grid = grid_for(rows * (cols / 8), cus, kQuantPerCu);
   const uint32_t* partials = workspace ? workspace : reinterpret_cast<const uint32_t*>(amax_out);
   uint8_t* o = static_cast<uint8_t*>(out);
@@ -239,7 +261,8 @@ static int tensorwise_transpose(const void* x, int32_t in_dtype, int32_t batch, 
   rc = device_cus(&cus);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  const int n = launch_amax(x, in_dtype, (int64_t)batch * rows, cols, cols, amax_out, workspace, cus, s);
+  const int n = launch_amax(x, in_dtype, (int64_t)batch * rows, cols, cols, amax_out, workspace, Next::kTransposing,
+                            cus, s);
   const uint32_t* partials = workspace ? workspace : reinterpret_cast<const uint32_t*>(amax_out);
   const bool f32 = in_dtype == GGEMM_IN_F32, e5 = out_format == GGEMM_FP8_E5M2;
   auto k = f32 ? (e5 ? qt::quant_transpose_kernel<true, true> : qt::quant_transpose_kernel<true, false>)

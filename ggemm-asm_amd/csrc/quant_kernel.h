@@ -94,12 +94,11 @@ __device__ __forceinline__ float clamp_fmax(float v) {
 __device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 
-// 8 consecutive elements of row `row`, chunk `c` (elements 8c .. 8c+7), as fp32. kKeep: ordinary loads, in
-// the amax pass, whose x the quantizing pass reads again, and in the transposing pass after it: what the
-// memory-side cache still holds is not fetched twice ([4, 5760, 2880] bf16 with its transpose 77.2 -> 72.5
-// us, in fp32 152.5 -> 108.8 us, [131072, 2880] 313.3 -> 307.4 us; of 1.5 GB nothing is left to find:
-// [131072, 5760] 614.6 -> 620.0 us). Else non-temporal ones: a streaming pass that reads x for the
-// last time is faster with them (331 us instead of 307 with ordinary loads there too).
+// 8 consecutive elements of row `row`, chunk `c` (elements 8c .. 8c+7), as fp32. kKeep: ordinary loads, which
+// leave x in the memory-side cache for a pass that reads it next (the amax pass, by the rule at its launch)
+// and find it there (the transposing pass: [4, 5760, 2880] bf16 with its transpose 77.2 -> 72.5 us, in fp32
+// 152.5 -> 108.8 us). Else non-temporal ones: a streaming pass that reads x for the last time is faster with
+// them (307 us, 331 with ordinary loads there too, for [131072, 2880]).
 template <bool kF32, bool kKeep = false>
 __device__ __forceinline__ void load8(const void* x, int64_t row, int64_t stride, int c, float v[8]) {
   if constexpr (kF32) {
@@ -201,7 +200,7 @@ __device__ __forceinline__ uint32_t partials_amax(const uint32_t* partials, int 
 // larger than +inf, so NaN propagates): one atomic per workgroup into *amax_bits, or (kPartials) the
 // workgroup's own maximum in amax_bits[blockIdx.x], which needs no zeroing launch before (4-5 us of a
 // small tensor's 14) and is combined by the pass that uses it (partials_amax)
-template <bool kF32, bool kPartials>
+template <bool kF32, bool kPartials, bool kKeep>
 __global__ void __launch_bounds__(kThreads) amax_kernel(const void* x, int64_t rows, int cols, int64_t stride,
                                                         uint32_t* amax_bits) {
   const int cpr = cols / 8;
@@ -215,7 +214,7 @@ __global__ void __launch_bounds__(kThreads) amax_kernel(const void* x, int64_t r
     float v[kUnroll][8];
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
-      if (i0 + u * T < n) load8<kF32, true>(x, cw.row[u], stride, cw.col[u], v[u]);
+      if (i0 + u * T < n) load8<kF32, kKeep>(x, cw.row[u], stride, cw.col[u], v[u]);
       else for (int k = 0; k < 8; ++k) v[u][k] = 0.0f;
     }
 #pragma unroll
