@@ -134,7 +134,7 @@ def quantize_fp8_tensorwise_delayed(x: torch.Tensor, amax_history: torch.Tensor,
         name, at = "ggemm_quant_fp8_tensorwise_delayed_dev", slot.data_ptr()
     else:
         name, at = "ggemm_quant_fp8_tensorwise_delayed", operator.index(slot)
-    _lib.launch(name, dev, cols, _ptr(x2), _IN[x.dtype], rows, cols, _row_stride(x2), code, qp.data_ptr(),
+    _lib.launch(name, dev, cols | H, _ptr(x2), _IN[x.dtype], rows, cols, _row_stride(x2), code, qp.data_ptr(),
                 q.stride(-2) if rows > 1 else cols, amax_history.data_ptr(), H, at, scale.data_ptr())
     return q, scale
 
@@ -205,7 +205,8 @@ def _transpose(x, fmt, keep, row_align, amax_history, slot):
         name, at = "ggemm_quant_fp8_tensorwise_transpose_delayed_dev", slot.data_ptr()
     else:
         name, at = "ggemm_quant_fp8_tensorwise_transpose_delayed", operator.index(slot)
-    _lib.launch(name, x.device, B | R | C, *common, amax_history.data_ptr(), amax_history.numel(), at, scale.data_ptr())
+    H = amax_history.numel()
+    _lib.launch(name, x.device, B | R | C | H, *common, amax_history.data_ptr(), H, at, scale.data_ptr())
     return q, q_t, scale, None
 
 

@@ -5,7 +5,7 @@ import torch
 from __graft_entry__ import load_package
 
 load_package()
-from ggemm_asm_amd import _lib, vark  # noqa: E402
+from ggemm_asm_amd import _lib, quant, vark  # noqa: E402
 
 
 @pytest.fixture
@@ -30,3 +30,13 @@ def test_weight_grad_scales_are_checked(launches, bad):
         with pytest.raises(ValueError, match="scales"):
             vark.weight_grad_fp8(dy, x, *scales, offs)
     assert len(launches) == 1
+
+
+@pytest.mark.parametrize("op", ["quantize_fp8_tensorwise_delayed", "quantize_fp8_tensorwise_transpose_delayed"])
+@pytest.mark.parametrize("slot", [3, 2 ** 32 + 3, torch.zeros(1, dtype=torch.int32, device="meta")], ids=str)
+def test_history_lengths_past_32_bits_are_refused(monkeypatch, op, slot):
+    """A history of 2^32 + 16 entries is no history of 16, nor its slot 2^32 + 3 the slot 3."""
+    monkeypatch.setattr(quant, "_check", lambda x, fmt: None)
+    x = torch.empty((32, 64), dtype=torch.bfloat16, device="meta")
+    with pytest.raises(OverflowError):
+        getattr(quant, op)(x, torch.empty(2 ** 32 + 16, device="meta"), slot)
