@@ -130,6 +130,35 @@ int64_t mid_tiles(int rows, int G, int N, int64_t M_total) {
   return (M_total / rows + (G < M_total ? G : M_total)) * ((N + 127) / 128);
 }
 
+// The second look at a launch that the estimate of mid_preferred gives to 128-row tiles: both sides in whole
+// rounds, for rows spread evenly over the groups and for any (half a row tile more for each group), and the
+// mean of the two. 569 of 6112 drawn launches for the mid tiles (1 to 64 groups, 1 to 60000 rows, features 64
+// to 5760, even, exponential and Zipf lengths) were given 128 rows, 51 of them more than 3 % slower than the
+// large tiles and 31 more than 10 %: 13 groups, 5788 rows, N = K = 2880 75 us, 51 on the wide tiles; 15, 7007,
+// N = 2560, K = 5760 112, 85. Of the 702 in another draw 21 were slower than before there were mid tiles, 10 by more
+// than 10 %; with this rule 10 and 2 are, and 12 lose a gain of 20 % or more (14
+// and 6 of the 851 that it leaves of a third draw).
+bool rows128_faster(int N, double M, double g, double stages, double mem, bool wide, int cus) {
+  constexpr int kRun = ggemm::mid::kXcdRun;
+  const int tn = wide ? 320 : ggemm::wide_tiles(N, false) ? 384 : 320;
+  double mid = 0, big = 0;
+  for (const bool even : {true, false}) {
+    auto tiles = [&](double h, double w) {
+      return (even ? g * std::ceil(M / g / h) : std::max(1.0, M / h + g / 2)) * std::ceil(N / w);
+    };
+    const double t = tiles(128, 128), all = ggemm::kXcds * kRun, runs = std::floor(t / all);
+    // half rounds of two workgroups on every CU of the XCD that takes most tiles (tile_of_block)
+    const double most = kRun * runs + std::min<double>(kRun, t - runs * all);
+    const double half = std::ceil(most * ggemm::kXcds / cus);
+    mid += 6.6 + (0.976 * half / 2 - 0.28) * (stages + 2) + 0.33 * mem;
+    const double r = std::ceil(tiles(wide ? ggemm::pw::kTM : ggemm::kTileM, tn) / cus);
+    big += wide        ? 2.6 + r * (1.19 * stages + 6.1) + 0.32 * mem
+           : tn == 320 ? 2.0 + r * (1.12 * stages + 6.8) + 0.29 * mem
+                       : 4.6 + r * (1.27 * stages + 5.0) + 0.43 * mem;
+  }
+  return mid < 1.05 * big;
+}
+
 // The mid-tile kernel's row-tile height (64 or 128) where it is the faster one, else 0: the estimated
 // microseconds of each kernel compared. The lengths of the groups are on the device; M_total rows over
 // G groups are taken to make max(g, M_total / height + g / 2) row tiles, g the groups that can have a
@@ -158,7 +187,8 @@ int mid_preferred(int G, int N, int K, int scm, int64_t M_total, bool wide, int 
   const double c64 = 4 + std::max(1.0, f64) * stages * (0.41 + 0.28 * std::min(1.0, f64)) + 0.3 * mem;
   const double c128 = 4 + std::max(1.0, f128) * stages * (0.64 + 0.42 * std::min(1.0, f128)) + 0.3 * mem;
   if (std::min(c64, c128) >= 0.92 * big) return 0;   // near the line the estimate is a few per cent off
-  return c64 < 0.97 * c128 ? 64 : 128;
+  if (c64 < 0.97 * c128) return 64;
+  return rows128_faster(N, M, g, (K + 127) / 128, mem, wide, cus) ? 128 : 0;
 }
 
 int launch(const void* a, const void* b, void* out, const float* a_scale, const float* b_scale,

@@ -86,6 +86,38 @@ int64_t mid_tiles(int G, int OUT_M, int OUT_N) {
          ((OUT_N + ggemm::mid::kWT - 1) / ggemm::mid::kWT);
 }
 
+// The second look at a launch that the estimate of mid_preferred gives to the mid tiles: with tiles of equal
+// lengths both sides run in whole rounds, which that estimate, made for the tails of many unlike tiles, spreads
+// out, and the larger tiles' rates and fixed costs are those of launches without the read of the dispatch
+// packet. Mid tiles: 1.15 of a tile's time a round of two to a CU, 0.8 the last one with one to a CU, on the
+// XCD that takes most of them (tile_of_block); 192-row ones: 1.62, and 1.1 to 1.6 for a last round; wide 1.67.
+// Over 3800 drawn launches that went to the mid tiles (1 to 64 groups, 1 to 131072 tokens, features 64 to
+// 5760, even, exponential and Zipf lengths) 102 were more than 3 % slower than before there were mid tiles, 58
+// more than 10 %: [1, 2880, 2880] of 100930 tokens 1843 us, 1403 on the large tiles; [5, 2544, 1744] of 17692
+// 122, 94; [2, 2880, 3312] of 106369 1574, 1122. With this rule 20 and 7 are (34 and 15 of the 3847 that it
+// leaves of another draw); 56 lose a gain of 20 % or more (lengths so unlike that the longest group alone
+// counts).
+bool whole_rounds_faster(int G, int OUT_M, int OUT_N, bool f32, double stages, int wide_tile, int cus) {
+  constexpr int kRun = ggemm::mid::kXcdRun;
+  const int64_t t = mid_tiles(G, OUT_M, OUT_N), all = ggemm::kXcds * kRun;
+  const double slots = 2.0 * cus / ggemm::kXcds;             // of an XCD
+  const double r = (kRun * (t / all) + std::min<int64_t>(kRun, t % all)) / slots, rest = r - std::floor(r);
+  const double c_us = (double)G * OUT_M * OUT_N * (f32 ? 6 : 2) / 5e6;   // C written; fp32: the two modes' mean
+  const double mid = 3.5 + (1.15 * std::floor(r) + (rest == 0 ? 0 : rest <= 0.5 ? 0.8 : 1.15)) * (0.88 * stages + 3.3) +
+                     (f32 ? 0.2 * c_us : 0);
+  auto rounds = [&](int h, int n) { return (double)G * ((OUT_M + h - 1) / h) * ((OUT_N + n - 1) / n) / cus; };
+  double big;
+  if (wide_tile) {
+    big = 9 + std::ceil(wide_tile == 320 ? rounds(320, 320) : rounds(256, 384)) * (1.67 * stages + 4) +
+          (f32 ? 0.7 * c_us : 0);
+  } else {
+    const double b = rounds(ggemm::kTileM, ggemm::wide_tiles(OUT_N, false) ? 384 : 320), last = b - std::floor(b);
+    big = 10 + (1.62 * std::floor(b) + (last == 0 ? 0 : b < 1 ? 1.2 + 0.55 * last : 1.1 + 0.5 * last)) * (stages + 1) +
+          0.85 * c_us;
+  }
+  return mid < 0.95 * big;
+}
+
 // Whether the mid-tile kernel is the faster one: the estimated microseconds of both sides compared,
 // M_total / G tokens in every group. Per 128-token stage and tile: 2.06 us for a wide tile and 1.2
 // (few CUs busy) to 2.1 us for a 192-row one, tiles one to a CU in whole rounds; 0.55 (few) to 1.27 us
@@ -115,7 +147,8 @@ bool mid_preferred(int G, int OUT_M, int OUT_N, int64_t scm, int64_t scg, const 
     const double t = tiles(ggemm::kTileM, ggemm::wide_tiles(OUT_N, false) ? 384 : 320) / cus;
     big = 7 + std::ceil(t) * (stages + 3) * (1.2 + 0.9 * std::min(1.0, t));
   }
-  return mid < 0.92 * big;                                   // near the line the estimate is a few per cent off
+  if (mid >= 0.92 * big) return false;                       // near the line the estimate is a few per cent off
+  return whole_rounds_faster(G, OUT_M, OUT_N, f32, stages, wide_tile, cus);
 }
 
 // swapped: e5m2 LHS, e4m3 RHS (bf16 C only)
