@@ -373,6 +373,40 @@ def make_runner(pkg, p, dev, mfma, kernel="auto", row_align=0):
     return run
 
 
+MID_TILES = "hip gfx950 {}x128 tiles, one to a 256-thread workgroup, 128-K stages, mfma k128"
+
+
+def fwd_kernel_text(pkg, p, kernel, stride, cus):
+    """The kernel that a forward / data-gradient launch runs on contiguous C rows: the one asked for, or the
+    library's choice for this many rows and groups."""
+    rows = {"wide": 256, "512": 192}.get(kernel)
+    rows = rows or pkg.persistent.tile_rows(p.G, p.N, p.K, stride, stride, p.N, p.M, cus)
+    if rows == 256:
+        return ("hip gfx950 persistent wide 256x320 tiles (256 threads, one wave per SIMD, generated assembly), 128-K "
+                "stages, mfma 32x32x64")
+    if rows == 192:
+        return "hip gfx950 persistent {tile_m}x{tile_n} tiles, 128-K stages, mfma k128".format(
+            **pkg.launch_geometry(p.N))
+    return MID_TILES.format(rows)
+
+
+def wgrad_kernel_text(pkg, p, mfma, out, cus):
+    """The kernel that a wgrad launch runs on a contiguous C; the MX entry takes no mid tiles."""
+    if p.is_mx:
+        rows = 320 if pkg.bf16_kernel(p.OUT_M, p.OUT_N) == "wide320" else 192
+    elif mfma != "k128":
+        rows = 192
+    else:
+        rows = pkg.load_library().ggemm_vark_tile_rows(p.G, p.OUT_M, p.OUT_N, p.OUT_N, int(out != "bf16"), p.M, cus)
+    if rows in (320, 256):
+        return ("hip gfx950 persistent {}x{} tiles, 256-thread workgroups (one wave per SIMD, hand-placed "
+                "accumulators), mfma 32x32x64".format(rows, 320 if rows == 320 else 384))
+    if rows == 192:
+        return "hip gfx950 persistent {tile_m}x{tile_n} tiles, mfma {mfma}".format(
+            mfma=mfma, **pkg.launch_geometry(p.OUT_N))
+    return MID_TILES.format(rows)
+
+
 def time_steps(run, steps, warmup):
     import torch
     for _ in range(warmup):
@@ -882,20 +916,15 @@ def run_bench(args, sampler):
     # traffic measured for this exact variant (profiles/traffic_<config>[_<out>][_reference_lens].txt)
     traffic, traffic_source = read_traffic(args.config + ("" if args.out == "bf16" else "_" + args.out)
                                            + ("" if args.lens == "multinomial" else "_reference_lens"))
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
     if fwd:
-        geo = pkg.launch_geometry(p.N)
         stride = -(-p.K // args.row_align) * args.row_align if args.row_align else p.K
-        kern = args.persistent_kernel
-        if kern == "auto":
-            kern = pkg.persistent.selected_kernel(p.N, p.K, stride, stride, p.N)
         config = {"workload": p.name, "G": p.G, "M_total": p.M, "K": p.K, "N": p.N,
                   "a": {"e4m3": "e4m3fn", "e5m2": "e5m2"}[p.a_format], "b": "e4m3fn [G, N, K] (trans_b)",
                   "out": "bf16", "acc": "fp32",
                   "inputs": "reference recipe: seed-42 exponential group sizes, randn bf16 cast to fp8, "
                             "scales 0.1, in HBM" + (f", A and B row strides {stride} bytes" if stride != p.K else ""),
-                  "kernel": ("hip gfx950 persistent wide 256x320 tiles (256 threads, one wave per SIMD, generated "
-                             "assembly), 128-K stages, mfma 32x32x64" if kern == "wide"
-                             else "hip gfx950 persistent {tile_m}x{tile_n} tiles, 128-K stages, mfma k128".format(**geo)),
+                  "kernel": fwd_kernel_text(pkg, p, args.persistent_kernel, stride, cus),
                   "baseline_number": "none published for this site"}
         vs_baseline = None
     else:
@@ -907,13 +936,7 @@ def run_bench(args, sampler):
                   "inputs": "seeded N(0,1) / N(0,1e-3) quantized per-tensor, {} group sizes, in HBM".format(
                       "the reference's seed-42 exponential" if args.lens == "reference" else
                       {"gate_up_zipf": "Zipf-skewed"}.get(p.name, "multinomial")),
-                  "kernel": ("hip gfx950 persistent {}x{} tiles, 256-thread workgroups (one wave per SIMD, "
-                             "hand-placed accumulators), mfma 32x32x64".format(
-                                 *((320, 320) if pkg.bf16_kernel(p.OUT_M, p.OUT_N) == "wide320" else (256, 384)))
-                             if args.mfma == "k128" and pkg.bf16_kernel(p.OUT_M, p.OUT_N) != "192-row"
-                             and (not p.is_mx or pkg.bf16_kernel(p.OUT_M, p.OUT_N) == "wide320")
-                             else "hip gfx950 persistent {tile_m}x{tile_n} tiles, mfma {mfma}".format(
-                                 mfma=args.mfma, **pkg.launch_geometry(p.OUT_N))),
+                  "kernel": wgrad_kernel_text(pkg, p, args.mfma, args.out, cus),
                   "baseline_number": ("reference optimized ASM 3.515 ms / 1237 TFLOPS (README.md:60)"
                                       if p.name == "gate_up_wgrad" else "none published for this workload")}
         if p.is_mx:

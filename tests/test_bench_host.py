@@ -4,6 +4,7 @@ reference bench.py:594-648, cosine at :641-646). The checker must accept an exac
 result within the bar, and reject each kind of mistake the bar names: one element off by more than
 2e-2 relative, a non-finite value, a non-zero empty group, a wrong group (the cosine)."""
 import sys
+import types
 
 import numpy as np
 import pytest
@@ -177,3 +178,26 @@ def test_power_sampler_child(tmp_path, monkeypatch):
     assert s.proc.poll() is not None
     good = [x for x in samples if "watts" in x]
     assert len(good) >= 2 and all(x["watts"] == 1234.0 and x["mhz"] == 1905.0 for x in good), samples[:3]
+
+
+@pytest.mark.parametrize("G,M,m,n,mx,mfma,out,tiles", [
+    (4, 512, 64, 128, False, "k128", "bf16", "128x128"), (4, 512, 64, 128, False, "k32", "bf16", "192x320"),
+    (4, 512, 64, 128, True, "k128", "bf16", "192x320"), (32, 131072, 2880, 5760, False, "k128", "bf16", "320x320"),
+    (32, 131072, 2880, 5760, True, "k128", "bf16", "320x320"),
+    (32, 131072, 2880, 5760, False, "k128", "f32_accum", "320x320"),
+    (32, 131072, 2048, 1536, False, "k128", "bf16", "256x384"), (32, 131072, 2048, 1536, False, "k128", "f32", "192x384"),
+])
+def test_wgrad_kernel_named_by_the_launch(pkg, G, M, m, n, mx, mfma, out, tiles):
+    """The JSON line names the kernel that the launch's token count selects."""
+    p = types.SimpleNamespace(G=G, M=M, OUT_M=m, OUT_N=n, is_mx=mx)
+    assert f" {tiles} tiles" in bench.wgrad_kernel_text(pkg, p, mfma, out, 256)
+
+
+@pytest.mark.parametrize("G,M,N,K,kernel,tiles", [
+    (32, 131072, 5760, 2880, "auto", "256x320"), (32, 131072, 5760, 2880, "512", "192x384"),
+    (32, 256, 5760, 2880, "auto", "64x128"), (32, 256, 5760, 2880, "wide", "256x320"),
+    (32, 3072, 5760, 2880, "auto", "128x128"), (7, 5003, 2048, 1424, "auto", "192x320"),
+])
+def test_fwd_kernel_named_by_the_launch(pkg, G, M, N, K, kernel, tiles):
+    p = types.SimpleNamespace(G=G, M=M, N=N, K=K)
+    assert f" {tiles} tiles" in bench.fwd_kernel_text(pkg, p, kernel, K, 256)
