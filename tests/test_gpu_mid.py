@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from oracle import vark_oracle
+from test_vark_backward_walk_host import walks_backwards
 
 pytestmark = pytest.mark.gpu
 
@@ -98,16 +99,25 @@ def test_wgrad_equals_192_row_kernel(pkg, cuda, lens, m, n):
         harness.unload_kernel(module)
 
 
-@pytest.mark.parametrize("m,n", [(1280, 960), (2112, 1904)])
-def test_fp32_backward_walk_of_light_tiles(pkg, cuda, m, n):
+# m, n, lengths, tile rows, tiles of a group, stage, and for the fp32 and the accumulating mode (epilogue weight,
+# stages that a tile's C is worth) as the kernels give them to make_sched
+WALKS = [
+    (1600, 1600, [900, 200, 31, 200, 200, 200, 4524, 4389, 200, 64, 900, 4443, 1, 1, 1, 1, 31, 900, 200, 0, 31, 900,
+                  0, 1], 320, 25, 64, ((3, 16), (3, 32))),
+    (2112, 1904, [5000, 3000, 0, 7, 64, 1, 31, 900] * 4, 192, 55, 128, ((2, 8), (4, 16))),
+]
+
+
+@pytest.mark.parametrize("m,n,lens,tile,tpg,stage,modes", WALKS, ids=["wide", "192row"])
+def test_fp32_backward_walk_of_light_tiles(pkg, cuda, m, n, lens, tile, tpg, stage, modes):
     """Skewed lengths whose many small groups make the odd XCDs walk their tiles backwards, on the
-    wide and the 192-row kernel: the fp32 result rounds to the bf16 one (whose walk is forward) and
-    accumulating adds it exactly; the shape's tiles outnumber the workgroups."""
-    lens = [5000, 3000, 0, 7, 64, 1, 31, 900] * 4
+    wide and the 192-row kernel, several rounds of them: the fp32 result rounds to the bf16 one (whose walk
+    is forward), lies within the exact result's bound, and accumulating adds it exactly."""
+    assert all(walks_backwards(lens, tpg, stage, *mode) for mode in modes)
     gen = torch.Generator().manual_seed(m)
     offs = torch.tensor([0] + lens, device=cuda).cumsum(0)
     rows = pkg.load_library().ggemm_vark_tile_rows
-    assert rows(len(lens), m, n, n, 1, sum(lens), 256) == rows(len(lens), m, n, n, 0, sum(lens), 256) != 128
+    assert [rows(len(lens), m, n, n, mode, sum(lens), 256) for mode in (0, 1, 2)] == [tile] * 3
     lhs, rhs = (_fp8_bytes((sum(lens), w), gen, 0, cuda) for w in (m, n))
     s = torch.tensor(0.01, device=cuda)
     run = pkg.grouped_gemm_fp8_tensorwise_variable_k
@@ -115,6 +125,12 @@ def test_fp32_backward_walk_of_light_tiles(pkg, cuda, m, n):
     f32 = run(lhs, rhs, s, s, offs, out=torch.full((len(lens), m, n), float("nan"), device=cuda),
               out_dtype=torch.float32)
     assert torch.equal(f32.bfloat16().view(torch.int16), bf16.view(torch.int16))
+    for g in (lens.index(max(lens)), lens.index(900), lens.index(31), lens.index(0)):
+        lo, hi = int(offs[g]), int(offs[g + 1])
+        l, r = lhs[lo:hi, :192].cpu().numpy(), rhs[lo:hi, n - 208:].cpu().numpy()
+        got = f32[g:g + 1, :192, n - 208:].double().cpu().numpy()
+        bad, _ = vark_oracle.mfma_bound_violations(got, l, r, [0, hi - lo], 0.01, 0.01, out_rounding=0.0)
+        assert not bad.any()
     c0 = torch.randn_like(f32)
     acc = c0.clone()
     run(lhs, rhs, s, s, offs, out=acc, accumulate=True)
@@ -188,6 +204,26 @@ def test_wgrad_empty_groups_do_not_see_the_scales(pkg, cuda, mode):
         for g in (0, 2):
             assert bool((c[g] == 0).all()) and bool(torch.signbit(c[g]).all()) == (mode == "accumulate")
         assert not bool(torch.isfinite(c[1]).any()) and not bool(torch.isfinite(c[3]).any())
+
+
+@pytest.mark.parametrize("offs", [[0, 100, 300], [0, 0], [0, 700], [0, 100, 2000], [0, 90, -5]], ids=str)
+def test_clear_tail_entry_equals_zero_tail(pkg, cuda, offs):
+    """ggemm_persistent_clear_tail, for C callers with a GEMM launch of their own: the rows that zero_tail
+    clears, of rows longer than N in a buffer with more rows, and no others."""
+    N, K, M, G = 208, 272, 700, len(offs) - 1
+    gen = torch.Generator().manual_seed(2)
+    s, at = torch.tensor(0.01, device=cuda), torch.tensor(offs, device=cuda)
+    a = _fp8_bytes((M, K), gen, 0, cuda).view(torch.float8_e4m3fn)
+    b = _fp8_bytes((G, N, K), gen, 0, cuda).view(torch.float8_e4m3fn)
+    buf = torch.full((2, M + 64, N + 16), 7.0, dtype=torch.bfloat16, device=cuda)
+    for z in (0, 1):
+        pkg.grouped_gemm_fp8_tensorwise(a, b, s, s, at, out=buf[z, :M, :N], zero_tail=bool(z))
+    assert pkg.load_library().ggemm_persistent_clear_tail(
+        buf[0].data_ptr(), N, N + 16, at.data_ptr(), G, M, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(buf[0].view(torch.int16), buf[1].view(torch.int16))
+    rows = min(max(offs[-1], 0), M)
+    assert bool((buf[0, rows:M, :N] == 0).all()) and bool((buf[0, M:] == 7).all()) and bool((buf[0, :, N:] == 7).all())
 
 
 @pytest.mark.parametrize("N,K,kernel", [(208, 272, "auto"), (2048, 528, "auto"), (208, 272, "512"), (640, 128, "wide")])

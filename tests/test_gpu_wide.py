@@ -312,7 +312,7 @@ def test_wide_mx_full_size(pkg, orc, cuda):
 
 STRIDE_CASES = [
     # (OUT_M, OUT_N, extra columns per C row, kernel the library picks)
-    (1280, 1920, 8, "wide320"), (1280, 1920, 4, "192-row"), (1024, 768, 8, "wide256"), (1024, 768, 4, "192-row"),
+    (1280, 2880, 8, "wide320"), (1280, 1920, 4, "192-row"), (1440, 2688, 8, "wide256"), (1024, 768, 4, "192-row"),
 ]
 
 
@@ -325,6 +325,8 @@ def test_strided_c_rows_bf16(pkg, orc, cuda, om, on, pad, kernel):
     lens = [300, 0, 517, 64]
     _say(f"strided bf16 C {om}x{on} pad {pad}: {kernel}")
     assert pkg.bf16_kernel(om, on, on + pad) == kernel
+    rows = {"wide320": 320, "wide256": 256, "192-row": 192}[kernel]
+    assert pkg.load_library().ggemm_vark_tile_rows(len(lens), om, on, on + pad, 0, sum(lens), 256) == rows
     lhs, rhs, offs, _, (sl, sr) = _rand_bytes_problem(lens, om, on, seed=om + pad)
     big = torch.full((len(lens), om, on + pad), 7.0, dtype=torch.bfloat16, device=cuda)
     out = pkg.grouped_gemm_fp8_tensorwise_variable_k(lhs.to(cuda), rhs.to(cuda), torch.tensor(sl, device=cuda),
@@ -340,8 +342,9 @@ def test_strided_c_rows_bf16(pkg, orc, cuda, om, on, pad, kernel):
 def test_strided_c_rows_fp32_accumulate(pkg, cuda, pad):
     """fp32 accumulate into C rows padded by `pad` floats (16-byte rows: the 320 x 320 kernel): C
     equals C0 + the contiguous fp32 result bit for bit, padding columns untouched."""
-    lens, om, on = [300, 0, 517, 64], 1280, 1920
+    lens, om, on = [300, 0, 517, 64], 1920, 2880
     _say(f"strided fp32-accumulate C pad {pad}")
+    assert pkg.load_library().ggemm_vark_tile_rows(len(lens), om, on, on + pad, 2, sum(lens), 256) == 320
     lhs, rhs, offs, _, (sl, sr) = _rand_bytes_problem(lens, om, on, seed=pad + 1)
     dl, dr, do = lhs.to(cuda), rhs.to(cuda), offs.to(cuda)
     s1, s2 = torch.tensor(sl, device=cuda), torch.tensor(sr, device=cuda)

@@ -63,3 +63,32 @@ def test_slice_bounds_also_of_one_tile():
     for w_slot, tpg in small + [([rng.randint(1, 99) for _ in range(rng.randint(1, 40))], rng.randint(1, 50))
                                 for _ in range(200)]:
         assert _bounds(w_slot, tpg) == _first_tiles(w_slot, tpg), (w_slot, tpg)
+
+
+def walks_backwards(lens, tiles_of_group, stage, epi_w, light, num_wg=256):
+    """Whether the odd XCDs of an fp32 launch walk back: the rounds deal is strictly the lighter one and the
+    stages that the tiles' C stores are worth (``light`` each) are a quarter of the work or more.
+    ``tiles_of_group`` tiles in every group, ``stage`` tokens a stage."""
+    w = sorted((-(-n // stage) + epi_w for n in lens), reverse=True)
+    tpg, total = tiles_of_group, len(lens) * tiles_of_group
+    bounds, wpx = _bounds(w, tpg), num_wg // 8
+
+    def heaviest(walk):
+        return max(sum(w[t // tpg] for t in walk(wg)) for wg in range(num_wg))
+
+    def slices(wg):
+        xcd = wg % 8
+        return range(bounds[xcd % 4] + xcd // 4 * wpx + wg // 8, bounds[xcd % 4 + 1], 2 * wpx)
+
+    rounds = heaviest(lambda wg: _forward(wg % 8 * wpx + wg // 8, num_wg, total))
+    return rounds < heaviest(slices) and 4 * sum(max(0, light + epi_w - x) for x in w) >= sum(w) and total > num_wg
+
+
+def test_the_full_size_lengths_walk_as_measured():
+    """Zipf lengths of 16384 tokens walk back on the 320 x 320 tiles of [32, 2880, 5760] in both fp32 modes,
+    even lengths of 131072 do not."""
+    raw = [1 / (i + 1) ** 1.2 for i in range(24)]
+    zipf = [int(16384 * r / sum(raw)) for r in raw] + [0] * 8
+    for light in (16, 32):
+        assert walks_backwards(zipf, 162, 64, 3, light)
+        assert not walks_backwards([4096] * 32, 162, 64, 3, light)
