@@ -432,6 +432,15 @@ __device__ __forceinline__ int64_t clamp_off(int64_t o, int64_t m_total) {
   return o < 0 ? 0 : (o > m_total ? m_total : o);
 }
 
+// Spreads the starts of the 32 workgroups of every XCD over some `us` microseconds, in sleeps of 64 cycles.
+// Workgroups that start as one stay in step: all of them multiply, then all of them store C. Those of the
+// library's kernels do since they no longer wait for the dispatch packet, up to 14 us one after the other;
+// launches of several short tiles a workgroup, bound by their C, got slower for it (rules and figures at the
+// callers). The drop-in code object's still wait for it.
+__device__ __forceinline__ void stagger(int us) {
+  for (int n = (int)blockIdx.x / kXcds % 32 * us; n > 0; --n) __builtin_amdgcn_s_sleep(1);
+}
+
 struct Tile {
   int g, m0, n0, nsteps;
   int64_t kb, klen;
@@ -603,6 +612,7 @@ __device__ __forceinline__ Sched make_sched(const VarKArgs& a, GG_LDS int* s_ord
   const int wgs_per_xcd = spread ? num_wg / kXcds : num_wg;
   const int tpg = S.tiles_per_group;
   const bool choose = S.sorted && spread;
+  float mean_w = 0;                           // a tile's work
   if (choose) {
     // bounds of the slices: slice x starts at the first tile whose preceding work reaches x / 4 of
     // all; the slots' work summed over the threads (kPer slots each), waves and workgroup
@@ -649,6 +659,7 @@ __device__ __forceinline__ Sched make_sched(const VarKArgs& a, GG_LDS int* s_ord
       before = after;
     }
     if (tid == 0) s_bound[kXcdPairs] = total;
+    mean_w = (float)total_w / (float)total;
   } else if (tid == 0) {
     for (int x = 0; x <= kXcdPairs; ++x) s_bound[x] = spread ? total * x / kXcdPairs : (x ? total : 0);
   }
@@ -714,6 +725,17 @@ __device__ __forceinline__ Sched make_sched(const VarKArgs& a, GG_LDS int* s_ord
     }
   }
   if (choose) __syncthreads();   // s_w and s_pred alias the first stage's scale region
+  // 320 x 320 tiles, several a workgroup, of few stages (128 tokens; more where C is fp32): starts spread over
+  // a tile's time, its C at the memory's rate included, 16 us at most. Measured (us, all starting as one ->
+  // spread): bf16 [6, 5760, 5760] of 1165 tokens 99.5 -> 90.0, MX [16, 5760, 5760] of 3168 238 -> 217, fp32
+  // [34, 2880, 2880] of 33491 340 -> 306; of 241 drawn launches of this kind 16 were more than 3 % slower than
+  // when they waited for the packet, 2 still are, at 1.02 times the speed of all starting as one in the mean (the
+  // worst 0.95). Of more stages, and on the other tiles, spread or not is the same in the mean.
+  if constexpr (kTM == 320) {
+    const float stages = (mean_w - kEpiW) * (kK / 128.0f);
+    if (a.num_wg > 0 && total >= 3 * num_wg && stages >= 1.0f && stages <= (kLight > 0 ? 17.0f : 4.0f))
+      stagger(__builtin_amdgcn_readfirstlane((int)fminf(16.0f, 7.5f + 1.65f * stages)));
+  }
   S.t_first = D.t_first;
   S.t_end = D.t_end;
   S.d0 = D.d0;

@@ -56,3 +56,41 @@ def test_offsets_past_token_count_are_clamped(pkg, orc, cuda, kind, on):
         ref = orc.vark_wgrad_tensorwise(lhs.numpy(), rhs.numpy(), sl, sr, clamped.numpy())
         parity._assert_parity(orc, pkg.as_bf16_bits(out), ref, clamped.numpy(), "192-row clamp/bf16")
     assert bool((out[1] == 0).all()) and bool((out[4:] == 0).all())
+
+
+def test_gemm_of_spread_starts(pkg, cuda):
+    """Three tiles a workgroup, C rows off the 128-byte lines: the workgroups start one after the other. The
+    same rows with C on the lines, where they start as one, have the same bits."""
+    G, N, K, s = 3, 16, 512, torch.tensor(0.01, device=cuda)
+    M = 768 * 192 + 5
+    gen = torch.Generator().manual_seed(4)
+    a = torch.randn((M, K), generator=gen).to(torch.float8_e4m3fn).to(cuda)
+    b = torch.randn((G, N, K), generator=gen).to(torch.float8_e4m3fn).to(cuda)
+    offs = torch.tensor([0, 700, 701, M], device=cuda)
+    outs = [torch.full((M, stride), 7.0, dtype=torch.bfloat16, device=cuda)[:, :N] for stride in (24, 64)]
+    for out in outs:
+        pkg.grouped_gemm_fp8_tensorwise(a, b, s, s, offs, out=out, kernel="512")
+    assert torch.equal(*(o.contiguous().view(torch.int16) for o in outs))
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_wgrad_of_spread_starts(pkg, orc, cuda, mode):
+    """Three 320 x 320 tiles a workgroup and one to four stages each, the workgroups started one after the
+    other: two groups against the exact result's bound."""
+    lens, m, n = [300, 1, 0, 517] * 12, 1280, 1280
+    assert pkg.load_library().ggemm_vark_tile_rows(len(lens), m, n, n, mode, sum(lens), 256) == 320
+    assert len(lens) * 16 >= 3 * 256 and 1 <= sum(-(-v // 64) for v in lens) / len(lens) / 2 <= 4
+    gen = torch.Generator().manual_seed(mode)
+    lhs, rhs = ((torch.randint(0, 256, (sum(lens), w), generator=gen).to(torch.uint8) & 0xbb) for w in (m, n))
+    offs, s = torch.tensor([0] + lens).cumsum(0), torch.tensor(0.01, device=cuda)
+    dt = torch.float32 if mode else torch.bfloat16
+    c0 = torch.zeros((len(lens), m, n), dtype=dt, device=cuda) if mode == 2 else None
+    c = pkg.grouped_gemm_fp8_tensorwise_variable_k(lhs.to(cuda), rhs.to(cuda), s, s, offs.to(cuda), out=c0,
+                                                   out_dtype=dt, accumulate=mode == 2)
+    for g in (1, 47):
+        lo, hi = int(offs[g]), int(offs[g + 1])
+        bad, _ = orc.mfma_bound_violations(c[g:g + 1, -160:, :176].double().cpu().numpy(), lhs[lo:hi, m - 160:].numpy(),
+                                           rhs[lo:hi, :176].numpy(), [0, hi - lo], 0.01, 0.01,
+                                           out_rounding=0.0 if mode else 2.0 ** -8)
+        assert not bad.any()
+    assert bool((c[2::4] == 0).all())
