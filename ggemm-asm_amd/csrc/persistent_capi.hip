@@ -130,14 +130,13 @@ int64_t mid_tiles(int rows, int G, int N, int64_t M_total) {
   return (M_total / rows + (G < M_total ? G : M_total)) * ((N + 127) / 128);
 }
 
-// The second look at a launch that the estimate of mid_preferred gives to 128-row tiles: both sides in whole
-// rounds, for rows spread evenly over the groups and for any (half a row tile more for each group), and the
-// mean of the two. 569 of 6112 drawn launches for the mid tiles (1 to 64 groups, 1 to 60000 rows, features 64
-// to 5760, even, exponential and Zipf lengths) were given 128 rows, 51 of them more than 3 % slower than the
-// large tiles and 31 more than 10 %: 13 groups, 5788 rows, N = K = 2880 75 us, 51 on the wide tiles; 15, 7007,
-// N = 2560, K = 5760 112, 85. Of the 702 in another draw 21 were slower than before there were mid tiles, 10 by more
-// than 10 %; with this rule 10 and 2 are, and 12 lose a gain of 20 % or more (14
-// and 6 of the 851 that it leaves of a third draw).
+// The second look at a launch of more than four groups that the estimate of mid_preferred gives to 128-row
+// tiles: both sides in whole rounds, for rows spread evenly over the groups and for any (half a row tile more
+// for each group), and the mean of the two. Of 1553 drawn launches on 128 rows (1 to 64 groups, 1 to 60000 rows,
+// features 64 to 5760, even, exponential and Zipf lengths) 35 were more than 3 % slower than before there were mid
+// tiles, 16 more than 10 %: 13 groups, 5788 rows, N = K = 2880 75 us, 51 on the wide tiles; 15, 7007, N = 2560, K
+// = 5760 112, 85. With this rule 27 and 9 are, and 7 lose a gain of 20 % or more. For up to four groups it lost
+// as often as it gained.
 bool rows128_faster(int N, double M, double g, double stages, double mem, bool wide, int cus) {
   constexpr int kRun = ggemm::mid::kXcdRun;
   const int tn = wide ? 320 : ggemm::wide_tiles(N, false) ? 384 : 320;
@@ -188,7 +187,7 @@ int mid_preferred(int G, int N, int K, int scm, int64_t M_total, bool wide, int 
   const double c128 = 4 + std::max(1.0, f128) * stages * (0.64 + 0.42 * std::min(1.0, f128)) + 0.3 * mem;
   if (std::min(c64, c128) >= 0.92 * big) return 0;   // near the line the estimate is a few per cent off
   if (c64 < 0.97 * c128) return 64;
-  return rows128_faster(N, M, g, (K + 127) / 128, mem, wide, cus) ? 128 : 0;
+  return g <= 4 || rows128_faster(N, M, g, (K + 127) / 128, mem, wide, cus) ? 128 : 0;
 }
 
 int launch(const void* a, const void* b, void* out, const float* a_scale, const float* b_scale,

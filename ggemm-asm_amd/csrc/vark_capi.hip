@@ -86,17 +86,18 @@ int64_t mid_tiles(int G, int OUT_M, int OUT_N) {
          ((OUT_N + ggemm::mid::kWT - 1) / ggemm::mid::kWT);
 }
 
-// The second look at a launch that the estimate of mid_preferred gives to the mid tiles: with tiles of equal
-// lengths both sides run in whole rounds, which that estimate, made for the tails of many unlike tiles, spreads
-// out, and the larger tiles' rates and fixed costs are those of launches without the read of the dispatch
-// packet. Mid tiles: 1.15 of a tile's time a round of two to a CU, 0.8 the last one with one to a CU, on the
-// XCD that takes most of them (tile_of_block); 192-row ones: 1.62, and 1.1 to 1.6 for a last round; wide 1.67.
-// Over 3800 drawn launches that went to the mid tiles (1 to 64 groups, 1 to 131072 tokens, features 64 to
-// 5760, even, exponential and Zipf lengths) 102 were more than 3 % slower than before there were mid tiles, 58
-// more than 10 %: [1, 2880, 2880] of 100930 tokens 1843 us, 1403 on the large tiles; [5, 2544, 1744] of 17692
-// 122, 94; [2, 2880, 3312] of 106369 1574, 1122. With this rule 20 and 7 are (34 and 15 of the 3847 that it
-// leaves of another draw); 56 lose a gain of 20 % or more (lengths so unlike that the longest group alone
-// counts).
+// The second look at a launch that the estimate of mid_preferred gives to the mid tiles, where both features
+// are over 1280: with tiles of equal lengths both sides run in whole rounds, which that estimate, made for the
+// tails of many unlike tiles, spreads out, and the larger tiles' rates and fixed costs are those of launches
+// without the read of the dispatch packet. Mid tiles: 1.15 of a tile's time a round of two to a CU, 0.8 the last
+// one with one to a CU, on the XCD that takes most of them (tile_of_block); 192-row ones: 1.62, and 1.1 to 1.6
+// for a last round; wide 1.67. Of 7661 drawn launches for the mid tiles (1 to 64 groups, 1 to 131072 tokens,
+// features 64 to 5760, even, exponential and Zipf lengths) 136 were more than 3 % slower than before there were
+// mid tiles, 73 more than 10 %: [1, 2880, 2880] of 100930 tokens 1843 us, 1403 on the large tiles; [5, 2544,
+// 1744] of 17692 122, 94; [2, 2880, 3312] of 106369 1574, 1122. With this rule 78 and 35 are, and 4 lose a gain
+// of 20 % or more. Narrower outputs stay with the mid tiles: of those that the same line would take back the even
+// lengths are slower on them (0.90 in the median), the unlike ones, whose longest group alone counts, faster
+// (1.2).
 bool whole_rounds_faster(int G, int OUT_M, int OUT_N, bool f32, double stages, int wide_tile, int cus) {
   constexpr int kRun = ggemm::mid::kXcdRun;
   const int64_t t = mid_tiles(G, OUT_M, OUT_N), all = ggemm::kXcds * kRun;
@@ -148,7 +149,7 @@ bool mid_preferred(int G, int OUT_M, int OUT_N, int64_t scm, int64_t scg, const 
     big = 7 + std::ceil(t) * (stages + 3) * (1.2 + 0.9 * std::min(1.0, t));
   }
   if (mid >= 0.92 * big) return false;                       // near the line the estimate is a few per cent off
-  return whole_rounds_faster(G, OUT_M, OUT_N, f32, stages, wide_tile, cus);
+  return std::min(OUT_M, OUT_N) <= 1280 || whole_rounds_faster(G, OUT_M, OUT_N, f32, stages, wide_tile, cus);
 }
 
 // swapped: e5m2 LHS, e4m3 RHS (bf16 C only)

@@ -72,7 +72,7 @@ def test_gemm_workgroups_cover_the_tiles_of_any_offsets():
 @pytest.mark.parametrize("G,m,n,M,mode,rows", [
     (1, 2880, 2880, 100930, 0, 320), (1, 2880, 2880, 100930, 2, 320), (2, 2880, 3312, 106369, 0, 192),
     (5, 2544, 1744, 17692, 0, 192), (1, 1984, 5760, 114333, 0, 256),
-    (8, 512, 1024, 1000, 0, 128), (2, 1024, 2048, 8000, 0, 128), (12, 1600, 1600, 1000, 1, 128),   # still mid
+    (14, 2880, 144, 80476, 2, 128), (8, 512, 1024, 1000, 0, 128), (2, 1024, 2048, 8000, 0, 128), (12, 1600, 1600, 1000, 1, 128),   # still mid
 ])
 def test_wgrad_of_whole_rounds(pkg, G, m, n, M, mode, rows):
     """Launches on which the mid tiles measured slower than the large ones, next to some they serve."""
@@ -80,7 +80,7 @@ def test_wgrad_of_whole_rounds(pkg, G, m, n, M, mode, rows):
 
 
 @pytest.mark.parametrize("G,N,K,M,rows", [
-    (13, 2880, 2880, 5788, 256), (15, 2560, 5760, 7007, 256), (2, 2320, 2880, 3715, 192),
+    (13, 2880, 2880, 5788, 256), (15, 2560, 5760, 7007, 256), (2, 2320, 2880, 3715, 128),
     (4, 2880, 2880, 8192, 128), (8, 512, 1024, 100000, 128), (32, 5760, 2880, 3072, 128), (32, 5760, 2880, 256, 64),
 ])
 def test_gemm_of_whole_rounds(pkg, G, N, K, M, rows):
