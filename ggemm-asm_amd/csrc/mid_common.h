@@ -26,7 +26,10 @@ __device__ __forceinline__ int tile_of_block(int b) {
 }
 
 // Four groups per lane: lane l of every wave holds groups 4 l .. 4 l + 3. Their offsets clamped to
-// [0, m_total]; each wave reads them for itself, so no barrier and no LDS is needed.
+// [0, m_total]; each wave reads them for itself, so no barrier and no LDS is needed. Where offsets decrease and
+// rise again, rows belong to the first group that holds them: the groups then have no more rows in all than
+// there are, nor more tiles than the launch has workgroups, and every row that a group holds is written (the
+// offsets begin with zero, so the rows up to the largest one so far are all held).
 struct Groups {
   int start[4], len[4];             // first row and row count (0 for g >= G and for decreasing offsets)
 };
@@ -41,11 +44,30 @@ __device__ __forceinline__ Groups load_groups(const int64_t* offs, int G, int64_
   }
   *any_negative = __ballot(neg) != 0;
   Groups r;
+  int end[4];
+  bool falls = false;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const int64_t lo = clamp_off(o[k], m_total), hi = clamp_off(o[k + 1], m_total);
-    r.start[k] = (int)lo;
-    r.len[k] = hi > lo ? (int)(hi - lo) : 0;
+    r.start[k] = (int)clamp_off(o[k], m_total);
+    end[k] = (int)clamp_off(o[k + 1], m_total);
+    r.len[k] = max(end[k] - r.start[k], 0);
+    falls |= end[k] < r.start[k];
+  }
+  if (__ballot(falls) != 0) {
+    int past = max(max(end[0], end[1]), max(end[2], end[3]));   // end of the rows held up to here
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int v = __shfl_up(past, d, 64);
+      if (lane >= d) past = max(past, v);
+    }
+    past = __shfl_up(past, 1, 64);
+    if (lane == 0) past = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      r.start[k] = max(r.start[k], past);
+      r.len[k] = max(end[k] - r.start[k], 0);
+      past = max(past, end[k]);
+    }
   }
   return r;
 }

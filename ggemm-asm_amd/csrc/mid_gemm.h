@@ -35,18 +35,29 @@ struct GemmCfg {
   static constexpr int BandN = 8;                            // column tiles of a band, rows tiles walked inside
 };
 
-// Tile t of the launch: before = tiles ahead of this lane's groups, cnt = theirs, holders = the lanes whose
-// groups end past tile t (not zero).
 template <bool kAE5M2, int kBM>
-__device__ __forceinline__ void gemm_tile(const nt::Args& a, GG_LDS uint8_t* lds, const Groups& gr, const int (&cnt)[4],
-                                          int before, uint64_t holders, int t) {
+__device__ __forceinline__ void gemm_body(const nt::Args& a, GG_LDS uint8_t* lds) {
   using C = GemmCfg<kBM>;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n_tn = (a.N + C::BN - 1) / C::BN;
 
-  const int gl = __builtin_ctzll(holders);
-  int in_g = t - __builtin_amdgcn_readlane(before, gl), gx = 0;
+  // ---- this workgroup's tile: groups hold ceil(len / BM) n_tn consecutive tiles each
+  const int t = tile_of_block(blockIdx.x);
+  bool negative;
+  const Groups gr = load_groups(a.group_offs, a.G, a.m_total, lane, &negative);
+  if (negative) return;                                      // as the persistent kernels: nothing is written
+  int cnt[4], sum = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    cnt[k] = (gr.len[k] + kBM - 1) / kBM * n_tn;
+    sum += cnt[k];
+  }
+  const int incl = wave_scan(sum, lane);
+  const uint64_t past = __ballot(incl > t);
+  if (past == 0) return;                                     // more workgroups than tiles
+  const int gl = __builtin_ctzll(past);
+  int in_g = t - __builtin_amdgcn_readlane(incl - sum, gl), gx = 0;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const int c = __builtin_amdgcn_readlane(cnt[k], gl);
@@ -138,37 +149,6 @@ __device__ __forceinline__ void gemm_tile(const nt::Args& a, GG_LDS uint8_t* lds
   store_bf16<C::NB>(acc, alpha, lds + cur * C::Slot + wave * (64 * 2 * kCols),
                     a.c + (int64_t)(row_base + m0 + 64 * wm) * a.stride_cm + n0 + kCols * wn, a.stride_cm,
                     rows - 64 * wm, cols - kCols * wn, lane);
-}
-
-// This workgroup's tile: groups hold ceil(len / BM) n_tn consecutive ones each. Offsets that decrease and
-// rise again give rows to several groups, whose tiles can outnumber the grid's workgroups (a multiple of
-// tile_of_block's runs): such a launch walks them in a loop of its own. The second path costs the others
-// 0.3 us of 94.5 (32 x 8 rows x 5760 x 2880), the loop as the only one 0.5.
-template <bool kAE5M2, int kBM>
-__device__ __forceinline__ void gemm_body(const nt::Args& a, GG_LDS uint8_t* lds) {
-  const int lane = threadIdx.x & 63, n_tn = (a.N + GemmCfg<kBM>::BN - 1) / GemmCfg<kBM>::BN;
-  bool negative;
-  const Groups gr = load_groups(a.group_offs, a.G, a.m_total, lane, &negative);
-  if (negative) return;                                      // as the persistent kernels: nothing is written
-  int cnt[4], sum = 0;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    cnt[k] = (gr.len[k] + kBM - 1) / kBM * n_tn;
-    sum += cnt[k];
-  }
-  const int incl = wave_scan(sum, lane);
-  int t = tile_of_block(blockIdx.x);
-  uint64_t holders = __ballot(incl > t);
-  if (__builtin_amdgcn_readlane(incl, 63) <= (int)gridDim.x) {
-    if (holders != 0) gemm_tile<kAE5M2, kBM>(a, lds, gr, cnt, incl - sum, holders, t);
-    return;
-  }
-  while (holders != 0) {
-    gemm_tile<kAE5M2, kBM>(a, lds, gr, cnt, incl - sum, holders, t);
-    lds_barrier();                                           // the waves' epilogues have read the slots
-    t += gridDim.x;
-    holders = __ballot(incl > t);
-  }
 }
 
 }  // namespace mid

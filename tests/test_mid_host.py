@@ -45,28 +45,29 @@ def test_wgrad_unaligned_rows_of_c_keep_the_192_row_kernel(pkg):
     assert rows(4, 64, 128, 132, 1, 512, 256) == 128
 
 
-def test_gemm_workgroups_cover_the_tiles_of_any_offsets():
-    """Model of the mid-tile GEMM's grid (capi) and walk (gemm_body): every tile is taken by one workgroup,
-    also where offsets decrease and rise again and the groups' tiles outnumber the workgroups."""
+def test_gemm_workgroups_cover_the_rows_of_any_offsets():
+    """Model of the mid-tile GEMM's rows (load_groups) and grid (capi): every row that a group holds is taken
+    once, by the first group that holds it, and the tiles are no more than the workgroups, also where offsets
+    decrease and rise again (from the first on, which is zero)."""
     rng = random.Random(0)
     for rows in (64, 128):
         for _ in range(300):
             G, M, n_tn = rng.randint(1, 256), rng.randint(1, 3000), rng.randint(1, 9)
-            offs = [rng.randint(0, M) for _ in range(G + 1)]
+            offs = [0] + [rng.randint(0, M) for _ in range(G)]
             if rng.random() < 0.5:
                 offs.sort()
-            bound = (M // rows + min(G, M)) * n_tn
-            grid = -(-bound // 256) * 256
-            total = sum(-(-max(b - a, 0) // rows) * n_tn for a, b in zip(offs, offs[1:]))
-            assert offs != sorted(offs) or total <= grid
-            taken = []
-            for b in range(grid):
-                r = b % 256
-                t = b - r + (r % 8) * 32 + r // 8
-                while t < total:
-                    taken.append(t)
-                    t += grid
-            assert sorted(taken) == list(range(total))
+            grid = -(-(M // rows + min(G, M)) * n_tn // 256) * 256
+            held, taken, tiles, past = set(), [], 0, 0
+            for a, b in zip(offs, offs[1:]):
+                held |= set(range(a, b))
+                start = max(a, past)
+                taken += range(start, b)
+                assert offs != sorted(offs) or start == a
+                tiles += -(-max(b - start, 0) // rows) * n_tn
+                past = max(past, b)
+            assert len(taken) == len(set(taken)) and set(taken) == held and tiles <= grid
+            order = [b - b % 256 + b % 8 * 32 + b % 256 // 8 for b in range(grid)]
+            assert sorted(order) == list(range(grid))
 
 
 @pytest.mark.parametrize("G,m,n,M,mode,rows", [
