@@ -50,12 +50,6 @@ def _check_inputs(lhs, rhs, group_offs, lhs_dt=_FP8_LHS, rhs_dt=_FP8_RHS):
                          f"{dev}); use the CPU oracle in tests for reference results")
 
 
-def _check_scales(lhs_scale, rhs_scale, dev):
-    for s in (lhs_scale, rhs_scale):
-        if s.dtype != torch.float32 or s.numel() != 1 or s.device != dev:
-            raise ValueError("scales must be single-element fp32 tensors on the input device")
-
-
 def _check_out(out, G, OUT_M, OUT_N, dev, dtype=torch.bfloat16):
     if out is None:
         return torch.empty((G, OUT_M, OUT_N), dtype=dtype, device=dev)
@@ -99,7 +93,9 @@ def grouped_gemm_fp8_tensorwise_variable_k(lhs: torch.Tensor, rhs: torch.Tensor,
     library picks (a wide tile for OUT_M >= 1024 where one fits).
     """
     _check_inputs(lhs, rhs, group_offs)
-    _check_scales(lhs_scale, rhs_scale, lhs.device)
+    for s in (lhs_scale, rhs_scale):
+        if s.dtype != torch.float32 or s.numel() != 1 or s.device != lhs.device:
+            raise ValueError("scales must be single-element fp32 tensors on the input device")
     G = group_offs.numel() - 1
     M_total, OUT_M = lhs.shape
     OUT_N = rhs.shape[1]
@@ -143,7 +139,9 @@ def weight_grad_fp8(dy: torch.Tensor, x: torch.Tensor, dy_scale: torch.Tensor, x
     the weight gradient in the weight's own orientation. dy: float8_e5m2 [M_total, N]; x:
     float8_e4m3fn [M_total, K]; scales: fp32 scalar tensors on the device."""
     _check_inputs(dy, x, group_offs, (torch.float8_e5m2,), (torch.float8_e4m3fn,))
-    _check_scales(dy_scale, x_scale, dy.device)
+    for s in (dy_scale, x_scale):
+        if s.dtype != torch.float32 or s.numel() != 1 or s.device != dy.device:
+            raise ValueError("scales must be single-element fp32 tensors on the input device")
     G = group_offs.numel() - 1
     M_total, N = dy.shape
     out = torch.empty((G, N, x.shape[1]), dtype=torch.bfloat16, device=dy.device)
