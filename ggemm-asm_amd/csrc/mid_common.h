@@ -1,6 +1,6 @@
 // What the two mid-tile kernels share (mid_gemm.h, mid_wgrad.h): one output tile per 256-thread
 // workgroup, several workgroups per CU, no persistent schedule. The wide and the 512-thread kernels
-// hold one tile of 200-300 KB of accumulators on each CU for as long as it takes; problems of fewer
+// hold one tile of 240-400 KiB of accumulators on each CU for as long as it takes; problems of fewer
 // such tiles than CUs, of short groups or of small feature sizes leave most of that idle. Here the
 // tiles are a quarter of that size or less, the hardware hands them out as workgroups finish, and
 // the other workgroups of a CU compute while one waits for its loads, starts or stores its results.

@@ -101,8 +101,8 @@ __device__ __forceinline__ void vark_wide_body(const VarKArgs& a, GG_LDS uint8_t
   GG_LDS uint8_t* misc = lds + (MX ? kMiscOffMX : kMiscOff);
   GG_LDS int* s_order = (GG_LDS int*)misc;
   GG_LDS int* s_kb = (GG_LDS int*)(misc + kKbOffset);
-  const Sched S = make_sched<TN, kKS, kEpiW, TM, kNT, OUT == kOutBF16 ? 0 : OUT == kOutF32 ? 16 : 32>(a, s_order, s_kb, (GG_LDS int*)(misc + kFlagOffset),
-                                                        (GG_LDS int64_t*)(misc + kBoundOffset));
+  const Sched S = make_sched<TN, kKS, kEpiW, TM, kNT, OUT == kOutBF16 ? 0 : OUT == kOutF32 ? 16 : 32>(
+      a, s_order, s_kb, (GG_LDS int*)(misc + kFlagOffset), (GG_LDS int64_t*)(misc + kBoundOffset));
   if (!S.valid) {
     poison_c<OUT>(a);
     return;

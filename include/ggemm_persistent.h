@@ -41,8 +41,8 @@ extern "C" {
  * M_total (rows of a and out) is not part of the reference kernarg; it bounds the 32-bit row and
  * tile indices here (M_total < 2^31 - 256, at most 2^30 output tiles of 192 x 320), and the
  * kernel clamps every group offset to M_total on the device, so offsets past it read and write no
- * row outside a and out (group g covers rows [min(offs[g], M_total), min(offs[g+1], M_total)));
- * a negative or decreasing offset array writes nothing.
+ * row outside a and out (group g covers rows [min(offs[g], M_total), min(offs[g+1], M_total)),
+ * none where that ends before it starts); with a negative offset nothing is written.
  * Requirements: 1 <= G <= GGEMM_PERSISTENT_MAX_GROUPS; N, K > 0 and multiples of 16; row strides
  * >= K and multiples of 16, stride_bg >= (N-1)*stride_bn + K and a multiple of 16, stride_cm >= N
  * and a multiple of 8; 192*stride_am and 384*stride_bn below 2^31 - 2^16; a, b, out 16-byte
@@ -53,7 +53,8 @@ int ggemm_persistent_fp8(const void* a, const void* b, void* out, const float* a
                          int32_t a_format, int64_t M_total, void* stream);
 
 /* Kernels behind ggemm_persistent_fp8 (same semantics; each deterministic, the two differ in
- * fp32 summation order): the 512-thread kernel of the reference's launch geometry (192-row tiles,
+ * fp32 summation order, so that a row's last bit can depend on G and M_total where the choice is
+ * automatic; a kernel chosen by code gives a row the same bits in any launch): the 512-thread kernel of the reference's launch geometry (192-row tiles,
  * also the drop-in code objects) and a wide-tile kernel (256 threads, one wave per SIMD, 256 x 320
  * tiles, 160 KiB of LDS) for N % 320 == 0, K % 64 == 0, 256*stride_am, 320*stride_bn and
  * 512*stride_cm below 2^31 - 2^16. ggemm_persistent_fp8 runs the wide kernel wherever it applies
@@ -63,12 +64,14 @@ int ggemm_persistent_fp8(const void* a, const void* b, void* out, const float* a
 #define GGEMM_PERSISTENT_KERNEL_512 1
 #define GGEMM_PERSISTENT_KERNEL_WIDE 2
 /* added to a kernel code: rows [min(offs[G], M_total), M_total) of out become zero in the same launch
- * (as by ggemm_persistent_clear_tail after it; ABI version 10) */
+ * (as by ggemm_persistent_clear_tail after it, also where an earlier group ends past offs[G]; ABI
+ * version 10) */
 #define GGEMM_PERSISTENT_ZERO_TAIL 0x100
 
 /* ggemm_persistent_fp8 with the kernel chosen by the caller: GGEMM_PERSISTENT_KERNEL_AUTO (as
  * ggemm_persistent_fp8), _512 or _WIDE (GGEMM_E_SHAPE where the wide kernel does not apply), plus
- * GGEMM_PERSISTENT_ZERO_TAIL. No reference counterpart (the reference ships one kernel); for comparisons of the two kernels. */
+ * GGEMM_PERSISTENT_ZERO_TAIL. No reference counterpart (the reference ships one kernel); for
+ * comparisons of the two kernels, and for rows whose bits must not depend on the launch's other rows. */
 int ggemm_persistent_fp8_kernel(const void* a, const void* b, void* out, const float* a_scale, const float* b_scale,
                                 const int64_t* group_offs, int32_t G, int32_t N, int32_t K, int32_t stride_am,
                                 int32_t stride_bg, int32_t stride_bn, int32_t stride_cm, int32_t stride_cn,
