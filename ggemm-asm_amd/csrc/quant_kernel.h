@@ -185,8 +185,10 @@ __device__ __forceinline__ void block_amax(uint32_t m, uint32_t* amax_bits) {
   if (threadIdx.x == 0 && m) atomicMax(amax_bits, m);
 }
 
-// The tensor's amax bits from the n partial maxima of an amax pass (n = 1: the finished amax).
+// The tensor's amax bits from the n partial maxima of an amax pass (n = 1: the finished amax, read as it is:
+// the loop and the barrier cost a small tensor's call 0.1 to 0.3 us).
 __device__ __forceinline__ uint32_t partials_amax(const uint32_t* partials, int n) {
+  if (n == 1) return *partials;
   uint32_t m = 0;
 #pragma unroll
   for (int k = 0; k < kMaxPartials / kThreads; ++k) {
