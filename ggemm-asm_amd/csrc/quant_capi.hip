@@ -39,8 +39,8 @@ int grid_for(int64_t chunks, int cus, int per_cu) {
   return (int)(want < 1 ? 1 : (want > cap ? cap : want));
 }
 
-// What reads x after its amax pass.
-enum class Next { kNothing, kStreaming, kTransposing };
+// What reads x after its amax pass; kTransposingOnce: the transposing pass with non-temporal loads.
+enum class Next { kNothing, kStreaming, kTransposing, kTransposingOnce };
 
 // Whether the amax pass loads x the ordinary way (load8), so that the next pass finds part of it in the
 // memory-side cache, or non-temporally, the faster way to read it once. Measured (us, non-temporal ->
@@ -49,10 +49,24 @@ enum class Next { kNothing, kStreaming, kTransposing };
 // 450 MB 247.8 -> 251.3, 1 GB 553.8 -> 565.3; bf16 alone 50 MB 24.7 -> 25.1, 1 GB 152.1 -> 163.8. fp32 takes
 // twice as long over a byte and gains at every size (33 MB 19.3 -> 15.5, 4 GB 1629 -> 1596; transposing
 // 22.6 -> 18.7, 1923 -> 1890); alone 300 MB 58.6 -> 59.3, 600 MB 104.2 -> 103.4, 4 GB 674.8 -> 647.9.
+constexpr int64_t kMB = 1000 * 1000;
+
 bool amax_keeps(int64_t bytes, bool f32, Next next) {
-  constexpr int64_t kMB = 1000 * 1000;
   if (f32) return next != Next::kNothing || bytes > 500 * kMB;
+  if (next == Next::kTransposingOnce) return true;
   return bytes <= (next == Next::kStreaming ? 1100 * kMB : next == Next::kTransposing ? 300 * kMB : 0);
+}
+
+// How the transposing pass loads x: the ordinary way, but for a bf16 x over 275 MB whose q^T rows don't start
+// on 128-byte lines, where ordinary loads and stores of part lines get in each other's way: there x is kept by
+// the amax pass (amax_keeps) and read non-temporally. Measured over shapes with such rows (speed of both passes
+// against non-temporal loads in both and a launch that zeroes the amax, mean and least; this way / ordinary
+// loads after an amax pass by amax_keeps' sizes): 250-275 MB 1.19 1.09 / 1.23 1.08, 275-350 MB 1.17 1.07 / 1.03
+// 0.92, 350-500 MB 1.11 1.04 / 1.01 0.91, 500-700 MB 1.08 1.01 / 1.00 0.92, 0.7-1 GB 1.04 0.98 / 0.98 0.92,
+// 1-1.8 GB 1.02 0.98 / 0.97 0.92; 150-250 MB 1.20 1.12 / 1.27 1.15. On whole lines the second way was never
+// below 0.99, and in fp32 ordinary loads in both passes were the faster ones.
+Next transposing(int64_t bytes, bool f32, int64_t out_t_stride) {
+  return f32 || out_t_stride % 128 == 0 || bytes <= 275 * kMB ? Next::kTransposing : Next::kTransposingOnce;
 }
 
 template <bool kPartials, bool kKeep>
@@ -261,12 +275,14 @@ static int tensorwise_transpose(const void* x, int32_t in_dtype, int32_t batch, 
   rc = device_cus(&cus);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  const int n = launch_amax(x, in_dtype, (int64_t)batch * rows, cols, cols, amax_out, workspace, Next::kTransposing,
-                            cus, s);
-  const uint32_t* partials = workspace ? workspace : reinterpret_cast<const uint32_t*>(amax_out);
   const bool f32 = in_dtype == GGEMM_IN_F32, e5 = out_format == GGEMM_FP8_E5M2;
-  auto k = f32 ? (e5 ? qt::quant_transpose_kernel<true, true> : qt::quant_transpose_kernel<true, false>)
-               : (e5 ? qt::quant_transpose_kernel<false, true> : qt::quant_transpose_kernel<false, false>);
+  const Next next = transposing((int64_t)batch * rows * cols * (f32 ? 4 : 2), f32, out_t_stride);
+  const int n = launch_amax(x, in_dtype, (int64_t)batch * rows, cols, cols, amax_out, workspace, next, cus, s);
+  const uint32_t* partials = workspace ? workspace : reinterpret_cast<const uint32_t*>(amax_out);
+  auto k = f32 ? (e5 ? qt::quant_transpose_kernel<true, true, true> : qt::quant_transpose_kernel<true, false, true>)
+               : (e5 ? qt::quant_transpose_kernel<false, true, true> : qt::quant_transpose_kernel<false, false, true>);
+  if (next == Next::kTransposingOnce)
+    k = e5 ? qt::quant_transpose_kernel<false, true, false> : qt::quant_transpose_kernel<false, false, false>;
   const int grid = transpose_grid(reinterpret_cast<const void*>(k), batch, rows, cols, cus);
   hipLaunchKernelGGL(k, dim3(grid), dim3(qt::kThreads), 0, s, x, batch, rows, cols, static_cast<uint8_t*>(out),
                      out_stride, static_cast<uint8_t*>(out_t), out_t_stride, partials, n,

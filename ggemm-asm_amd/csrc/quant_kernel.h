@@ -96,8 +96,8 @@ __device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w 
 
 // 8 consecutive elements of row `row`, chunk `c` (elements 8c .. 8c+7), as fp32. kKeep: ordinary loads, which
 // leave x in the memory-side cache for a pass that reads it next (the amax pass, by the rule at its launch)
-// and find it there (the transposing pass: [4, 5760, 2880] bf16 with its transpose 77.2 -> 72.5 us, in fp32
-// 152.5 -> 108.8 us). Else non-temporal ones: a streaming pass that reads x for the last time is faster with
+// and find it there (the transposing pass, but for some large tensors: [4, 5760, 2880] bf16 with its transpose
+// 77.2 -> 72.5 us, in fp32 152.5 -> 108.8 us). Else non-temporal ones: a streaming pass that reads x for the last time is faster with
 // them (307 us, 331 with ordinary loads there too, for [131072, 2880]).
 template <bool kF32, bool kKeep = false>
 __device__ __forceinline__ void load8(const void* x, int64_t row, int64_t stride, int c, float v[8]) {
@@ -393,8 +393,8 @@ __global__ void __launch_bounds__(kThreads) quant_tensorwise_delayed_kernel(cons
 // four q^T rows, so the 8 threads of a column group cover one 128-byte line per store instruction.
 // The 16-element segments of a ragged edge tile are wholly inside the matrix or outside.
 
-// kGiven as in tensorwise_body: guarded quotients, and the thread's max |x| returned.
-template <bool kF32, bool kE5M2, bool kFast, bool kGiven = false>
+// kKeep as in load8; kGiven as in tensorwise_body: guarded quotients, and the thread's max |x| returned.
+template <bool kF32, bool kE5M2, bool kKeep, bool kFast, bool kGiven = false>
 __device__ __forceinline__ uint32_t transpose_body(const void* x, int batch, int rows, int cols, uint8_t* out,
                                                    int64_t out_stride, uint8_t* out_t, int64_t out_t_stride,
                                                    const ScaleDiv& d, uint8_t* s_t) {
@@ -417,8 +417,8 @@ __device__ __forceinline__ uint32_t transpose_body(const void* x, int batch, int
     for (int h = 0; h < 4; ++h) {
       const int64_t row = (int64_t)b * rows + r0 + tr + 32 * h;
       if (col_in && r0 + tr + 32 * h < rows) {
-        load8<kF32, !kGiven>(x, row, cols, (c0 + tc) / 8, v[h]);
-        load8<kF32, !kGiven>(x, row, cols, (c0 + tc) / 8 + 1, v[h] + 8);
+        load8<kF32, kKeep>(x, row, cols, (c0 + tc) / 8, v[h]);
+        load8<kF32, kKeep>(x, row, cols, (c0 + tc) / 8 + 1, v[h] + 8);
       }
     }
 #pragma unroll
@@ -461,7 +461,7 @@ __device__ __forceinline__ uint32_t transpose_body(const void* x, int batch, int
   return m;
 }
 
-template <bool kF32, bool kE5M2>
+template <bool kF32, bool kE5M2, bool kKeep>
 __global__ void __launch_bounds__(kThreads) quant_transpose_kernel(const void* x, int batch, int rows, int cols,
                                                                    uint8_t* out, int64_t out_stride, uint8_t* out_t,
                                                                    int64_t out_t_stride, const uint32_t* partials,
@@ -474,9 +474,9 @@ __global__ void __launch_bounds__(kThreads) quant_transpose_kernel(const void* x
     if (amax_out) *amax_out = __uint_as_float(bits);
   }
   if (d.fast)
-    transpose_body<kF32, kE5M2, true>(x, batch, rows, cols, out, out_stride, out_t, out_t_stride, d, s_t);
+    transpose_body<kF32, kE5M2, kKeep, true>(x, batch, rows, cols, out, out_stride, out_t, out_t_stride, d, s_t);
   else
-    transpose_body<kF32, kE5M2, false>(x, batch, rows, cols, out, out_stride, out_t, out_t_stride, d, s_t);
+    transpose_body<kF32, kE5M2, kKeep, false>(x, batch, rows, cols, out, out_stride, out_t, out_t_stride, d, s_t);
 }
 
 // Delayed scaling of the transposing pass: the scale from the history's entries other than `slot`
@@ -493,9 +493,10 @@ __global__ void __launch_bounds__(kThreads) quant_transpose_delayed_kernel(const
   const ScaleDiv d = scale_div_given(tensor_scale<kE5M2>(history_amax(hist, H, slot)));
   if (blockIdx.x == 0 && threadIdx.x == 0) *scale_out = d.scale;
   const uint32_t m =
-      d.fast ? transpose_body<kF32, kE5M2, true, true>(x, batch, rows, cols, out, out_stride, out_t, out_t_stride, d, s_t)
-             : transpose_body<kF32, kE5M2, false, true>(x, batch, rows, cols, out, out_stride, out_t, out_t_stride, d,
-                                                        s_t);
+      d.fast ? transpose_body<kF32, kE5M2, false, true, true>(x, batch, rows, cols, out, out_stride, out_t,
+                                                              out_t_stride, d, s_t)
+             : transpose_body<kF32, kE5M2, false, false, true>(x, batch, rows, cols, out, out_stride, out_t,
+                                                               out_t_stride, d, s_t);
   block_amax(m, reinterpret_cast<uint32_t*>(hist + slot));
 }
 

@@ -1,4 +1,4 @@
-"""The amax pass's two ways to load x, on both sides of the sizes where the choice changes."""
+"""The quantizers' two ways to load x, on both sides of the sizes where the choice changes."""
 import pytest
 import torch
 
@@ -21,3 +21,23 @@ def test_amax_on_both_sides_of_the_size_rule(pkg, cuda, dtype, mb):
         assert float(scale) == float(scale_t) == float(torch.tensor(abs(v)) / 448)
         assert torch.equal(q.view(torch.uint8).t(), q_t.view(torch.uint8))
         assert float(q[at].float()) == (448.0 if v > 0 else -448.0)
+
+
+@pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
+@pytest.mark.parametrize("rows,align", [(5744, None), (5760, None), (5744, 128)])
+@pytest.mark.parametrize("mb", [274, 276])
+def test_transposing_pass_on_both_sides_of_its_load_rule(pkg, cuda, mb, rows, align, fmt):
+    """q^T rows off 128-byte lines, on them and padded to them, just below 275 MB of bf16 and just above: the
+    same bytes as the streaming pass writes, which has one way to load."""
+    batch = 16
+    cols = mb * 1000 * 1000 // (2 * batch * rows) // 16 * 16 + (16 if mb > 275 else 0)
+    x = torch.empty((batch, rows, cols), dtype=torch.bfloat16, device=cuda).normal_()
+    x[-1, -1, -1], x[0, 0, 0] = 100.0, -200.0
+    assert (x.nbytes > 275e6) == (mb > 275)
+    q, scale, am = pkg.quantize_fp8_tensorwise(x.view(batch * rows, cols), fmt=fmt)
+    q2, q_t, scale_t, am_t = pkg.quantize_fp8_tensorwise_transpose(x, fmt=fmt, row_align=align)
+    assert q_t.stride(-2) == (rows if align is None else -(-rows // align) * align)
+    assert float(am) == float(am_t) == 200.0 and float(scale) == float(scale_t)
+    u = q.view(torch.uint8).view(batch, rows, cols)
+    assert torch.equal(u, q2.view(torch.uint8))
+    assert torch.equal(u.transpose(1, 2), q_t.view(torch.uint8))
